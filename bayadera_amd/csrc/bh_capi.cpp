@@ -899,7 +899,25 @@ uint32_t acor_lag(uint32_t n, uint32_t wgs) {
     return std::max(lag, 10u);
 }
 
-// acor on a device series (dim x n), which it overwrites.
+// When acor runs split over the chip (acor_slice_kernel and its kin) and not
+// one block per column.  Short series stay on the single launch, which walks
+// one slice for them: whole calls at WGS 256, one block against split, 1 to
+// 64 columns: 128 steps 40-51 / 44-48 us, 200 steps 45-57 / 45-48, 1000
+// steps 86-143 / 49-53.  Many columns fill the chip with one block each: 1024
+// columns x 300 steps 130 / 223 us, 2048 x 2000 457 / 460, but 512 x 20,000
+// 1795 / 804.  The scratch is about 8 bytes per value of the series.
+constexpr uint32_t kAcorSplitSteps = 160;
+constexpr uint32_t kAcorSplitStepsPerColumn = 4;
+constexpr size_t kAcorSplitBytes = (size_t)256 << 20;
+
+bool acor_split(uint32_t cols, uint32_t max_stride, uint32_t n, uint32_t lag, uint32_t wgs,
+                bh::AcorSplit* plan) {
+    if (n <= kAcorSplitSteps || cols > std::min(n / kAcorSplitStepsPerColumn, 65535u)) return false;
+    *plan = bh::acor_split_plan(cols, max_stride, n, lag, wgs);
+    return plan->floats * sizeof(float) <= kAcorSplitBytes;
+}
+
+// acor on a device series (dim x n), which it may overwrite.
 int acor_device(bh_ctx* c, hipStream_t st, float* d_series, uint32_t dim, uint32_t n, float* tau,
                 float* mean, float* sigma, uint32_t* lag_out) {
     const uint32_t lag = acor_lag(n, c->wgs);
@@ -914,11 +932,18 @@ int acor_device(bh_ctx* c, hipStream_t st, float* d_series, uint32_t dim, uint32
     const uint32_t half = (n + local_n_mean - 1) / local_n_mean + (n + c->wgs - 1) / c->wgs + 8;
     const uint32_t per_dim = 2 * half;
     DevBuf scratch, out;
-    BH_TRY(scratch.alloc((size_t)per_dim * dim * sizeof(float)));
     BH_TRY(out.alloc((size_t)3 * dim * sizeof(float)));
     float* o = out.as<float>();
-    BH_HIP(bh::launch_acor(st, d_series, dim, n, lag, c->wgs, scratch.as<float>(), per_dim, o,
-                           o + dim, o + 2 * dim));
+    bh::AcorSplit plan;
+    if (acor_split(dim, dim, n, lag, c->wgs, &plan)) {
+        BH_TRY(scratch.alloc(plan.floats * sizeof(float)));
+        BH_HIP(bh::launch_acor_split(st, d_series, nullptr, nullptr, dim, dim, plan, c->wgs,
+                                     scratch.as<float>(), o, o + dim, o + 2 * dim));
+    } else {
+        BH_TRY(scratch.alloc((size_t)per_dim * dim * sizeof(float)));
+        BH_HIP(bh::launch_acor(st, d_series, dim, n, lag, c->wgs, scratch.as<float>(), per_dim, o,
+                               o + dim, o + 2 * dim));
+    }
     std::vector<float> h(3 * dim);
     BH_HIP(hipMemcpyAsync(h.data(), o, h.size() * sizeof(float), hipMemcpyDeviceToHost, st));
     BH_TRY(sync(st));
@@ -1414,9 +1439,10 @@ int bh_acor_batch(bh_ctx* ctx, const float* series, uint32_t problems, const uin
     std::vector<unsigned long long> off;
     std::vector<unsigned> stride;
     uint64_t base = 0;
-    uint32_t per_dim = 0;
+    uint32_t per_dim = 0, max_dim = 0;
     for (uint32_t p = 0; p < problems; ++p) {
         BH_ARG(dims[p] > 0, "problem %u: empty series", p);
+        max_dim = std::max(max_dim, dims[p]);
         for (uint32_t d = 0; d < dims[p]; ++d) {
             off.push_back(base + d);
             stride.push_back(dims[p]);
@@ -1431,7 +1457,6 @@ int bh_acor_batch(bh_ctx* ctx, const float* series, uint32_t problems, const uin
     hipStream_t st = ctx->stream;
     DevBuf copy, scratch, out, doff, dstride;
     BH_TRY(copy.alloc((size_t)base * sizeof(float)));
-    BH_TRY(scratch.alloc((size_t)per_dim * cols * sizeof(float)));
     BH_TRY(out.alloc((size_t)3 * cols * sizeof(float)));
     BH_TRY(doff.alloc(off.size() * sizeof(unsigned long long)));
     BH_TRY(dstride.alloc(stride.size() * sizeof(unsigned)));
@@ -1441,9 +1466,18 @@ int bh_acor_batch(bh_ctx* ctx, const float* series, uint32_t problems, const uin
     BH_HIP(hipMemcpyAsync(dstride.p, stride.data(), stride.size() * sizeof(unsigned),
                           hipMemcpyHostToDevice, st));
     float* o = out.as<float>();
-    BH_HIP(bh::launch_acor_batch(st, copy.as<float>(), doff.as<unsigned long long>(),
-                                 dstride.as<unsigned>(), cols, n, lg, wgs, scratch.as<float>(),
-                                 per_dim, o, o + cols, o + 2 * cols));
+    bh::AcorSplit plan;
+    if (acor_split(cols, max_dim, n, lg, wgs, &plan)) {
+        BH_TRY(scratch.alloc(plan.floats * sizeof(float)));
+        BH_HIP(bh::launch_acor_split(st, copy.as<float>(), doff.as<unsigned long long>(),
+                                     dstride.as<unsigned>(), 0, cols, plan, wgs,
+                                     scratch.as<float>(), o, o + cols, o + 2 * cols));
+    } else {
+        BH_TRY(scratch.alloc((size_t)per_dim * cols * sizeof(float)));
+        BH_HIP(bh::launch_acor_batch(st, copy.as<float>(), doff.as<unsigned long long>(),
+                                     dstride.as<unsigned>(), cols, n, lg, wgs,
+                                     scratch.as<float>(), per_dim, o, o + cols, o + 2 * cols));
+    }
     std::vector<float> h(3 * (size_t)cols);
     BH_HIP(hipMemcpyAsync(h.data(), o, h.size() * sizeof(float), hipMemcpyDeviceToHost, st));
     BH_TRY(sync(st));

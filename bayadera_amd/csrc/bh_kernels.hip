@@ -433,7 +433,6 @@ __device__ __forceinline__ void acor_column(float* __restrict__ col, unsigned cs
                                             float* __restrict__ sigma) {
     const unsigned wgs = blockDim.x;
     const unsigned l = threadIdx.x;
-    const unsigned win_mult = 5, min_lag = 10;
     __shared__ float lacc[kMaxGroupThreads];
     __shared__ float lm[2 * kMaxGroupThreads];
     float* dacc = c0acc + scratch_per_dim / 2;
@@ -524,9 +523,8 @@ __device__ __forceinline__ void acor_column(float* __restrict__ col, unsigned cs
     while (true) {
         const float start_c0 = (stride == 1) ? c0 : orig_c0;
         const float tv = dd / ((stride == 1) ? c0 : prev_c0);
-        const unsigned lag2 =
-            (cur_lag * win_mult < prev_n) ? cur_lag : ((prev_n / win_mult) > 10u ? prev_n / win_mult : 10u);
-        if (min_lag < lag2 && (float)lag2 < tv * (float)win_mult) {
+        const unsigned lag2 = acor_next_lag(cur_lag, prev_n);
+        if (kAcorMinLag < lag2 && (float)lag2 < tv * (float)kAcorWinMult) {
             const unsigned n2 = prev_n / 2;
             const unsigned w2 = wgs < n2 ? wgs : n2;
             const size_t step = (size_t)stride * cs;
@@ -582,6 +580,323 @@ acor_batch_kernel(float* __restrict__ series, const unsigned long long* __restri
     acor_column(series + col_off[b], cs, n, lag, inv_n, wgs / wgsm,
                 scratch + (size_t)b * scratch_per_dim, scratch_per_dim, tau + b, mean + b,
                 sigma + b);
+}
+
+// --------------------------------------------------------------------------
+// The same estimator split over the chip, for long series of few columns.
+// acor_column walks a column's slices in turn with ~30 barriers each, on one
+// compute unit per column: 5.0 ms for 112,640 steps x 2 (440 slices per
+// level-0 pass), all of it latency.  Nothing in the walk depends on an
+// earlier slice, and the only data-dependent choice, at which halving of the
+// series to stop, can be made last: the lags and lengths of every level
+// follow from n alone.  So the mean's trees, the series of every level (the
+// pairwise sums are a pyramid over the centred series), the lag sums of
+// every slice of every level, and the reduction over slices each become one
+// launch over all slices, and one thread per column then picks the level.
+// Levels past the one that is picked cost at most as much as level 0 does.
+// Every sum keeps acor_column's shape, so the results are the same bit for
+// bit.  5-6 launches, 0.046 ms for 112,640 x 2.
+// --------------------------------------------------------------------------
+
+// The column a block works on: of one n x dim series, or of many (col_off and
+// col_stride as in acor_batch_kernel).
+struct AcorCols {
+    const unsigned long long* off;  // null: one series of `dim` columns
+    const unsigned* stride;
+    unsigned dim;
+    __device__ __forceinline__ const float* base(const float* series, unsigned c) const {
+        return series + (off ? off[c] : c);
+    }
+    __device__ __forceinline__ unsigned step(unsigned c) const { return off ? stride[c] : dim; }
+};
+
+__device__ __forceinline__ unsigned acor_mean_group(unsigned cs, unsigned wgs) {
+    unsigned w = cs < 16 ? cs : 16;
+    if (wgs < w) w = wgs;
+    return wgs / w;
+}
+
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// group_tree's sum of v[0 .. len) by `p` lanes of one wave (lane sl of them):
+// at each level an item l < i/2 adds item l + i/2 (and item i/2 - 1 first the
+// last one when i is odd), which only reads at or past i/2 and only writes
+// before it.  Left in v[0].  All lanes of the wave call it together.
+__device__ __forceinline__ void sub_tree(float* v, unsigned len, unsigned p, unsigned sl,
+                                         unsigned longest) {
+    unsigned i = len;
+    for (unsigned m = longest; m > 1; m >>= 1) {  // as many levels as the longest of the wave
+        wave_lds_sync();
+        const bool odd = i & 1u;
+        const unsigned h = i >> 1;
+        for (unsigned l = sl; l < h; l += p) {
+            float a = v[l];
+            if (odd && l == h - 1) a += v[2 * h];
+            v[l] = a + v[l + h];
+        }
+        if (i > 1) i = h;
+    }
+    wave_lds_sync();
+}
+
+// Lanes that share one group of at most `longest` values: a power of two.
+__device__ __forceinline__ unsigned sub_lanes(unsigned longest) {
+    unsigned p = 1;
+    while (p < longest && p < 64) p <<= 1;
+    return p;
+}
+
+// One pass of the mean's enq-reduce!: group g of local_n values (element t at
+// src[t * cs]) to dst[g], 64 / p groups per wave and round.
+__device__ __forceinline__ void acor_mean_pass(const float* __restrict__ src, size_t cs, unsigned count,
+                                               unsigned local_n, float* __restrict__ dst,
+                                               float* lds, unsigned wave, unsigned waves) {
+    const unsigned lane = threadIdx.x & 63u;
+    const unsigned p = sub_lanes(local_n), per = 64 / p, sl = lane % p;
+    const unsigned groups = (count + local_n - 1) / local_n;
+    float* v = lds + (lane / p) * local_n;
+    for (unsigned g0 = wave * per; g0 < groups; g0 += waves * per) {
+        const unsigned g = g0 + lane / p;
+        unsigned len = 0;
+        if (g < groups) {
+            const unsigned start = g * local_n;
+            len = count - start < local_n ? count - start : local_n;
+            for (unsigned l = sl; l < len; l += p) v[l] = src[(size_t)(start + l) * cs];
+        }
+        sub_tree(v, len, p, sl, local_n);
+        if (g < groups && sl == 0) dst[g] = v[0];
+        wave_lds_sync();
+    }
+}
+
+// LDS floats of one wave in acor_mean_pass: 64 / p groups of local_n.
+constexpr unsigned kAcorMeanLds = kMaxGroupThreads;
+
+// First pass of the mean over all columns: grid (blocks, columns).
+__global__ void __launch_bounds__(256)
+acor_mean_kernel(const float* __restrict__ series, AcorCols cols, unsigned n, unsigned wgs,
+                 float* __restrict__ part, unsigned part_stride) {
+    __shared__ float lds[4][kAcorMeanLds];
+    const unsigned c = blockIdx.y, cs = cols.step(c), wave = threadIdx.x >> 6;
+    acor_mean_pass(cols.base(series, c), cs, n, acor_mean_group(cs, wgs),
+                   part + (size_t)c * part_stride, lds[wave], blockIdx.x * 4 + wave,
+                   gridDim.x * 4);
+}
+
+// The passes that are left, one block per column, back and forth between the
+// two halves of its scratch; mu[c] = the mean.
+__global__ void __launch_bounds__(512)
+acor_mean_finish_kernel(AcorCols cols, unsigned n, unsigned wgs, float inv_n,
+                        float* __restrict__ part, unsigned part_stride, float* __restrict__ part2,
+                        float* __restrict__ mu) {
+    __shared__ float lds[8][kAcorMeanLds];
+    const unsigned c = blockIdx.x, wave = threadIdx.x >> 6;
+    const unsigned local_n = acor_mean_group(cols.step(c), wgs);
+    unsigned count = (n + local_n - 1) / local_n;
+    float* a = part + (size_t)c * part_stride;
+    float* b = part2 + (size_t)c * part_stride;
+    while (count > 1) {
+        acor_mean_pass(a, 1, count, local_n, b, lds[wave], wave, 8);
+        __syncthreads();
+        float* t = a;
+        a = b;
+        b = t;
+        count = (count + local_n - 1) / local_n;
+    }
+    if (threadIdx.x == 0) mu[c] = a[0] * inv_n;
+}
+
+// The series of levels l0 .. l0 + kAcorPyramid: a block takes 2^kAcorPyramid
+// values of level l0 (of the series itself minus its mean when l0 is 0) and
+// sums neighbours pairwise, level by level; level l holds n >> l values at
+// lev + c * lev_stride + t.data[l].  An odd last value is dropped, as the
+// halved series does.
+__global__ void __launch_bounds__(256)
+acor_pyramid_kernel(const float* __restrict__ series, AcorCols cols, AcorLevels t, unsigned l0,
+                    const float* __restrict__ mu, float* __restrict__ lev, size_t lev_stride) {
+    constexpr unsigned N = 1u << kAcorPyramid;
+    __shared__ float buf[2][N];
+    const unsigned c = blockIdx.y;
+    float* out = lev + (size_t)c * lev_stride;
+    const unsigned long long first = (unsigned long long)blockIdx.x * N;
+    if (l0 == 0) {
+        const float* src = cols.base(series, c);
+        const unsigned cs = cols.step(c);
+        const float m = mu[c];
+#pragma unroll
+        for (unsigned q = 0; q < N / 256; ++q) {
+            const unsigned i = q * 256 + threadIdx.x;
+            const unsigned long long g = first + i;
+            float v = 0.0f;
+            if (g < t.n[0]) {
+                v = src[g * cs] - m;
+                out[g] = v;
+            }
+            buf[0][i] = v;
+        }
+    } else {
+#pragma unroll
+        for (unsigned q = 0; q < N / 256; ++q) {
+            const unsigned i = q * 256 + threadIdx.x;
+            const unsigned long long g = first + i;
+            buf[0][i] = g < t.n[l0] ? out[t.data[l0] + g] : 0.0f;
+        }
+    }
+    unsigned which = 0;
+    for (unsigned s = 1; s <= kAcorPyramid && l0 + s < t.levels; ++s) {
+        __syncthreads();
+        const unsigned l = l0 + s;
+        const unsigned long long at = first >> s;
+        for (unsigned i = threadIdx.x; i < (N >> s); i += 256) {
+            const float v = buf[which][2 * i] + buf[which][2 * i + 1];
+            buf[which ^ 1][i] = v;
+            if (at + i < t.n[l]) out[t.data[l] + at + i] = v;
+        }
+        which ^= 1;
+    }
+}
+
+// Two of group_tree's sums at once (they share the barriers); lacc has twice
+// blockDim floats.
+__device__ __forceinline__ void group_tree2(float& a, float& b, unsigned lsize, float* lacc) {
+    const unsigned l = threadIdx.x;
+    float* lb = lacc + blockDim.x;
+    __syncthreads();
+    if (l < lsize) {
+        lacc[l] = a;
+        lb[l] = b;
+    }
+    __syncthreads();
+    unsigned i = lsize;
+    while (i > 0) {
+        const bool odd = (i & 1u) && (l == (i >> 1) - 1);
+        i >>= 1;
+        if (odd) {
+            a += lacc[l + i + 1];
+            b += lb[l + i + 1];
+        }
+        if (l < i) {
+            a += lacc[l + i];
+            b += lb[l + i];
+            lacc[l] = a;
+            lb[l] = b;
+        }
+        __syncthreads();
+    }
+    a = lacc[0];
+    b = lb[0];
+}
+
+// acor_1d's sums (acor.cl:26-86) of one slice of one level of one column:
+// grid (slices of all levels, columns), wgs threads.
+__global__ void __launch_bounds__(kMaxGroupThreads)
+acor_slice_kernel(AcorLevels t, const float* __restrict__ lev, size_t lev_stride,
+                  float* __restrict__ sums, unsigned total_groups) {
+    __shared__ float lacc[2 * kMaxGroupThreads];
+    __shared__ float lm[2 * kMaxGroupThreads];
+    const unsigned wgs = blockDim.x, l = threadIdx.x, c = blockIdx.y;
+    unsigned k = 0;
+    while (k + 1 < t.levels && blockIdx.x >= t.group[k + 1]) ++k;
+    const unsigned gsize = t.n[k], lg = t.lag[k], lw = wgs < gsize ? wgs : gsize;
+    const unsigned g = blockIdx.x - t.group[k];
+    const float* col = lev + (size_t)c * lev_stride + t.data[k];
+    const unsigned start = g * lw;
+    const unsigned lsize = gsize - start < lw ? gsize - start : lw;
+    const bool has_next = start + lw < gsize;
+    lm[l] = 0.0f;
+    lm[l + wgs] = 0.0f;
+    __syncthreads();
+    if (l < lsize) {
+        const unsigned gid = start + l;
+        const bool load_lag = (l < lg) && has_next && (gid + lsize < gsize);
+        lm[l] = gid + lg < gsize ? col[gid] : 0.0f;
+        lm[l + lsize] = load_lag ? col[gid + lsize] : 0.0f;
+    }
+    __syncthreads();
+    float xv = 0.0f, xacc = 0.0f;
+    if (l < lsize) {
+        xv = lm[l];
+        for (unsigned s = 0; s < lg; ++s) {
+            const unsigned idx = l + s + 1;
+            xacc += idx < 2 * lsize ? lm[idx] : 0.0f;
+        }
+        xacc = xv * __builtin_fmaf(2.0f, xacc, xv);
+    }
+    float c0 = xv * xv;
+    group_tree2(c0, xacc, lsize, lacc);
+    if (l == 0) {
+        float* o = sums + (size_t)c * 2 * total_groups + blockIdx.x;
+        o[0] = c0;
+        o[total_groups] = xacc;
+    }
+}
+
+// sum_reduction_acor's reduction (acor.cl:88-130) of every level, a wave per
+// level, then the choice of the level and the results by one thread: one
+// block of 4 waves per column.  LDS: 8 wgs floats.
+__global__ void __launch_bounds__(256)
+acor_choose_kernel(AcorLevels t, unsigned wgs, const float* __restrict__ sums,
+                   unsigned total_groups, const float* __restrict__ mu, float* __restrict__ tau,
+                   float* __restrict__ mean, float* __restrict__ sigma) {
+    extern __shared__ float red[];
+    __shared__ float lc0[kAcorMaxLevels], ldd[kAcorMaxLevels];
+    const unsigned c = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+    float* va = red + (size_t)wave * 2 * wgs;
+    float* vb = va + wgs;
+    for (unsigned k = wave; k < t.levels; k += 4) {
+        const unsigned lw = wgs < t.n[k] ? wgs : t.n[k];
+        const unsigned groups = (t.n[k] + lw - 1) / lw;
+        const unsigned lsize = groups < wgs ? groups : wgs;
+        const float* sa = sums + (size_t)c * 2 * total_groups + t.group[k];
+        const float* sb = sa + total_groups;
+        for (unsigned i = lane; i < lsize; i += 64) {
+            float a = 0.0f, b = 0.0f;
+            for (unsigned q = i; q < groups; q += lsize) {
+                a += sa[q];
+                b += sb[q];
+            }
+            va[i] = a;
+            vb[i] = b;
+        }
+        sub_tree(va, lsize, 64, lane, lsize);
+        sub_tree(vb, lsize, 64, lane, lsize);
+        if (lane == 0) {
+            lc0[k] = va[0];
+            ldd[k] = vb[0];
+        }
+        wave_lds_sync();
+    }
+    __syncthreads();
+    if (threadIdx.x) return;
+    // acor_column's loop over levels, on the sums that are there already
+    const unsigned n = t.n[0];
+    unsigned stride = 1, cur_lag = t.lag[0], prev_n = n, k = 0;
+    float c0 = lc0[0], dd = ldd[0], orig_c0 = 0.0f, prev_c0 = 0.0f;
+    while (true) {
+        const float start_c0 = (stride == 1) ? c0 : orig_c0;
+        const float tv = dd / ((stride == 1) ? c0 : prev_c0);
+        const unsigned lag2 = acor_next_lag(cur_lag, prev_n);
+        if (k + 1 < t.levels && (float)lag2 < tv * (float)kAcorWinMult) {
+            orig_c0 = start_c0;
+            prev_c0 = c0;
+            ++k;
+            c0 = lc0[k];
+            dd = ldd[k];
+            stride *= 2;
+            cur_lag = lag2;
+            prev_n = t.n[k];
+        } else {
+            const float scale = (float)stride * (float)(prev_n - lag2);
+            tau[c] = dd * (float)(n - cur_lag) / (scale * start_c0);
+            sigma[c] = sqrtf(dd / (scale * (float)n));
+            mean[c] = mu[c];
+            break;
+        }
+    }
 }
 
 // --------------------------------------------------------------------------
@@ -744,6 +1059,64 @@ hipError_t launch_acor_batch(hipStream_t s, float* series, const unsigned long l
     const float inv_n = (float)(1.0 / (double)n);
     acor_batch_kernel<<<cols, wgs, 0, s>>>(series, col_off, col_stride, n, lag, inv_n, scratch,
                                            scratch_per_dim, tau, mean, sigma);
+    return hipGetLastError();
+}
+
+AcorSplit acor_split_plan(unsigned cols, unsigned max_stride, unsigned n, unsigned lag,
+                          unsigned wgs) {
+    AcorSplit p{};
+    AcorLevels& t = p.t;
+    size_t data = 0;
+    unsigned nn = n, lg = lag, groups = 0;
+    while (true) {
+        const unsigned k = t.levels++, lw = wgs < nn ? wgs : nn;
+        t.n[k] = nn;
+        t.lag[k] = lg;
+        t.data[k] = data;
+        t.group[k] = groups;
+        data += nn;
+        groups += (nn + lw - 1) / lw;
+        const unsigned lag2 = acor_next_lag(lg, nn);
+        if (lag2 <= kAcorMinLag || t.levels == kAcorMaxLevels) break;
+        lg = lag2;
+        nn /= 2;
+    }
+    p.total_groups = groups;
+    p.lev_stride = (data + 63) / 64 * 64;
+    // the smallest group of the mean's reduction leaves the most partial sums
+    unsigned w = max_stride < 16 ? max_stride : 16;
+    if (wgs < w) w = wgs;
+    p.part_stride = (n + wgs / w - 1) / (wgs / w);
+    p.floats = (size_t)cols * (p.lev_stride + 2 * (size_t)p.part_stride + 2 * (size_t)groups + 1);
+    return p;
+}
+
+hipError_t launch_acor_split(hipStream_t s, const float* series, const unsigned long long* col_off,
+                             const unsigned* col_stride, unsigned dim, unsigned cols,
+                             const AcorSplit& p, unsigned wgs, float* scratch, float* tau,
+                             float* mean, float* sigma) {
+    const AcorLevels& t = p.t;
+    const unsigned n = t.n[0];
+    const AcorCols c{col_off, col_stride, dim};
+    const float inv_n = (float)(1.0 / (double)n);
+    float* lev = scratch;
+    float* part = lev + (size_t)cols * p.lev_stride;
+    float* part2 = part + (size_t)cols * p.part_stride;
+    float* sums = part2 + (size_t)cols * p.part_stride;
+    float* mu = sums + (size_t)cols * 2 * p.total_groups;
+    const unsigned waves = (p.part_stride + 3) / 4;
+    const unsigned mb = waves < 1024 ? waves : 1024;
+    acor_mean_kernel<<<dim3(mb, cols), 256, 0, s>>>(series, c, n, wgs, part, p.part_stride);
+    acor_mean_finish_kernel<<<cols, 512, 0, s>>>(c, n, wgs, inv_n, part, p.part_stride, part2, mu);
+    for (unsigned l0 = 0; l0 == 0 || l0 + 1 < t.levels; l0 += kAcorPyramid) {
+        const unsigned blocks = (t.n[l0] + (1u << kAcorPyramid) - 1) >> kAcorPyramid;
+        acor_pyramid_kernel<<<dim3(blocks, cols), 256, 0, s>>>(series, c, t, l0, mu, lev,
+                                                               p.lev_stride);
+    }
+    acor_slice_kernel<<<dim3(p.total_groups, cols), wgs, 0, s>>>(t, lev, p.lev_stride, sums,
+                                                                 p.total_groups);
+    acor_choose_kernel<<<cols, 256, 8 * wgs * sizeof(float), s>>>(t, wgs, sums, p.total_groups, mu,
+                                                                   tau, mean, sigma);
     return hipGetLastError();
 }
 

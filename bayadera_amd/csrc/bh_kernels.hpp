@@ -46,6 +46,35 @@ hipError_t launch_row_tree_sum(hipStream_t s, const float* a, unsigned rows, uns
                                float scale, float* out, unsigned long long out_stride);
 hipError_t launch_sum_u32(hipStream_t s, const unsigned* v, unsigned n, unsigned long long* out);
 hipError_t launch_sum_f64(hipStream_t s, const double* v, unsigned n, double* out);
+// acor split over the chip (long series of few columns): the lengths, lags,
+// offsets and slices of every level the estimator can reach, which follow
+// from n, and the scratch they need.
+constexpr unsigned kAcorMaxLevels = 32;  // halvings of a series of < 2^31 steps
+constexpr unsigned kAcorPyramid = 11;    // levels per pyramid launch (2048 values per block)
+constexpr unsigned kAcorWinMult = 5, kAcorMinLag = 10;
+// the lag of the level after one of prev_n points with lag `lag` (acor.cl:143-168)
+__host__ __device__ inline unsigned acor_next_lag(unsigned lag, unsigned prev_n) {
+    if (lag * kAcorWinMult < prev_n) return lag;
+    return prev_n / kAcorWinMult > kAcorMinLag ? prev_n / kAcorWinMult : kAcorMinLag;
+}
+struct AcorLevels {
+    unsigned levels;
+    unsigned n[kAcorMaxLevels], lag[kAcorMaxLevels], group[kAcorMaxLevels];
+    size_t data[kAcorMaxLevels];
+};
+struct AcorSplit {
+    AcorLevels t;
+    unsigned total_groups, part_stride;
+    size_t lev_stride, floats;  // floats: of the scratch
+};
+AcorSplit acor_split_plan(unsigned cols, unsigned max_stride, unsigned n, unsigned lag,
+                          unsigned wgs);
+// series (device) is only read; col_off and col_stride as acor_batch's, or
+// null for one series of `dim` = `cols` columns.
+hipError_t launch_acor_split(hipStream_t s, const float* series, const unsigned long long* col_off,
+                             const unsigned* col_stride, unsigned dim, unsigned cols,
+                             const AcorSplit& p, unsigned wgs, float* scratch, float* tau,
+                             float* mean, float* sigma);
 hipError_t launch_acor_batch(hipStream_t s, float* series, const unsigned long long* col_off,
                              const unsigned* col_stride, unsigned cols, unsigned n, unsigned lag,
                              unsigned wgs, float* scratch, unsigned scratch_per_dim, float* tau,
