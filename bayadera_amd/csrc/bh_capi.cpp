@@ -245,6 +245,7 @@ struct bh_ctx {
     int device = 0;
     uint32_t wgs = 256;
     int cu = 0;
+    int lds_max = 0;  // LDS of one work-group
     std::string arch;
     hipStream_t stream = nullptr;
     DevBuf scratch;
@@ -307,7 +308,8 @@ struct bh_stretch_factory {
     bh_ctx* ctx = nullptr;
     uint32_t dim = 0, params_len = 0;
     Module mod;
-    hipFunction_t logfn = nullptr, bare = nullptr, accu = nullptr, resident = nullptr;
+    hipFunction_t logfn = nullptr, bare = nullptr, accu = nullptr, resident = nullptr,
+                  resident_out = nullptr, draws = nullptr, trace_accu = nullptr;
     std::unique_ptr<GlmData> glm;
     hipFunction_t glm_propose = nullptr, glm_split = nullptr, glm_logpost = nullptr,
                   glm_accept = nullptr, glm_screen = nullptr, glm_resolve = nullptr,
@@ -344,7 +346,8 @@ struct bh_stretch {
     hipStream_t stream = nullptr;
     uint32_t dim = 0, W = 0, K = 0, wgs = 0, groups = 0;
     uint32_t params_count = 0, data_len = 0, params_len = 0;
-    DevBuf xs, logfn, params, accept, means_acc, tmp;
+    DevBuf xs, logfn, params, accept, means_acc;
+    DevBuf rdraws, rtrace, rsink;  // a chunk of resident steps' draws and positions
     uint64_t means_cap = 0;
     uint32_t bare_seed = 0, move_seed = 0, bare_counter = 0, move_counter = 0;
     uint64_t iter = 0;
@@ -379,6 +382,23 @@ struct bh_stretch {
 };
 
 constexpr size_t kKernelTimerPairs = 1024;
+
+// When an ensemble that fits in one compute unit's LDS runs there (see
+// use_resident).  Steps, per-half-step kernels against resident, us per bare /
+// accounted step:
+//   1024 walkers   dim 4   5.1 / 8.5 -> 0.7 / 0.8    dim 24  17 / 27 -> 11 / 10
+//   4096           dim 1   5.3 / 7.5 -> 3.0 / 2.6    dim 7  6.8 / 12 -> 5.0 / 5.2
+//   8192           dim 1   5.3 / 7.6 -> 3.8 / 5.1    dim 2  5.3 / 8.2 -> 5.1 / 4.7
+//   12,288         dim 2   5.2 / 8.4 -> 5.7 / 7.5
+// A density that loops over data keeps one compute unit busy for longer than
+// the launches take on all of them (gaussian likelihood, bare): 50 values,
+// 1024 walkers 12.6 -> 7.0, 2048 12.9 -> 13.6, 4096 13.8 -> 23; 5000 values,
+// 1024 walkers 929 -> 535, 2048 930 -> 1216.  So past 1024 walkers the data
+// and the parameters a step reads are bounded too.
+constexpr uint32_t kResidentWalkers = 8192;
+constexpr uint32_t kResidentAnyDensity = 1024;
+constexpr uint64_t kResidentData = 100000;
+constexpr uint64_t kResidentParams = 1000000;
 
 // rounds of work-groups per logistic likelihood launch
 constexpr unsigned kGlmRounds = 4;
@@ -444,53 +464,97 @@ int ktimed(bh_stretch* s, F&& launch_fn) {
     return BH_OK;
 }
 
-// block size of the resident kernel: a multiple of WGS dividing K, <= 1024
+// Threads of the resident kernel: K walkers in as few passes ("slots") of at
+// most 1024 as it takes, evenly filled.
+unsigned resident_slots(const bh_stretch* s) { return (s->K + 1023) / 1024; }
 unsigned resident_block(const bh_stretch* s) {
+    const unsigned slots = resident_slots(s);
+    return ((s->K + slots - 1) / slots + 63) / 64 * 64;
+}
+
+// Its LDS: both halves with their wrapped tails (bh_resident_half), the log
+// densities and the accept counts.
+size_t resident_lds(const bh_stretch* s) {
+    const size_t half = ((size_t)s->K * s->dim + s->dim - 1 + 3) / 4 * 4;
+    return (2 * half + s->W + s->groups) * 4;
+}
+
+// The ensembles BH_EXEC_RESIDENT accepts: positions, log densities and 8
+// floats per thread within 64 KB.
+bool resident_accepted(const bh_stretch* s) {
     unsigned nb = s->K <= 1024 ? s->K : 1024;
     while (nb > s->wgs && (s->K % nb) != 0) nb -= s->wgs;
-    return nb;
-}
-
-size_t resident_lds(const bh_stretch* s, int mode) {
-    const unsigned nb = resident_block(s);
-    // positions, logfn values, and the accounting staging areas (the
-    // kernel's BH_ACCU_CHUNK = min(DIM, 8) floats per thread, the odd half's
-    // group sums and the groups' accept counts)
     const size_t chunk = s->dim < 8 ? s->dim : 8;
-    const size_t groups = s->K / s->wgs;
-    size_t floats = (size_t)s->W * s->dim + s->W +
-                    (mode == 1 ? chunk * nb + groups * s->dim + groups : 0);
-    return floats * 4 + (nb / 64) * 4;
+    const size_t floats = (size_t)s->W * s->dim + s->W + chunk * nb + (size_t)s->groups * (s->dim + 1);
+    return floats * 4 + (nb / 64) * 4 <= 64 * 1024;
 }
 
-constexpr size_t kResidentLdsMax = 64 * 1024;
+// Draws and trace of one chunk of resident steps; kept by the sampler.  (Two
+// rounds of the kernel's four draws in flight lie past the last half-step.)
+constexpr uint32_t kResidentPad = 8;
+constexpr size_t kResidentWork = (size_t)16 << 20;
+constexpr uint32_t kResidentSteps = 16384;
 
-bool use_resident(const bh_stretch* s, int mode) {
+bool use_resident(const bh_stretch* s) {
     if (s->exec == BH_EXEC_STEPWISE || s->f->glm) return false;
-    const bool fits = resident_lds(s, mode) <= kResidentLdsMax;
-    if (s->exec == BH_EXEC_RESIDENT) return fits;
-    // a single work-group pays off while the ensemble is small
-    return fits && s->W <= 4096;
+    if (s->exec == BH_EXEC_RESIDENT) return true;
+    if (s->W > kResidentWalkers || resident_lds(s) > (size_t)s->ctx->lds_max) return false;
+    return s->W <= kResidentAnyDensity ||
+           ((uint64_t)s->data_len * s->W <= kResidentData &&
+            (uint64_t)s->params_count * s->W <= kResidentParams);
 }
 
-int run_resident(bh_stretch* s, int mode, uint32_t seed_odd, uint32_t seed_even, uint32_t c_odd,
+// nsteps resident steps: per chunk the draws, the steps and, with accu, the
+// accounting from their trace; with sample_out the positions after every
+// step go there (nsteps whole ensembles).
+int run_resident(bh_stretch* s, bool accu, uint32_t seed_odd, uint32_t seed_even, uint32_t c_odd,
                  uint32_t c_even, float a, float beta, const float* d_betas, uint32_t step0,
-                 uint32_t nsteps, float* sample_out, unsigned long long sample_floats) {
+                 uint32_t nsteps, float* sample_out) {
+    if (nsteps == 0) return BH_OK;
+    const unsigned nb = resident_block(s), Kp = nb * resident_slots(s);
+    const size_t draw_bytes = (size_t)2 * Kp * 16;
+    const size_t step_floats = (size_t)s->W * s->dim;
+    const size_t per_step = draw_bytes + (accu ? step_floats * sizeof(float) : 0);
+    const uint32_t most = (uint32_t)std::min<size_t>(
+        kResidentSteps, std::max<size_t>(1, kResidentWork / per_step));
+    const uint32_t chunk = std::min(nsteps, most);
+    BH_TRY(s->rdraws.alloc(draw_bytes * chunk + (size_t)kResidentPad * nb * 16));
+    BH_TRY(s->rsink.alloc(step_floats / 2 * sizeof(float)));
+    if (accu) BH_TRY(s->rtrace.alloc(step_floats * sizeof(float) * chunk));
     unsigned data_len = s->data_len, params_len = s->params_len, K = s->K;
     const float* params = s->params.as<float>();
     float* xs = s->xs.as<float>();
     float* lf = s->logfn.as<float>();
+    float4* draws = s->rdraws.as<float4>();
+    const float4* drawsc = draws;
     int partner = s->partner;
-    unsigned* acc = mode == 1 ? s->accept.as<unsigned>() : nullptr;
-    float* means = mode == 1 ? s->means_acc.as<float>() : nullptr;
-    void* args[] = {&seed_odd, &seed_even, &c_odd,   &c_even,      &data_len, &params_len,
-                    &params,   &xs,        &lf,      &K,           &a,        &beta,
-                    &d_betas,  &step0,     &nsteps,  &partner,     &mode,     &acc,
-                    &means,    &sample_out, &sample_floats};
-    return ktimed(s, [&] {
-        return launch(s->f->resident, 1, resident_block(s), (unsigned)resident_lds(s, mode),
-                      s->stream, args);
-    });
+    unsigned* acc = accu ? s->accept.as<unsigned>() : nullptr;
+    float* means = s->means_acc.as<float>();
+    float* sink = s->rsink.as<float>();
+    for (uint32_t done = 0; done < nsteps; done += chunk) {
+        unsigned n = std::min(chunk, nsteps - done), step = step0 + done;
+        unsigned kp = Kp;
+        void* da[] = {&seed_odd, &seed_even, &c_odd, &c_even, &K, &kp, &a, &step, &n, &partner,
+                      &draws};
+        BH_HIP(hipModuleLaunchKernel(s->f->draws, (K + 255) / 256, std::min(2 * n, 65535u), 1, 256,
+                                     1, 1, 0, s->stream, da, nullptr));
+        const float* betas = d_betas ? d_betas + done : nullptr;
+        float* out = accu ? s->rtrace.as<float>() : nullptr;
+        if (sample_out) out = sample_out + step_floats * done;
+        void* ra[] = {&drawsc, &data_len, &params_len, &params, &xs,  &lf,  &K,
+                      &beta,   &betas,    &n,          &partner, &acc, &out, &sink};
+        BH_TRY(ktimed(s, [&] {
+            return launch(out ? s->f->resident_out : s->f->resident, 1, nb,
+                          (unsigned)resident_lds(s), s->stream, ra);
+        }));
+        if (accu) {
+            const float* trace = s->rtrace.as<float>();
+            void* ta[] = {&trace, &K, &step, &means};
+            BH_HIP(hipModuleLaunchKernel(s->f->trace_accu, s->groups, n, 1, s->wgs, 1, 1, 0,
+                                         s->stream, ta, nullptr));
+        }
+    }
+    return BH_OK;
 }
 
 // ---------------------------------------------------------------- GLM
@@ -827,7 +891,7 @@ int accu_pair(bh_stretch* s) {
 
 int bare_steps(bh_stretch* s, uint64_t n, const float* h_betas) {
     if (n == 0) return BH_OK;
-    if (use_resident(s, 0)) {
+    if (use_resident(s)) {
         DevBuf d_betas;
         const float* db = nullptr;
         if (h_betas) {
@@ -840,9 +904,8 @@ int bare_steps(bh_stretch* s, uint64_t n, const float* h_betas) {
         uint64_t done = 0;
         while (done < n) {
             const uint32_t chunk = (uint32_t)std::min<uint64_t>(n - done, 1u << 20);
-            BH_TRY(run_resident(s, 0, s->bare_seed, s->bare_seed + 1u, 3333, 4444, s->bare_a,
-                                s->beta, db ? db + done : nullptr, s->bare_counter, chunk, nullptr,
-                                0));
+            BH_TRY(run_resident(s, false, s->bare_seed, s->bare_seed + 1u, 3333, 4444, s->bare_a,
+                                s->beta, db ? db + done : nullptr, s->bare_counter, chunk, nullptr));
             s->bare_counter += chunk;
             done += chunk;
         }
@@ -878,9 +941,9 @@ int accu_steps(bh_stretch* s, uint64_t n) {
         return fail(BH_ERR_STATE, "move! beyond the %llu steps reserved by init-move!",
                     (unsigned long long)s->means_cap);
     if (n == 0) return BH_OK;
-    if (use_resident(s, 1)) {
-        BH_TRY(run_resident(s, 1, s->move_seed, s->move_seed + 1u, 1111, 2222, s->accu_a, 1.0f,
-                            nullptr, s->move_counter, (uint32_t)n, nullptr, 0));
+    if (use_resident(s)) {
+        BH_TRY(run_resident(s, true, s->move_seed, s->move_seed + 1u, 1111, 2222, s->accu_a, 1.0f,
+                            nullptr, s->move_counter, (uint32_t)n, nullptr));
         s->move_counter += (uint32_t)n;
         return sync(s->stream);
     }
@@ -1016,6 +1079,7 @@ int bh_ctx_create(int device, uint32_t wgs, bh_ctx** out) {
     c->device = device;
     c->wgs = wgs;
     c->cu = prop.multiProcessorCount;
+    BH_HIP(hipDeviceGetAttribute(&c->lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, device));
     std::string arch = prop.gcnArchName;
     c->arch = arch.substr(0, arch.find(':'));
     // the address of this device's copy of bh_dataset_variance_noalloc's
@@ -1523,6 +1587,9 @@ int bh_stretch_factory_create(bh_ctx* ctx, const char* source, const char* logfn
     BH_TRY(f->mod.fn("bh_stretch_move_bare", &f->bare));
     BH_TRY(f->mod.fn("bh_stretch_move_accu", &f->accu));
     BH_TRY(f->mod.fn("bh_stretch_resident", &f->resident));
+    BH_TRY(f->mod.fn("bh_stretch_resident_out", &f->resident_out));
+    BH_TRY(f->mod.fn("bh_stretch_draws", &f->draws));
+    BH_TRY(f->mod.fn("bh_trace_accu", &f->trace_accu));
     *out = f.release();
     return BH_OK;
 }
@@ -1793,7 +1860,7 @@ int bh_stretch_set_exec(bh_stretch* s, int mode) {
     BH_ARG(s, "NULL sampler");
     BH_ARG(mode == BH_EXEC_AUTO || mode == BH_EXEC_STEPWISE || mode == BH_EXEC_RESIDENT,
            "unknown execution mode %d", mode);
-    if (mode == BH_EXEC_RESIDENT && resident_lds(s, 1) > kResidentLdsMax)
+    if (mode == BH_EXEC_RESIDENT && !resident_accepted(s))
         return fail(BH_ERR_RANGE, "ensemble (%u walkers x %u) does not fit in one work-group's LDS",
                     s->W, s->dim);
     s->exec = mode;
@@ -2920,9 +2987,19 @@ int bh_stretch_sample(bh_stretch* s, float* out, uint64_t ncols) {
     DevOut o;
     BH_TRY(o.init(out, req * sizeof(float)));
     Timed t(s);
-    if (use_resident(s, 0) && steps < (1ull << 31)) {
-        BH_TRY(run_resident(s, 0, s->bare_seed, s->bare_seed + 1u, 3333, 4444, s->bare_a, 1.0f,
-                            nullptr, s->bare_counter, (uint32_t)steps, o.as<float>(), req));
+    if (use_resident(s) && steps < (1ull << 31)) {
+        // whole ensembles straight into the output; of a last part, its step
+        // and a copy
+        const uint32_t whole = (uint32_t)(req / avail);
+        BH_TRY(run_resident(s, false, s->bare_seed, s->bare_seed + 1u, 3333, 4444, s->bare_a, 1.0f,
+                            nullptr, s->bare_counter, whole, o.as<float>()));
+        if (whole < steps) {
+            BH_TRY(run_resident(s, false, s->bare_seed, s->bare_seed + 1u, 3333, 4444, s->bare_a,
+                                1.0f, nullptr, s->bare_counter + whole, 1, nullptr));
+            BH_HIP(hipMemcpyAsync(o.as<float>() + (size_t)whole * avail, s->xs.p,
+                                  (req - (size_t)whole * avail) * sizeof(float),
+                                  hipMemcpyDeviceToDevice, s->stream));
+        }
         s->bare_counter += (uint32_t)steps;
     } else {
         uint64_t ofst = 0;

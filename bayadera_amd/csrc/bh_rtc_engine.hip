@@ -295,47 +295,6 @@ bh_logfn(unsigned data_len, unsigned params_len, const float* __restrict__ param
     if (w < n) res[w] = LOGFN(data_len, params_len, params, DIM, x + (size_t)w * DIM);
 }
 
-// The same accounting inside the resident kernel, without global
-// read-modify-writes in the step loop: a slice's accept count goes to LDS
-// (acc_lds[g], added to accept[g] once at the end of the launch), the odd
-// half's per-group sums wait in LDS (odd_lds[g][d]) and the even half stores
-// (0 + odd) + even to the step's means slot -- the value the two
-// read-modify-writes of the per-half-step kernels leave in a zeroed slot.
-__device__ __forceinline__ void bh_accu_resident(const float (&xk)[DIM], bool accepted, unsigned g,
-                                                 unsigned groups, unsigned mstep, int half,
-                                                 unsigned* acc_lds, float* odd_lds, float* means,
-                                                 float* red, unsigned* wave_counts,
-                                                 bool last_pass) {
-    const bool leader = (threadIdx.x & (WGS - 1)) == 0;
-    float* m = means + (size_t)groups * DIM * mstep + g;
-#pragma unroll
-    for (int d0 = 0; d0 < DIM; d0 += BH_ACCU_CHUNK) {
-        float v[BH_ACCU_CHUNK], sums[BH_ACCU_CHUNK];
-#pragma unroll
-        for (int c = 0; c < BH_ACCU_CHUNK; ++c) v[c] = (d0 + c < DIM) ? xk[d0 + c] : 0.0f;
-        // the half-step's own barrier follows its last pass over walkers
-        const bool sync = d0 + BH_ACCU_CHUNK < DIM || !last_pass;
-        if (d0 == 0) {
-            unsigned cnt;
-            bh_slice_count_tree_sums<BH_ACCU_CHUNK>(accepted, v, red, wave_counts, sums, cnt,
-                                                    sync);
-            if (leader) acc_lds[g] += cnt;
-        } else {
-            bh_slice_tree_sums<BH_ACCU_CHUNK>(v, red, sums, sync);
-        }
-        if (leader) {
-#pragma unroll
-            for (int c = 0; c < BH_ACCU_CHUNK; ++c) {
-                if (d0 + c < DIM) {
-                    float* o = odd_lds + (size_t)g * DIM + d0 + c;
-                    if (half == 0) *o = sums[c];
-                    else m[(size_t)(d0 + c) * groups] = (0.0f + *o) + sums[c];
-                }
-            }
-        }
-    }
-}
-
 // One half-step over K walkers, one thread per walker, WGS walkers per block
 // (stretch_move_bare / stretch_move_accu, amd-gcn-mcmc-stretch.cl:83-134).
 // The walker's own record and log density are read and written once per
@@ -600,112 +559,333 @@ bh_stretch_move_accu(unsigned seed, unsigned odd_or_even, unsigned data_len,
                                                  S, X, logfn_X, a, 1.0f, step, K, accept, means);
 }
 
-// Resident multi-step kernel: one work-group holds the whole ensemble
-// (positions and logfn values) in LDS and runs nsteps full steps -- both
-// half-steps each -- without returning to the host.  Every walker's
-// arithmetic and every accounting tree is the same as in the per-half-step
-// kernels, so the results are bit-identical; what goes away is two kernel
-// launches per step, which bound small ensembles (W = 1024: 16 KB of state).
-//   mode 0: bare steps (burn-in!, anneal! with betas[s], sample! with out)
-//   mode 1: accounting steps (move!): accept/means as stretch_move_accu
-// blockDim.x is a multiple of WGS dividing K.
-template <int PARTNER>
-__device__ __forceinline__ void bh_resident_impl(
-    unsigned seed_odd, unsigned seed_even, unsigned c_odd, unsigned c_even, unsigned data_len,
-    unsigned params_len, const float* __restrict__ params, float* __restrict__ xs,
-    float* __restrict__ logfn, unsigned K, float a, float beta, const float* __restrict__ betas,
-    unsigned step0, unsigned nsteps, int mode, unsigned* __restrict__ accept,
-    float* __restrict__ means, float* __restrict__ sample_out, unsigned long long sample_floats) {
-    extern __shared__ __attribute__((aligned(16))) float lds[];
-    const unsigned W = 2 * K;
-    const unsigned nb = blockDim.x;
-    const unsigned t = threadIdx.x;
-    float* sx = lds;                       // W*DIM
-    float* sl = sx + (size_t)W * DIM;      // W
-    float* red = sl + W;                   // BH_ACCU_CHUNK*nb (mode 1)
-    const unsigned groups = K / WGS;
-    float* odd_lds = red + (mode == 1 ? BH_ACCU_CHUNK * nb : 0);       // groups*DIM (mode 1)
-    unsigned* acc_lds = (unsigned*)(odd_lds + (mode == 1 ? groups * DIM : 0));  // groups
-    unsigned* wave_counts = acc_lds + (mode == 1 ? groups : 0);
-    for (unsigned i = t; i < W * DIM; i += nb) sx[i] = xs[i];
-    for (unsigned i = t; i < W; i += nb) sl[i] = logfn[i];
-    if (mode == 1)
-        for (unsigned i = t; i < groups; i += nb) acc_lds[i] = 0u;
-    __syncthreads();
-    unsigned long long written = 0;
-    for (unsigned s = 0; s < nsteps; ++s) {
-        const unsigned step = step0 + s;
-        const float b = betas ? betas[s] : beta;
-        for (int h = 0; h < 2; ++h) {
-            float* X = sx + (h ? (size_t)K * DIM : 0);
-            const float* S = sx + (h ? 0 : (size_t)K * DIM);
-            float* L = sl + (h ? K : 0);
-            const unsigned seed = h ? seed_even : seed_odd;
-            const unsigned oe = h ? c_even : c_odd;
-            for (unsigned k0 = 0; k0 < K; k0 += nb) {
-                const unsigned k = k0 + t;
-                float xk[DIM];
-#pragma unroll
-                for (int i = 0; i < DIM; ++i) xk[i] = X[(size_t)k * DIM + i];
-                float lx = L[k];
-                const bool acc = bh_stretch_walker<PARTNER>(k, K, seed, oe, step, a,
-                                                            mode == 1 ? 1.0f : b, S, xk, lx,
-                                                            data_len, params_len, params);
-                if (acc) {
-#pragma unroll
-                    for (int i = 0; i < DIM; ++i) X[(size_t)k * DIM + i] = xk[i];
-                    L[k] = lx;
-                }
-                if (mode == 1)
-                    bh_accu_resident(xk, acc, k / WGS, groups, step, h, acc_lds, odd_lds, means,
-                                     red, wave_counts, k0 + nb >= K);
-            }
-            __syncthreads();
-        }
-        if (sample_out && written < sample_floats) {
-            const unsigned long long left = sample_floats - written;
-            const unsigned chunk = left < (unsigned long long)W * DIM ? (unsigned)left : W * DIM;
-            float* dst = sample_out + written;
-            if (((unsigned long long)dst & 15ull) == 0 && chunk % 4 == 0) {
-                // 16-byte pieces (the LDS ensemble starts 16-byte aligned)
-                const float4* src4 = reinterpret_cast<const float4*>(sx);
-                float4* dst4 = reinterpret_cast<float4*>(dst);
-                for (unsigned i = t; i < chunk / 4; i += nb) dst4[i] = src4[i];
-            } else {
-                for (unsigned i = t; i < chunk; i += nb) dst[i] = sx[i];
-            }
-            written += chunk;
-            // the next step's first half writes accepted proposals into sx:
-            // every wave finishes copying this step's ensemble first (the
-            // condition is uniform over the work-group)
-            __syncthreads();
-        }
-    }
-    for (unsigned i = t; i < W * DIM; i += nb) xs[i] = sx[i];
-    for (unsigned i = t; i < W; i += nb) logfn[i] = sl[i];
-    if (mode == 1) {
-        __syncthreads();
-        for (unsigned i = t; i < groups; i += nb) accept[i] += acc_lds[i];
+// Small ensembles: one work-group holds the whole ensemble (positions and
+// log densities) in LDS and runs many full steps without returning to the
+// host, so that no launch sits between half-steps.  What bounds it is then
+// what one compute unit must do per half-step, in sequence, and two thirds of
+// that does not depend on the ensemble: the draws (Philox alone is ~20
+// quarter-rate multiplies per walker) and the accounting's trees (two barriers
+// and a reduction per half-step).  With both inside, 1024 walkers x 4 took 1.5
+// us per bare step and 2.9 per accounted one; without, 0.69 and 0.73.  So each
+// chunk of steps is three launches:
+//   bh_stretch_draws     z, the partner's offset, u2 and z^(DIM-1) of every
+//                        walker of every half-step of the chunk (whole chip)
+//   bh_stretch_resident  the steps: partner from LDS, density, accept test;
+//                        the positions after each half-step go to a trace
+//                        (accounting) or straight to the caller's samples
+//   bh_trace_accu        the accounting's sums of every step from the trace
+//                        (whole chip)
+// Every walker's arithmetic and every tree is that of the per-half-step
+// kernels, so the results are bit-identical.
+
+// Draw i of the launch is half-step i / Kp, walker i % Kp of the Kp >= K
+// slots per half-step (those past K are not filled).
+extern "C" __global__ void __launch_bounds__(256)
+bh_stretch_draws(unsigned seed_odd, unsigned seed_even, unsigned c_odd, unsigned c_even,
+                 unsigned K, unsigned Kp, float a, unsigned step0, unsigned nsteps, int partner,
+                 float4* __restrict__ draws) {
+    const unsigned k = blockIdx.x * 256 + threadIdx.x;
+    if (k >= K) return;
+    for (unsigned hs = blockIdx.y; hs < 2 * nsteps; hs += gridDim.y) {
+        const bool even = hs & 1u;
+        const unsigned seed = even ? seed_even : seed_odd, oe = even ? c_even : c_odd;
+        const unsigned step = step0 + hs / 2;
+        float z;
+        unsigned e;
+        const float u2 =
+            partner == BH_PARTNER_FLAT
+                ? bh_stretch_draw<BH_PARTNER_FLAT>(k, K, seed, oe, step, a, z, e)
+                : bh_stretch_draw<BH_PARTNER_WALKER>(k, K, seed, oe, step, a, z, e);
+        draws[(size_t)hs * Kp + k] = make_float4(z, __uint_as_float(e), u2, bh_zpow(z));
     }
 }
 
-extern "C" __global__ void __launch_bounds__(1024)
-bh_stretch_resident(unsigned seed_odd, unsigned seed_even, unsigned c_odd, unsigned c_even,
-                    unsigned data_len, unsigned params_len, const float* __restrict__ params,
-                    float* __restrict__ xs, float* __restrict__ logfn, unsigned K, float a,
-                    float beta, const float* __restrict__ betas, unsigned step0,
-                    unsigned nsteps, int partner, int mode, unsigned* __restrict__ accept,
-                    float* __restrict__ means, float* __restrict__ sample_out,
-                    unsigned long long sample_floats) {
-    if (partner == BH_PARTNER_FLAT)
-        bh_resident_impl<BH_PARTNER_FLAT>(seed_odd, seed_even, c_odd, c_even, data_len,
-                                          params_len, params, xs, logfn, K, a, beta, betas, step0,
-                                          nsteps, mode, accept, means, sample_out, sample_floats);
-    else
-        bh_resident_impl<BH_PARTNER_WALKER>(seed_odd, seed_even, c_odd, c_even, data_len,
-                                            params_len, params, xs, logfn, K, a, beta, betas,
-                                            step0, nsteps, mode, accept, means, sample_out,
-                                            sample_floats);
+// Floats from one half-ensemble to the next in LDS: the K * DIM coordinates,
+// then the first DIM - 1 of them again, so that a FLAT partner's coordinates
+// are read without wrapping; a multiple of 4, so that records stay aligned.
+__device__ __forceinline__ unsigned bh_resident_half(unsigned K) {
+    return (K * DIM + DIM - 1 + 3) / 4 * 4;
+}
+
+// The ensemble in LDS: both halves, then the log densities, then the accept
+// counts per group of WGS walkers.
+__device__ __forceinline__ void bh_resident_load(float* sx, unsigned H, unsigned K,
+                                                 const float* __restrict__ xs) {
+    for (unsigned h = 0; h < 2; ++h) {
+        for (unsigned i = threadIdx.x; i < K * DIM; i += blockDim.x)
+            sx[h * H + i] = xs[h * K * DIM + i];
+        for (unsigned i = threadIdx.x; i < DIM - 1; i += blockDim.x)
+            sx[h * H + K * DIM + i] = xs[h * K * DIM + i];
+    }
+}
+
+template <int PARTNER>
+__device__ __forceinline__ void bh_resident_partner(const float* S, unsigned e,
+                                                    float (&sj)[DIM]) {
+    if constexpr (PARTNER == BH_PARTNER_FLAT) {
+#pragma unroll
+        for (int i = 0; i < DIM; ++i) sj[i] = S[e + i];
+    } else {
+        bh_load_walker(S + e, sj);
+    }
+}
+
+template <int PARTNER>
+__device__ __forceinline__ void bh_resident_accept(float* X, unsigned K, unsigned k,
+                                                   const float (&y)[DIM]) {
+    bh_store_walker(X + k * DIM, y);
+    if (PARTNER == BH_PARTNER_FLAT && DIM > 1 && k == 0) {
+#pragma unroll
+        for (int i = 0; i < DIM - 1; ++i) X[K * DIM + i] = y[i];
+    }
+}
+
+// Each thread keeps the draws of its next BH_RESIDENT_AHEAD walkers in
+// flight: they come from another XCD's writes, some 0.7 us away, a half-step
+// takes 0.35.  These loads, and the stores of the positions, sit in no
+// branch: the hardware retires both in order through one counter, and only
+// where every path issues the same number of them can the compiler wait for
+// the one load it needs instead of for all (which would be 0.7 us every
+// half-step).  For the same reason the loops have one way out, after whole
+// rounds of BH_RESIDENT_AHEAD; in what is past the last half-step nothing is
+// decided and the positions go to `sink` (K * DIM floats).
+#define BH_RESIDENT_AHEAD 4
+
+// nsteps steps with one walker of each half per thread (blockDim.x == K): the
+// thread's own records and log densities stay in registers, LDS holds what
+// the other half reads.  Eight waves share four SIMDs, so at 1024 walkers the
+// half-step takes the instructions it issues, ~65 VALU at dim 4 (500 of its
+// 830 cycles, the rest LDS and barrier latency); the general form below reads
+// and addresses everything anew: 1.1 us per step where this takes 0.73.
+//   draws: K per half-step, and 2 * BH_RESIDENT_AHEAD * K more that are read
+//        but not used
+//   betas: one inverse temperature per step, or null (beta for all)
+//   out (OUT): the positions after each half-step, half after half
+//   accept: null, or the accept counts per group of WGS walkers, added to
+template <int PARTNER, bool OUT>
+__device__ __forceinline__ void bh_resident_one(
+    const float4* __restrict__ draws, unsigned data_len, unsigned params_len,
+    const float* __restrict__ params, float* __restrict__ xs, float* __restrict__ logfn,
+    unsigned K, float beta, const float* __restrict__ betas, unsigned nsteps,
+    unsigned* __restrict__ accept, float* __restrict__ out, float* __restrict__ sink) {
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    static_assert(BH_RESIDENT_AHEAD == 4, "two steps per round");
+    typedef float bh_f4 __attribute__((ext_vector_type(4)));
+    const unsigned k = threadIdx.x, H = bh_resident_half(K);
+    float* sx = lds;
+    bh_resident_load(sx, H, K, xs);
+    float x[2][DIM], lx[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        bh_load_walker(xs + ((size_t)h * K + k) * DIM, x[h]);
+        lx[h] = logfn[h * K + k];
+    }
+    const bh_f4* dp = reinterpret_cast<const bh_f4*>(draws);
+    bh_f4 d[BH_RESIDENT_AHEAD];
+#pragma unroll
+    for (int r = 0; r < BH_RESIDENT_AHEAD; ++r) {
+        d[r] = dp[k];
+        dp += K;
+        __builtin_amdgcn_sched_barrier(0);  // in this order, which the waits count on
+    }
+    unsigned count = 0;  // of the wave's walkers, which are of one group
+    float b[2] = {beta, beta};
+    __syncthreads();
+    for (unsigned s = 0; s < nsteps; s += 2) {
+        if (betas) {
+            b[0] = betas[s];
+            b[1] = betas[s + 1 < nsteps ? s + 1 : s];
+        }
+#pragma unroll
+        for (int r = 0; r < BH_RESIDENT_AHEAD; ++r) {
+            constexpr int NH = 2;
+            const int h = r % NH;
+            const bool live = r < NH || s + 1 < nsteps;  // (uniform)
+            // (used as a whole, so that the draw goes round the loop in one
+            // register tuple: copied in parts it would be waited for there)
+            asm volatile("" : "+v"(d[r]));
+            float* X = sx + (h ? H : 0u);
+            float sj[DIM], y[DIM];
+            bh_resident_partner<PARTNER>(sx + (h ? 0u : H), live ? __float_as_uint(d[r].y) : 0u, sj);
+#pragma unroll
+            for (int i = 0; i < DIM; ++i) y[i] = __builtin_fmaf(d[r].x, x[h][i] - sj[i], sj[i]);
+            const float ly = LOGFN(data_len, params_len, params, DIM, y);
+            // (u2 > 0: a log density that is not finite is never accepted)
+            const float q = d[r].w * expf(b[r / NH] * (ly - lx[h]));
+            const bool acc = live && __builtin_isfinite(ly) && d[r].z <= q;
+#pragma unroll
+            for (int i = 0; i < DIM; ++i) x[h][i] = acc ? y[i] : x[h][i];
+            lx[h] = acc ? ly : lx[h];
+            if (acc) bh_resident_accept<PARTNER>(X, K, k, x[h]);
+            count += (unsigned)__popcll(__ballot(acc));
+            if constexpr (OUT) {
+                float* dst = live ? out : sink;
+#pragma unroll
+                for (int i = 0; i < DIM; ++i) dst[k * DIM + i] = x[h][i];
+                out += K * DIM;
+            }
+            d[r] = dp[k];  // BH_RESIDENT_AHEAD half-steps on, into the registers now free
+            dp += K;
+            __syncthreads();
+        }
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        bh_store_walker(xs + ((size_t)h * K + k) * DIM, x[h]);
+        logfn[h * K + k] = lx[h];
+    }
+    if (accept && (k & 63u) == 0) atomicAdd(&accept[k / WGS], count);
+}
+
+// The same for larger halves, slots = ceil(K / blockDim.x) walkers per thread
+// and half (draws: slots * blockDim.x per half-step, and 2 *
+// BH_RESIDENT_AHEAD * blockDim.x more); threads past K take walker K - 1,
+// decide nothing and write to the sink.
+template <int PARTNER, bool OUT>
+__device__ __forceinline__ void bh_resident_slots(
+    const float4* __restrict__ draws, unsigned data_len, unsigned params_len,
+    const float* __restrict__ params, float* __restrict__ xs, float* __restrict__ logfn,
+    unsigned K, float beta, const float* __restrict__ betas, unsigned nsteps,
+    unsigned* __restrict__ accept, float* __restrict__ out, float* __restrict__ sink) {
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    typedef float bh_f4 __attribute__((ext_vector_type(4)));
+    const unsigned nb = blockDim.x, t = threadIdx.x;
+    const unsigned H = bh_resident_half(K), W = 2 * K, groups = K / WGS;
+    float* sx = lds;                          // 2 H
+    float* sl = sx + 2 * H;                   // W
+    unsigned* acc_lds = (unsigned*)(sl + W);  // groups
+    bh_resident_load(sx, H, K, xs);
+    for (unsigned i = t; i < W; i += nb) sl[i] = logfn[i];
+    for (unsigned i = t; i < groups; i += nb) acc_lds[i] = 0u;
+    const unsigned total = 2 * nsteps * ((K + nb - 1) / nb);
+    const bh_f4* dp = reinterpret_cast<const bh_f4*>(draws) + t;
+    bh_f4 d[BH_RESIDENT_AHEAD];
+#pragma unroll
+    for (int r = 0; r < BH_RESIDENT_AHEAD; ++r) {
+        d[r] = *dp;
+        dp += nb;
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    float b = betas ? betas[0] : beta;
+    float b_next = betas && nsteps > 1 ? betas[1] : beta;
+    unsigned h = 0, k0 = 0, s = 0;
+    __syncthreads();
+    for (unsigned i0 = 0; i0 < total; i0 += BH_RESIDENT_AHEAD) {
+#pragma unroll
+        for (int r = 0; r < BH_RESIDENT_AHEAD; ++r) {
+            const unsigned kt = k0 + t;
+            const bool live = kt < K && i0 + r < total;
+            const unsigned k = kt < K ? kt : K - 1;
+            asm volatile("" : "+v"(d[r]));
+            float* X = sx + h * H;
+            float xk[DIM], sj[DIM], y[DIM];
+            bh_resident_partner<PARTNER>(sx + (h ^ 1u) * H, live ? __float_as_uint(d[r].y) : 0u, sj);
+            bh_load_walker(X + k * DIM, xk);
+            const float lx = sl[h * K + k];
+#pragma unroll
+            for (int i = 0; i < DIM; ++i) y[i] = __builtin_fmaf(d[r].x, xk[i] - sj[i], sj[i]);
+            const float ly = LOGFN(data_len, params_len, params, DIM, y);
+            const float q = d[r].w * expf(b * (ly - lx));
+            const bool acc = live && __builtin_isfinite(ly) && d[r].z <= q;
+#pragma unroll
+            for (int i = 0; i < DIM; ++i) xk[i] = acc ? y[i] : xk[i];
+            if (acc) {
+                bh_resident_accept<PARTNER>(X, K, k, xk);
+                sl[h * K + k] = ly;
+            }
+            if constexpr (OUT) {
+                float* dst = live ? out : sink;
+#pragma unroll
+                for (int i = 0; i < DIM; ++i) dst[(size_t)k * DIM + i] = xk[i];
+            }
+            if (accept) {
+                const unsigned long long m = __ballot(acc);
+                if ((t & 63u) == 0) atomicAdd(&acc_lds[k / WGS], (unsigned)__popcll(m));
+            }
+            d[r] = *dp;
+            dp += nb;
+            k0 += nb;
+            if (k0 >= K) {
+                k0 = 0;
+                if constexpr (OUT) out += K * DIM;
+                if (h) {
+                    ++s;
+                    b = b_next;
+                    if (betas && s + 1 < nsteps) b_next = betas[s + 1];
+                }
+                h ^= 1u;
+                __syncthreads();
+            }
+        }
+    }
+    for (unsigned hh = 0; hh < 2; ++hh)
+        for (unsigned i = t; i < K * DIM; i += nb) xs[hh * K * DIM + i] = sx[hh * H + i];
+    for (unsigned i = t; i < W; i += nb) logfn[i] = sl[i];
+    if (accept)
+        for (unsigned i = t; i < groups; i += nb) accept[i] += acc_lds[i];
+}
+
+// With and without positions to write: two kernels, so that each has its own
+// registers and its own loops.
+#define BH_RESIDENT_KERNEL(NAME, OUT)                                                             \
+    extern "C" __global__ void __launch_bounds__(1024) NAME(                                      \
+        const float4* __restrict__ draws, unsigned data_len, unsigned params_len,                 \
+        const float* __restrict__ params, float* __restrict__ xs, float* __restrict__ logfn,      \
+        unsigned K, float beta, const float* __restrict__ betas, unsigned nsteps, int partner,    \
+        unsigned* __restrict__ accept, float* __restrict__ out, float* __restrict__ sink) {       \
+        if (blockDim.x == K) {                                                                    \
+            if (partner == BH_PARTNER_FLAT)                                                       \
+                bh_resident_one<BH_PARTNER_FLAT, OUT>(draws, data_len, params_len, params, xs,    \
+                                                      logfn, K, beta, betas, nsteps, accept, out, \
+                                                      sink);                                      \
+            else                                                                                  \
+                bh_resident_one<BH_PARTNER_WALKER, OUT>(draws, data_len, params_len, params, xs,  \
+                                                        logfn, K, beta, betas, nsteps, accept,    \
+                                                        out, sink);                               \
+        } else if (partner == BH_PARTNER_FLAT) {                                                  \
+            bh_resident_slots<BH_PARTNER_FLAT, OUT>(draws, data_len, params_len, params, xs,      \
+                                                    logfn, K, beta, betas, nsteps, accept, out,   \
+                                                    sink);                                        \
+        } else {                                                                                  \
+            bh_resident_slots<BH_PARTNER_WALKER, OUT>(draws, data_len, params_len, params, xs,    \
+                                                      logfn, K, beta, betas, nsteps, accept, out, \
+                                                      sink);                                      \
+        }                                                                                         \
+    }
+BH_RESIDENT_KERNEL(bh_stretch_resident, false)
+BH_RESIDENT_KERNEL(bh_stretch_resident_out, true)
+#undef BH_RESIDENT_KERNEL
+
+// The accounting of stretch_move_accu for steps step0 .. step0 + gridDim.y
+// from their traced positions (each step's two halves of K records): the
+// group sums of the odd half, then (0 + odd) + even, the value the two
+// read-modify-writes of the per-half-step kernels leave in a zeroed slot.
+// One work-group per group and step.
+extern "C" __global__ void __launch_bounds__(WGS)
+bh_trace_accu(const float* __restrict__ trace, unsigned K, unsigned step0,
+              float* __restrict__ means) {
+    __shared__ float red[BH_ACCU_CHUNK * WGS];
+    const unsigned g = blockIdx.x, groups = gridDim.x, t = threadIdx.x;
+    const float* rec = trace + ((size_t)blockIdx.y * 2 * K + g * WGS + t) * DIM;
+    float xo[DIM], xe[DIM];
+    bh_load_walker(rec, xo);
+    bh_load_walker(rec + (size_t)K * DIM, xe);
+    float* m = means + (size_t)groups * DIM * (step0 + blockIdx.y) + g;
+#pragma unroll
+    for (int d0 = 0; d0 < DIM; d0 += BH_ACCU_CHUNK) {
+        float v[BH_ACCU_CHUNK], odd[BH_ACCU_CHUNK], even[BH_ACCU_CHUNK];
+#pragma unroll
+        for (int c = 0; c < BH_ACCU_CHUNK; ++c) v[c] = d0 + c < DIM ? xo[d0 + c] : 0.0f;
+        bh_slice_tree_sums<BH_ACCU_CHUNK>(v, red, odd);
+#pragma unroll
+        for (int c = 0; c < BH_ACCU_CHUNK; ++c) v[c] = d0 + c < DIM ? xe[d0 + c] : 0.0f;
+        bh_slice_tree_sums<BH_ACCU_CHUNK>(v, red, even, d0 + BH_ACCU_CHUNK < DIM);
+        if (t == 0) {
+#pragma unroll
+            for (int c = 0; c < BH_ACCU_CHUNK; ++c)
+                if (d0 + c < DIM) m[(size_t)(d0 + c) * groups] = (0.0f + odd[c]) + even[c];
+        }
+    }
 }
 
 #endif  // LOGFN
