@@ -308,8 +308,13 @@ struct bh_stretch_factory {
     bh_ctx* ctx = nullptr;
     uint32_t dim = 0, params_len = 0;
     Module mod;
-    hipFunction_t logfn = nullptr, bare = nullptr, accu = nullptr, resident = nullptr,
-                  resident_out = nullptr, draws = nullptr, trace_accu = nullptr;
+    hipFunction_t logfn = nullptr, bare = nullptr, accu = nullptr;
+    // the resident steps' kernels, compiled for the first sampler that takes them
+    std::string source, logfn_name;
+    std::mutex resident_mu;
+    Module resident_mod;
+    hipFunction_t resident = nullptr, resident_out = nullptr, draws = nullptr,
+                  trace_accu = nullptr;
     std::unique_ptr<GlmData> glm;
     hipFunction_t glm_propose = nullptr, glm_split = nullptr, glm_logpost = nullptr,
                   glm_accept = nullptr, glm_screen = nullptr, glm_resolve = nullptr,
@@ -385,17 +390,18 @@ constexpr size_t kKernelTimerPairs = 1024;
 
 // When an ensemble that fits in one compute unit's LDS runs there (see
 // use_resident).  Steps, per-half-step kernels against resident, us per bare /
-// accounted step:
-//   1024 walkers   dim 4   5.1 / 8.5 -> 0.7 / 0.8    dim 24  17 / 27 -> 11 / 10
-//   4096           dim 1   5.3 / 7.5 -> 3.0 / 2.6    dim 7  6.8 / 12 -> 5.0 / 5.2
-//   8192           dim 1   5.3 / 7.6 -> 3.8 / 5.1    dim 2  5.3 / 8.2 -> 5.1 / 4.7
-//   12,288         dim 2   5.2 / 8.4 -> 5.7 / 7.5
+// accounted step (correlated Gaussian):
+//   1024 walkers   dim 4   5.7 / 8.0 -> 0.7 / 0.9    dim 24  17 / 27 -> 11 / 10
+//   4096           dim 1   6.3 / 7.8 -> 1.4 / 1.9    dim 7   7.3 / 12 -> 3.6 / 4.7
+//   8192           dim 1   5.7 / 7.6 -> 2.6 / 3.5    dim 2   5.7 / 7.7 -> 3.0 / 4.1
+// A half-step takes as long as its passes of 1024 walkers, so the line is
+// where six of them reach the launches' 2.8 us.
 // A density that loops over data keeps one compute unit busy for longer than
 // the launches take on all of them (gaussian likelihood, bare): 50 values,
 // 1024 walkers 12.6 -> 7.0, 2048 12.9 -> 13.6, 4096 13.8 -> 23; 5000 values,
 // 1024 walkers 929 -> 535, 2048 930 -> 1216.  So past 1024 walkers the data
 // and the parameters a step reads are bounded too.
-constexpr uint32_t kResidentWalkers = 8192;
+constexpr uint32_t kResidentWalkers = 12288;
 constexpr uint32_t kResidentAnyDensity = 1024;
 constexpr uint64_t kResidentData = 100000;
 constexpr uint64_t kResidentParams = 1000000;
@@ -504,6 +510,26 @@ bool use_resident(const bh_stretch* s) {
             (uint64_t)s->params_count * s->W <= kResidentParams);
 }
 
+// The resident kernels of a sampler's factory: a module of their own, since
+// compiling a user's density into them takes as long as the rest (mvn of 4
+// dimensions 0.6 s) and larger ensembles do not need them.  Compiled when a
+// sampler is made that takes them, not in its first steps.
+int resident_module(bh_stretch_factory* f) {
+    std::lock_guard<std::mutex> lk(f->resident_mu);
+    if (f->draws) return BH_OK;
+    BH_HIP(hipSetDevice(f->ctx->device));
+    std::vector<char> code;
+    BH_TRY(rtc_compile(f->ctx->arch, f->source,
+                       {"-DWGS=" + std::to_string(f->ctx->wgs), "-DDIM=" + std::to_string(f->dim),
+                        "-DLOGFN=" + f->logfn_name, "-DBH_RESIDENT=1"},
+                       code, nullptr, 0));
+    if (!f->resident_mod.mod) BH_TRY(f->resident_mod.load(code));
+    BH_TRY(f->resident_mod.fn("bh_stretch_resident", &f->resident));
+    BH_TRY(f->resident_mod.fn("bh_stretch_resident_out", &f->resident_out));
+    BH_TRY(f->resident_mod.fn("bh_trace_accu", &f->trace_accu));
+    return f->resident_mod.fn("bh_stretch_draws", &f->draws);
+}
+
 // nsteps resident steps: per chunk the draws, the steps and, with accu, the
 // accounting from their trace; with sample_out the positions after every
 // step go there (nsteps whole ensembles).
@@ -511,6 +537,7 @@ int run_resident(bh_stretch* s, bool accu, uint32_t seed_odd, uint32_t seed_even
                  uint32_t c_even, float a, float beta, const float* d_betas, uint32_t step0,
                  uint32_t nsteps, float* sample_out) {
     if (nsteps == 0) return BH_OK;
+    BH_TRY(resident_module(s->f));
     const unsigned nb = resident_block(s), Kp = nb * resident_slots(s);
     const size_t draw_bytes = (size_t)2 * Kp * 16;
     const size_t step_floats = (size_t)s->W * s->dim;
@@ -541,8 +568,8 @@ int run_resident(bh_stretch* s, bool accu, uint32_t seed_odd, uint32_t seed_even
         const float* betas = d_betas ? d_betas + done : nullptr;
         float* out = accu ? s->rtrace.as<float>() : nullptr;
         if (sample_out) out = sample_out + step_floats * done;
-        void* ra[] = {&drawsc, &data_len, &params_len, &params, &xs,  &lf,  &K,
-                      &beta,   &betas,    &n,          &partner, &acc, &out, &sink};
+        void* ra[] = {&drawsc, &data_len, &params_len, &params, &xs,  &lf, &K,
+                      &beta,   &betas,    &n,          &acc,    &out, &sink};
         BH_TRY(ktimed(s, [&] {
             return launch(out ? s->f->resident_out : s->f->resident, 1, nb,
                           (unsigned)resident_lds(s), s->stream, ra);
@@ -1586,10 +1613,8 @@ int bh_stretch_factory_create(bh_ctx* ctx, const char* source, const char* logfn
     BH_TRY(f->mod.fn("bh_logfn", &f->logfn));
     BH_TRY(f->mod.fn("bh_stretch_move_bare", &f->bare));
     BH_TRY(f->mod.fn("bh_stretch_move_accu", &f->accu));
-    BH_TRY(f->mod.fn("bh_stretch_resident", &f->resident));
-    BH_TRY(f->mod.fn("bh_stretch_resident_out", &f->resident_out));
-    BH_TRY(f->mod.fn("bh_stretch_draws", &f->draws));
-    BH_TRY(f->mod.fn("bh_trace_accu", &f->trace_accu));
+    f->source = source;
+    f->logfn_name = logfn_name;
     *out = f.release();
     return BH_OK;
 }
@@ -1784,6 +1809,7 @@ int bh_stretch_create(bh_stretch_factory* f, uint32_t seed, uint32_t walkers,
         BH_HIP(hipMemcpyAsync(s->params.p, params, (size_t)params_count * sizeof(float),
                               hipMemcpyDefault, s->stream));
     BH_TRY(sync(s->stream));
+    if (use_resident(s.get())) BH_TRY(resident_module(f));
     BH_TRY(bh_stretch_init(s.get(), seed));
     *out = s.release();
     return BH_OK;
@@ -1864,6 +1890,7 @@ int bh_stretch_set_exec(bh_stretch* s, int mode) {
         return fail(BH_ERR_RANGE, "ensemble (%u walkers x %u) does not fit in one work-group's LDS",
                     s->W, s->dim);
     s->exec = mode;
+    if (use_resident(s)) BH_TRY(resident_module(s->f));
     return BH_OK;
 }
 

@@ -287,6 +287,9 @@ __device__ __forceinline__ bool bh_stretch_walker(unsigned k, unsigned K, unsign
     return accepted;
 }
 
+// The modules of a model: its per-half-step kernels, and on their own (a user's
+// density is compiled into each kernel) the resident and the batched ones.
+#if !defined(BH_RESIDENT) && !defined(BH_BATCH)
 // logfn kernel (amd-gcn-mcmc-stretch.cl:161-167): res[w] = LOGFN(x + DIM*w).
 extern "C" __global__ void __launch_bounds__(WGS)
 bh_logfn(unsigned data_len, unsigned params_len, const float* __restrict__ params,
@@ -559,6 +562,9 @@ bh_stretch_move_accu(unsigned seed, unsigned odd_or_even, unsigned data_len,
                                                  S, X, logfn_X, a, 1.0f, step, K, accept, means);
 }
 
+#endif  // !BH_RESIDENT && !BH_BATCH
+
+#ifdef BH_RESIDENT
 // Small ensembles: one work-group holds the whole ensemble (positions and
 // log densities) in LDS and runs many full steps without returning to the
 // host, so that no launch sits between half-steps.  What bounds it is then
@@ -601,8 +607,9 @@ bh_stretch_draws(unsigned seed_odd, unsigned seed_even, unsigned c_odd, unsigned
 }
 
 // Floats from one half-ensemble to the next in LDS: the K * DIM coordinates,
-// then the first DIM - 1 of them again, so that a FLAT partner's coordinates
-// are read without wrapping; a multiple of 4, so that records stay aligned.
+// then the first DIM - 1 of them again, so that every partner's coordinates
+// are read in a row from its offset, without wrapping and whatever the
+// partner mode; a multiple of 4, so that records stay aligned.
 __device__ __forceinline__ unsigned bh_resident_half(unsigned K) {
     return (K * DIM + DIM - 1 + 3) / 4 * 4;
 }
@@ -619,22 +626,10 @@ __device__ __forceinline__ void bh_resident_load(float* sx, unsigned H, unsigned
     }
 }
 
-template <int PARTNER>
-__device__ __forceinline__ void bh_resident_partner(const float* S, unsigned e,
-                                                    float (&sj)[DIM]) {
-    if constexpr (PARTNER == BH_PARTNER_FLAT) {
-#pragma unroll
-        for (int i = 0; i < DIM; ++i) sj[i] = S[e + i];
-    } else {
-        bh_load_walker(S + e, sj);
-    }
-}
-
-template <int PARTNER>
 __device__ __forceinline__ void bh_resident_accept(float* X, unsigned K, unsigned k,
                                                    const float (&y)[DIM]) {
     bh_store_walker(X + k * DIM, y);
-    if (PARTNER == BH_PARTNER_FLAT && DIM > 1 && k == 0) {
+    if (DIM > 1 && k == 0) {
 #pragma unroll
         for (int i = 0; i < DIM - 1; ++i) X[K * DIM + i] = y[i];
     }
@@ -656,13 +651,13 @@ __device__ __forceinline__ void bh_resident_accept(float* X, unsigned K, unsigne
 // the other half reads.  Eight waves share four SIMDs, so at 1024 walkers the
 // half-step takes the instructions it issues, ~65 VALU at dim 4 (500 of its
 // 830 cycles, the rest LDS and barrier latency); the general form below reads
-// and addresses everything anew: 1.1 us per step where this takes 0.73.
+// and addresses everything anew: 0.45 us per half-step where this takes 0.35.
 //   draws: K per half-step, and 2 * BH_RESIDENT_AHEAD * K more that are read
 //        but not used
 //   betas: one inverse temperature per step, or null (beta for all)
 //   out (OUT): the positions after each half-step, half after half
 //   accept: null, or the accept counts per group of WGS walkers, added to
-template <int PARTNER, bool OUT>
+template <bool OUT>
 __device__ __forceinline__ void bh_resident_one(
     const float4* __restrict__ draws, unsigned data_len, unsigned params_len,
     const float* __restrict__ params, float* __restrict__ xs, float* __restrict__ logfn,
@@ -706,7 +701,9 @@ __device__ __forceinline__ void bh_resident_one(
             asm volatile("" : "+v"(d[r]));
             float* X = sx + (h ? H : 0u);
             float sj[DIM], y[DIM];
-            bh_resident_partner<PARTNER>(sx + (h ? 0u : H), live ? __float_as_uint(d[r].y) : 0u, sj);
+            const float* S = sx + (h ? 0u : H) + (live ? __float_as_uint(d[r].y) : 0u);
+#pragma unroll
+            for (int i = 0; i < DIM; ++i) sj[i] = S[i];
 #pragma unroll
             for (int i = 0; i < DIM; ++i) y[i] = __builtin_fmaf(d[r].x, x[h][i] - sj[i], sj[i]);
             const float ly = LOGFN(data_len, params_len, params, DIM, y);
@@ -716,7 +713,7 @@ __device__ __forceinline__ void bh_resident_one(
 #pragma unroll
             for (int i = 0; i < DIM; ++i) x[h][i] = acc ? y[i] : x[h][i];
             lx[h] = acc ? ly : lx[h];
-            if (acc) bh_resident_accept<PARTNER>(X, K, k, x[h]);
+            if (acc) bh_resident_accept(X, K, k, x[h]);
             count += (unsigned)__popcll(__ballot(acc));
             if constexpr (OUT) {
                 float* dst = live ? out : sink;
@@ -741,13 +738,14 @@ __device__ __forceinline__ void bh_resident_one(
 // and half (draws: slots * blockDim.x per half-step, and 2 *
 // BH_RESIDENT_AHEAD * blockDim.x more); threads past K take walker K - 1,
 // decide nothing and write to the sink.
-template <int PARTNER, bool OUT>
+template <bool OUT>
 __device__ __forceinline__ void bh_resident_slots(
     const float4* __restrict__ draws, unsigned data_len, unsigned params_len,
     const float* __restrict__ params, float* __restrict__ xs, float* __restrict__ logfn,
     unsigned K, float beta, const float* __restrict__ betas, unsigned nsteps,
     unsigned* __restrict__ accept, float* __restrict__ out, float* __restrict__ sink) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
+    constexpr int AHEAD = 2;
     typedef float bh_f4 __attribute__((ext_vector_type(4)));
     const unsigned nb = blockDim.x, t = threadIdx.x;
     const unsigned H = bh_resident_half(K), W = 2 * K, groups = K / WGS;
@@ -759,9 +757,9 @@ __device__ __forceinline__ void bh_resident_slots(
     for (unsigned i = t; i < groups; i += nb) acc_lds[i] = 0u;
     const unsigned total = 2 * nsteps * ((K + nb - 1) / nb);
     const bh_f4* dp = reinterpret_cast<const bh_f4*>(draws) + t;
-    bh_f4 d[BH_RESIDENT_AHEAD];
+    bh_f4 d[AHEAD];
 #pragma unroll
-    for (int r = 0; r < BH_RESIDENT_AHEAD; ++r) {
+    for (int r = 0; r < AHEAD; ++r) {
         d[r] = *dp;
         dp += nb;
         __builtin_amdgcn_sched_barrier(0);
@@ -770,16 +768,18 @@ __device__ __forceinline__ void bh_resident_slots(
     float b_next = betas && nsteps > 1 ? betas[1] : beta;
     unsigned h = 0, k0 = 0, s = 0;
     __syncthreads();
-    for (unsigned i0 = 0; i0 < total; i0 += BH_RESIDENT_AHEAD) {
+    for (unsigned i0 = 0; i0 < total; i0 += AHEAD) {
 #pragma unroll
-        for (int r = 0; r < BH_RESIDENT_AHEAD; ++r) {
+        for (int r = 0; r < AHEAD; ++r) {
             const unsigned kt = k0 + t;
             const bool live = kt < K && i0 + r < total;
             const unsigned k = kt < K ? kt : K - 1;
             asm volatile("" : "+v"(d[r]));
             float* X = sx + h * H;
             float xk[DIM], sj[DIM], y[DIM];
-            bh_resident_partner<PARTNER>(sx + (h ^ 1u) * H, live ? __float_as_uint(d[r].y) : 0u, sj);
+            const float* S = sx + (h ^ 1u) * H + (live ? __float_as_uint(d[r].y) : 0u);
+#pragma unroll
+            for (int i = 0; i < DIM; ++i) sj[i] = S[i];
             bh_load_walker(X + k * DIM, xk);
             const float lx = sl[h * K + k];
 #pragma unroll
@@ -790,7 +790,7 @@ __device__ __forceinline__ void bh_resident_slots(
 #pragma unroll
             for (int i = 0; i < DIM; ++i) xk[i] = acc ? y[i] : xk[i];
             if (acc) {
-                bh_resident_accept<PARTNER>(X, K, k, xk);
+                bh_resident_accept(X, K, k, xk);
                 sl[h * K + k] = ly;
             }
             if constexpr (OUT) {
@@ -831,26 +831,14 @@ __device__ __forceinline__ void bh_resident_slots(
     extern "C" __global__ void __launch_bounds__(1024) NAME(                                      \
         const float4* __restrict__ draws, unsigned data_len, unsigned params_len,                 \
         const float* __restrict__ params, float* __restrict__ xs, float* __restrict__ logfn,      \
-        unsigned K, float beta, const float* __restrict__ betas, unsigned nsteps, int partner,    \
+        unsigned K, float beta, const float* __restrict__ betas, unsigned nsteps,                 \
         unsigned* __restrict__ accept, float* __restrict__ out, float* __restrict__ sink) {       \
-        if (blockDim.x == K) {                                                                    \
-            if (partner == BH_PARTNER_FLAT)                                                       \
-                bh_resident_one<BH_PARTNER_FLAT, OUT>(draws, data_len, params_len, params, xs,    \
-                                                      logfn, K, beta, betas, nsteps, accept, out, \
-                                                      sink);                                      \
-            else                                                                                  \
-                bh_resident_one<BH_PARTNER_WALKER, OUT>(draws, data_len, params_len, params, xs,  \
-                                                        logfn, K, beta, betas, nsteps, accept,    \
-                                                        out, sink);                               \
-        } else if (partner == BH_PARTNER_FLAT) {                                                  \
-            bh_resident_slots<BH_PARTNER_FLAT, OUT>(draws, data_len, params_len, params, xs,      \
-                                                    logfn, K, beta, betas, nsteps, accept, out,   \
-                                                    sink);                                        \
-        } else {                                                                                  \
-            bh_resident_slots<BH_PARTNER_WALKER, OUT>(draws, data_len, params_len, params, xs,    \
-                                                      logfn, K, beta, betas, nsteps, accept, out, \
-                                                      sink);                                      \
-        }                                                                                         \
+        if (blockDim.x == K)                                                                      \
+            bh_resident_one<OUT>(draws, data_len, params_len, params, xs, logfn, K, beta, betas,  \
+                                 nsteps, accept, out, sink);                                      \
+        else                                                                                      \
+            bh_resident_slots<OUT>(draws, data_len, params_len, params, xs, logfn, K, beta,       \
+                                   betas, nsteps, accept, out, sink);                             \
     }
 BH_RESIDENT_KERNEL(bh_stretch_resident, false)
 BH_RESIDENT_KERNEL(bh_stretch_resident_out, true)
@@ -888,6 +876,7 @@ bh_trace_accu(const float* __restrict__ trace, unsigned K, unsigned step0,
     }
 }
 
+#endif  // BH_RESIDENT
 #endif  // LOGFN
 
 #ifdef BH_BATCH

@@ -42,7 +42,7 @@ def _same_state(a, b):
 # do not fill the kernel's rounds of four
 @pytest.mark.parametrize("dim,walkers", [(1, 512), (3, 512), (4, 1024), (7, 1536), (9, 1024),
                                          (2, 2560), (3, 3072), (1, 5120), (2, 4608),
-                                         (1, 8192), (4, 7168)])
+                                         (1, 12288), (4, 7168)])
 @pytest.mark.parametrize("partner", [FLAT, WALKER])
 def test_resident_equals_stepwise(fac, dim, walkers, partner):
     sf, (a, b) = _pair(fac, dim, walkers, partner)
