@@ -36,74 +36,6 @@ __device__ __forceinline__ float bh_wave_tree_sum(float x) {
     return x;
 }
 
-// Sum v over each aligned slice of WGS threads with the reference's
-// work-group tree (amd-gcn-mcmc-stretch.cl:5-29 for power-of-two WGS: level
-// i adds item l+i into item l, i = WGS/2 ... 1).  Float addition is not
-// associative, so the tree shape is kept exactly: the result is
-// bit-identical to the reference's.  Values are staged in
-// buf[d*blockDim + t]; after one barrier lane l < 64 of the slice reads
-// items l + 64j (j < WGS/64) and applies the levels i >= 64 to them in the
-// tree's pairing (item l + 64j gets item l + 64(j + i/64)), then the slice's
-// first wave applies levels 32 ... 1 with cross-lane moves.  The total of
-// dim d is returned in out[d] by the slice's lane 0.  With count non-null
-// the slice's set flags are counted too (ballot counts staged with the
-// values; order-independent integers), returned in *count by lane 0.
-// tail_sync: a barrier at the end, before the caller writes buf or
-// wave_counts again (not needed when a barrier or the kernel's end comes
-// first).
-template <int ND>
-__device__ __forceinline__ void bh_slice_tree(const float (&v)[ND], float* buf, float (&out)[ND],
-                                              bool flag, unsigned* wave_counts,
-                                              unsigned* count, bool tail_sync) {
-    static_assert(WGS >= 64 && (WGS & (WGS - 1)) == 0, "WGS: a power of two >= 64");
-    constexpr unsigned R = WGS / 64;
-    const unsigned t = threadIdx.x;
-    const unsigned nb = blockDim.x;
-    const unsigned l = t & (WGS - 1);
-    if (count) {
-        const unsigned long long m = __ballot(flag);
-        if ((t & 63u) == 0) wave_counts[t >> 6] = (unsigned)__popcll(m);
-    }
-#pragma unroll
-    for (int d = 0; d < ND; ++d) buf[d * nb + t] = v[d];
-    __syncthreads();
-    if (l < 64) {
-#pragma unroll
-        for (int d = 0; d < ND; ++d) {
-            float x[R];
-#pragma unroll
-            for (unsigned j = 0; j < R; ++j) x[j] = buf[d * nb + t + 64 * j];
-#pragma unroll
-            for (unsigned h = R / 2; h >= 1; h >>= 1)
-#pragma unroll
-                for (unsigned j = 0; j < h; ++j) x[j] = x[j] + x[j + h];
-            out[d] = bh_wave_tree_sum(x[0]);
-        }
-        if (count && l == 0) {
-            unsigned total = 0;
-            const unsigned w0 = t >> 6;
-            for (unsigned w = 0; w < R; ++w) total += wave_counts[w0 + w];
-            *count = total;
-        }
-    }
-    if (tail_sync) __syncthreads();
-}
-
-template <int ND>
-__device__ __forceinline__ void bh_slice_tree_sums(const float (&v)[ND], float* buf,
-                                                   float (&out)[ND], bool tail_sync = true) {
-    bh_slice_tree<ND>(v, buf, out, false, nullptr, nullptr, tail_sync);
-}
-
-template <int ND>
-__device__ __forceinline__ void bh_slice_count_tree_sums(bool flag, const float (&v)[ND],
-                                                         float* buf, unsigned* wave_counts,
-                                                         float (&out)[ND], unsigned& count,
-                                                         bool tail_sync = true) {
-    count = 0;
-    bh_slice_tree<ND>(v, buf, out, flag, wave_counts, &count, tail_sync);
-}
-
 #if defined(LOGFN) || defined(BH_GLM)
 
 // A walker's DIM coordinates.  Walkers start at multiples of DIM floats from
@@ -207,39 +139,23 @@ __device__ __forceinline__ float bh_zpow(float z) {
 }
 
 // Accounting of stretch_move_accu (amd-gcn-mcmc-stretch.cl:98-114) for the
-// slice of WGS threads holding group g: accept[g] += accepted count;
+// work-group of WGS threads holding group g: accept[g] += accepted count;
 // means[groups*DIM*step + i*groups + g] += tree sum of coordinate i.
-// Dimensions are reduced BH_ACCU_CHUNK at a time so the LDS staging area
-// stays at BH_ACCU_CHUNK floats per thread whatever DIM is.
+// Coordinates are staged BH_ACCU_CHUNK at a time, so that the staging area
+// stays at BH_ACCU_CHUNK floats per thread whatever DIM is, and the
+// work-group's waves take the trees of a chunk between them (wave w the
+// coordinates w, w + WGS/64, ...).  What the sums are added to is read before
+// the move (BhAccuOld): lane i of a wave holds the old value, later the new
+// one, of the wave's i-th coordinate.  The kernel's end is then a staging, a
+// barrier, two trees and a store; with one wave taking every tree and its
+// first lane reading, adding and writing the sums one after the other, a
+// half-step of 32,768 walkers x 7 took 6.96 us, now 4.54 (bound by the latency
+// of the walker's and then the partner's loads).
 #define BH_ACCU_CHUNK (DIM < 8 ? DIM : 8)
-
-__device__ __forceinline__ void bh_accu(const float (&xk)[DIM], bool accepted, unsigned g,
-                                        unsigned groups, unsigned mstep, unsigned* accept,
-                                        float* means, float* red, unsigned* wave_counts) {
-    const bool leader = (threadIdx.x & (WGS - 1)) == 0;
-    float* m = means + (size_t)groups * DIM * mstep + g;
-#pragma unroll
-    for (int d0 = 0; d0 < DIM; d0 += BH_ACCU_CHUNK) {
-        float v[BH_ACCU_CHUNK], sums[BH_ACCU_CHUNK];
-#pragma unroll
-        for (int c = 0; c < BH_ACCU_CHUNK; ++c) v[c] = (d0 + c < DIM) ? xk[d0 + c] : 0.0f;
-        // every caller ends its kernel here: no barrier after the last chunk
-        const bool more = d0 + BH_ACCU_CHUNK < DIM;
-        if (d0 == 0) {
-            unsigned cnt;
-            bh_slice_count_tree_sums<BH_ACCU_CHUNK>(accepted, v, red, wave_counts, sums, cnt,
-                                                    more);
-            if (leader) accept[g] += cnt;
-        } else {
-            bh_slice_tree_sums<BH_ACCU_CHUNK>(v, red, sums, more);
-        }
-        if (leader) {
-#pragma unroll
-            for (int c = 0; c < BH_ACCU_CHUNK; ++c)
-                if (d0 + c < DIM) m[(size_t)(d0 + c) * groups] += sums[c];
-        }
-    }
-}
+constexpr unsigned kBhWaves = WGS / 64;
+constexpr unsigned kBhAccuChunks = (DIM + BH_ACCU_CHUNK - 1) / BH_ACCU_CHUNK;
+constexpr unsigned kBhAccuPer = (BH_ACCU_CHUNK + kBhWaves - 1) / kBhWaves;  // of a chunk, per wave
+constexpr unsigned kBhAccuRegs = (kBhAccuChunks * kBhAccuPer + 63) / 64;
 
 // The accounting's LDS staging, one area for every instantiation of a
 // half-step in a kernel.
@@ -251,6 +167,85 @@ struct BhAccuLds {
 __device__ __forceinline__ BhAccuLds& bh_accu_lds() {
     __shared__ BhAccuLds st;
     return st;
+}
+
+// Sum of row c of the staged values (WGS of them) with the reference's
+// work-group tree (amd-gcn-mcmc-stretch.cl:5-29 for power-of-two WGS: level i
+// adds item l+i into item l, i = WGS/2 ... 1), by one wave: lane l takes the
+// items l + 64j and their levels i >= 64 in the tree's pairing, then the
+// levels 32 ... 1 with cross-lane moves.  Float addition is not associative,
+// so the tree's shape is kept exactly.
+__device__ __forceinline__ float bh_row_tree_sum(const float* red, unsigned c) {
+    const float* p = red + c * WGS + (threadIdx.x & 63u);
+    float x[kBhWaves];
+#pragma unroll
+    for (unsigned j = 0; j < kBhWaves; ++j) x[j] = p[64 * j];
+#pragma unroll
+    for (unsigned h = kBhWaves / 2; h >= 1; h >>= 1)
+#pragma unroll
+        for (unsigned j = 0; j < h; ++j) x[j] = x[j] + x[j + h];
+    return __uint_as_float(
+        __builtin_amdgcn_readfirstlane(__float_as_uint(bh_wave_tree_sum(x[0]))));
+}
+
+struct BhAccuOld {
+    float m[kBhAccuRegs];
+    unsigned accept;
+
+    // the coordinate of this lane's item in register r, or DIM
+    __device__ __forceinline__ static unsigned dim_of(unsigned r) {
+        const unsigned it = r * 64 + (threadIdx.x & 63u);
+        const unsigned c = (threadIdx.x >> 6) + it % kBhAccuPer * kBhWaves;
+        const unsigned d = it / kBhAccuPer * BH_ACCU_CHUNK + c;
+        return it < kBhAccuChunks * kBhAccuPer && c < BH_ACCU_CHUNK && d < DIM ? d : DIM;
+    }
+    __device__ __forceinline__ void load(unsigned g, unsigned groups, unsigned mstep,
+                                         const unsigned* acc, const float* means) {
+        accept = acc[g];
+        const float* p = means + (size_t)groups * DIM * mstep + g;
+#pragma unroll
+        for (unsigned r = 0; r < kBhAccuRegs; ++r) {
+            const unsigned d = dim_of(r);
+            m[r] = d < DIM ? p[(size_t)d * groups] : 0.0f;
+        }
+    }
+};
+
+__device__ __forceinline__ void bh_accu(const float (&xk)[DIM], bool accepted, unsigned g,
+                                        unsigned groups, unsigned mstep, unsigned* accept,
+                                        float* means, BhAccuOld& old, BhAccuLds& lds) {
+    const unsigned t = threadIdx.x, lane = t & 63u, wave = t >> 6;
+    const unsigned long long b = __ballot(accepted);
+    if (lane == 0) lds.wave_counts[wave] = (unsigned)__popcll(b);
+#pragma unroll
+    for (unsigned n = 0; n < kBhAccuChunks; ++n) {
+        const unsigned d0 = n * BH_ACCU_CHUNK;
+        if (n > 0) __syncthreads();  // the previous chunk's trees have read it
+#pragma unroll
+        for (unsigned c = 0; c < BH_ACCU_CHUNK; ++c)
+            if (d0 + c < DIM) lds.red[c * WGS + t] = xk[d0 + c];
+        __syncthreads();
+#pragma unroll
+        for (unsigned q = 0; q < kBhAccuPer; ++q) {
+            const unsigned c = wave + q * kBhWaves;
+            if (c < BH_ACCU_CHUNK && d0 + c < DIM) {
+                const float sum = bh_row_tree_sum(lds.red, c);
+                const unsigned it = n * kBhAccuPer + q;
+                if (lane == it % 64) old.m[it / 64] += sum;
+            }
+        }
+    }
+    float* p = means + (size_t)groups * DIM * mstep + g;
+#pragma unroll
+    for (unsigned r = 0; r < kBhAccuRegs; ++r) {
+        const unsigned d = BhAccuOld::dim_of(r);
+        if (d < DIM) p[(size_t)d * groups] = old.m[r];
+    }
+    if (t == 0) {
+        unsigned cnt = 0;
+        for (unsigned w = 0; w < kBhWaves; ++w) cnt += lds.wave_counts[w];
+        accept[g] = old.accept + cnt;
+    }
 }
 
 #endif  // LOGFN || BH_GLM
@@ -388,6 +383,8 @@ __device__ __forceinline__ void bh_stretch_half_staged(unsigned seed, unsigned o
     const unsigned t = threadIdx.x;
     const unsigned k = blockIdx.x * WGS + t;
     float* xb = X + (size_t)blockIdx.x * WGS * DIM;
+    BhAccuOld old;
+    if (ACCU) old.load(blockIdx.x, gridDim.x, step, accept, means);
     // own records: piece g = i*WGS + t is piece g % NP of record g / NP
     float xs[NP * (V4 ? 4 : 1)];
     if constexpr (V4) {
@@ -493,11 +490,8 @@ __device__ __forceinline__ void bh_stretch_half_staged(unsigned seed, unsigned o
             }
         }
     }
-    if (ACCU) {
-        BhAccuLds& al = bh_accu_lds();
-        bh_accu(xk, accepted, blockIdx.x, gridDim.x, step, accept, means, al.red,
-                al.wave_counts);
-    }
+    if (ACCU)
+        bh_accu(xk, accepted, blockIdx.x, gridDim.x, step, accept, means, old, bh_accu_lds());
 }
 
 template <bool ACCU, int PARTNER>
@@ -519,17 +513,16 @@ __device__ __forceinline__ void bh_stretch_half(unsigned seed, unsigned odd_or_e
         float* xp = X + (size_t)k * DIM;
         bh_load_walker_nt(xp, xk);
         float lx = __builtin_nontemporal_load(logfn_X + k);
+        BhAccuOld old;
+        if (ACCU) old.load(blockIdx.x, gridDim.x, step, accept, means);
         const bool accepted = bh_stretch_walker<PARTNER>(k, K, seed, odd_or_even, step, a, beta, S,
                                                          xk, lx, data_len, params_len, params);
         if (accepted) {
             bh_store_walker_nt(xp, xk);
             __builtin_nontemporal_store(lx, logfn_X + k);
         }
-        if (ACCU) {
-            BhAccuLds& al = bh_accu_lds();
-            bh_accu(xk, accepted, blockIdx.x, gridDim.x, step, accept, means, al.red,
-                    al.wave_counts);
-        }
+        if (ACCU)
+            bh_accu(xk, accepted, blockIdx.x, gridDim.x, step, accept, means, old, bh_accu_lds());
     }
 }
 
@@ -852,26 +845,32 @@ BH_RESIDENT_KERNEL(bh_stretch_resident_out, true)
 extern "C" __global__ void __launch_bounds__(WGS)
 bh_trace_accu(const float* __restrict__ trace, unsigned K, unsigned step0,
               float* __restrict__ means) {
-    __shared__ float red[BH_ACCU_CHUNK * WGS];
+    __shared__ float red[2][BH_ACCU_CHUNK * WGS];
     const unsigned g = blockIdx.x, groups = gridDim.x, t = threadIdx.x;
+    const unsigned lane = t & 63u, wave = t >> 6;
     const float* rec = trace + ((size_t)blockIdx.y * 2 * K + g * WGS + t) * DIM;
     float xo[DIM], xe[DIM];
     bh_load_walker(rec, xo);
     bh_load_walker(rec + (size_t)K * DIM, xe);
     float* m = means + (size_t)groups * DIM * (step0 + blockIdx.y) + g;
 #pragma unroll
-    for (int d0 = 0; d0 < DIM; d0 += BH_ACCU_CHUNK) {
-        float v[BH_ACCU_CHUNK], odd[BH_ACCU_CHUNK], even[BH_ACCU_CHUNK];
+    for (unsigned n = 0; n < kBhAccuChunks; ++n) {
+        const unsigned d0 = n * BH_ACCU_CHUNK;
+        if (n > 0) __syncthreads();
 #pragma unroll
-        for (int c = 0; c < BH_ACCU_CHUNK; ++c) v[c] = d0 + c < DIM ? xo[d0 + c] : 0.0f;
-        bh_slice_tree_sums<BH_ACCU_CHUNK>(v, red, odd);
+        for (unsigned c = 0; c < BH_ACCU_CHUNK; ++c)
+            if (d0 + c < DIM) {
+                red[0][c * WGS + t] = xo[d0 + c];
+                red[1][c * WGS + t] = xe[d0 + c];
+            }
+        __syncthreads();
 #pragma unroll
-        for (int c = 0; c < BH_ACCU_CHUNK; ++c) v[c] = d0 + c < DIM ? xe[d0 + c] : 0.0f;
-        bh_slice_tree_sums<BH_ACCU_CHUNK>(v, red, even, d0 + BH_ACCU_CHUNK < DIM);
-        if (t == 0) {
-#pragma unroll
-            for (int c = 0; c < BH_ACCU_CHUNK; ++c)
-                if (d0 + c < DIM) m[(size_t)(d0 + c) * groups] = (0.0f + odd[c]) + even[c];
+        for (unsigned q = 0; q < kBhAccuPer; ++q) {
+            const unsigned c = wave + q * kBhWaves;
+            if (c < BH_ACCU_CHUNK && d0 + c < DIM) {
+                const float odd = bh_row_tree_sum(red[0], c), even = bh_row_tree_sum(red[1], c);
+                if (lane == 0) m[(size_t)(d0 + c) * groups] = (0.0f + odd) + even;
+            }
         }
     }
 }
@@ -1705,6 +1704,8 @@ bh_glm_accept(const float* __restrict__ Y, const float* __restrict__ zbuf,
               unsigned* __restrict__ accept, float* __restrict__ means, unsigned mstep,
               const unsigned* __restrict__ flag, const double* __restrict__ corr) {
     const unsigned k = blockIdx.x * WGS + threadIdx.x;
+    BhAccuOld old;
+    if (accu) old.load(blockIdx.x, gridDim.x, mstep, accept, means);
     float y[DIM], xk[DIM];
 #pragma unroll
     for (int i = 0; i < DIM; ++i) y[i] = Y[(size_t)k * DIM + i];
@@ -1726,11 +1727,8 @@ bh_glm_accept(const float* __restrict__ Y, const float* __restrict__ zbuf,
 #pragma unroll
         for (int i = 0; i < DIM; ++i) xk[i] = X[(size_t)k * DIM + i];
     }
-    if (accu) {
-        __shared__ float red[BH_ACCU_CHUNK * WGS];
-        __shared__ unsigned wave_counts[WGS / 64];
-        bh_accu(xk, accepted, blockIdx.x, gridDim.x, mstep, accept, means, red, wave_counts);
-    }
+    if (accu)
+        bh_accu(xk, accepted, blockIdx.x, gridDim.x, mstep, accept, means, old, bh_accu_lds());
 }
 // The guarded path's accept step, with every decision already in flag (1
 // reject, 2 accept) and the proposals' log posteriors in lpy: work-group
@@ -1748,6 +1746,13 @@ bh_glm_accept_split(const float* __restrict__ Y, const double* __restrict__ lpy,
     const unsigned k = g * WGS + threadIdx.x;
     const bool accepted = flag[k] == 2u;
     const unsigned d0 = c * BH_ACCU_CHUNK;
+    // lane q of a wave: the wave's q-th coordinate of the chunk (bh_accu)
+    const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const unsigned cm = wave + lane * kBhWaves;
+    const bool mine = accu && lane < kBhAccuPer && cm < BH_ACCU_CHUNK && d0 + cm < DIM;
+    float* m = means + (size_t)gridDim.x * DIM * mstep + (size_t)(d0 + cm) * gridDim.x + g;
+    float old = mine ? *m : 0.0f;
+    const unsigned old_acc = accu && c == 0 ? accept[g] : 0u;
     float v[BH_ACCU_CHUNK];
 #pragma unroll
     for (int i = 0; i < BH_ACCU_CHUNK; ++i) {
@@ -1764,19 +1769,25 @@ bh_glm_accept_split(const float* __restrict__ Y, const double* __restrict__ lpy,
     }
     if (c == 0 && accepted) lp[k] = lpy[k];
     if (accu) {
-        __shared__ float red[BH_ACCU_CHUNK * WGS];
-        __shared__ unsigned wave_counts[WGS / 64];
-        const unsigned groups = gridDim.x;
-        const bool leader = threadIdx.x == 0;
-        float sums[BH_ACCU_CHUNK];
-        unsigned cnt;
-        bh_slice_count_tree_sums<BH_ACCU_CHUNK>(accepted, v, red, wave_counts, sums, cnt, false);
-        if (c == 0 && leader) accept[g] += cnt;
-        if (leader) {
-            float* m = means + (size_t)groups * DIM * mstep + g;
+        BhAccuLds& lds = bh_accu_lds();
+        const unsigned long long b = __ballot(accepted);
+        if (lane == 0) lds.wave_counts[wave] = (unsigned)__popcll(b);
 #pragma unroll
-            for (int i = 0; i < BH_ACCU_CHUNK; ++i)
-                if (d0 + i < DIM) m[(size_t)(d0 + i) * groups] += sums[i];
+        for (int i = 0; i < BH_ACCU_CHUNK; ++i) lds.red[i * WGS + threadIdx.x] = v[i];
+        __syncthreads();
+#pragma unroll
+        for (unsigned q = 0; q < kBhAccuPer; ++q) {
+            const unsigned i = wave + q * kBhWaves;
+            if (i < BH_ACCU_CHUNK && d0 + i < DIM) {
+                const float sum = bh_row_tree_sum(lds.red, i);
+                if (lane == q) old += sum;
+            }
+        }
+        if (mine) *m = old;
+        if (c == 0 && threadIdx.x == 0) {
+            unsigned cnt = 0;
+            for (unsigned w = 0; w < kBhWaves; ++w) cnt += lds.wave_counts[w];
+            accept[g] = old_acc + cnt;
         }
     }
 }
