@@ -269,7 +269,7 @@ struct GlmData {
     int kind = 0;
     unsigned long long N = 0;
     uint32_t d = 0;
-    uint32_t D = 0;           // linear regression: padded column count of Xf
+    uint32_t D = 0;           // linear regression: padded column count
     double prior_prec = 1.0;  // logistic: 1 / prior_sd^2
     DevBuf X;                 // logistic: bf16, N x d row-major
     DevBuf lin;               // logistic: double[d]: X'y; linear regression: the
@@ -278,7 +278,7 @@ struct GlmData {
     DevBuf half_colsum;       // logistic: double[d]: (1/2) X'1
     DevBuf X16;               // logistic: fp16 copy of X in fragment order, made on first fp16 use
     mutable unsigned bpc[BH_GLM_FP16 + 1] = {};  // resident work-groups per CU, by precision
-    DevBuf Xf, y;             // linear regression: fp32 N x D and N
+    DevBuf Xf, y;             // linear regression: fp32 X and y as the kernels read them
 };
 
 // The linear coefficients of a precision's log-likelihood: the logistic
@@ -408,6 +408,8 @@ constexpr uint64_t kResidentParams = 1000000;
 
 // rounds of work-groups per logistic likelihood launch
 constexpr unsigned kGlmRounds = 4;
+// and per linear-regression launch
+constexpr unsigned kGaussRounds = 1;
 
 // Guarded accept test: the list holds every walker of a half (K), so no
 // walker inside the guard is ever decided on reduced-precision values; the
@@ -671,16 +673,12 @@ int glm_prepare(bh_stretch_factory* f, int prec) {
 // last round leaves compute units idle; a few rounds of smaller ranges even
 // out the ranges' finishing times.
 unsigned glm_ranges(const bh_ctx* c, const GlmData& g, int prec, unsigned n) {
-    unsigned groups = std::max(n / bh::glm_point_quantum(prec), 1u);
-    // the linear-regression kernel's work-groups can take twice 256 points:
-    // twice the ranges keep the work-group count
-    if (g.kind == BH_GLM_GAUSSIAN)
-        groups = std::max(groups / bh::glm_gauss_points_per_thread(prec, g.D, n), 1u);
-    unsigned blocks = 4u * (unsigned)c->cu;
-    if (g.kind == BH_GLM_LOGISTIC) {
-        if (!g.bpc[prec]) g.bpc[prec] = bh::glm_blocks_per_cu(prec, g.d);
-        blocks = kGlmRounds * g.bpc[prec] * (unsigned)c->cu;
-    }
+    const unsigned groups = std::max(n / bh::glm_point_quantum(prec), 1u);
+    if (!g.bpc[prec])
+        g.bpc[prec] = g.kind == BH_GLM_GAUSSIAN ? bh::glm_gauss_blocks_per_cu(prec, g.D)
+                                                : bh::glm_blocks_per_cu(prec, g.d);
+    const unsigned rounds = g.kind == BH_GLM_GAUSSIAN ? kGaussRounds : kGlmRounds;
+    const unsigned blocks = rounds * g.bpc[prec] * (unsigned)c->cu;
     unsigned r = (blocks + groups - 1) / groups;
     r = (r + 7) / 8 * 8;
     const unsigned long long max_r = std::max(8ull, (g.N / 64 + 7) / 8 * 8);
@@ -1718,20 +1716,14 @@ int bh_glm_gaussian_factory_create(bh_ctx* ctx, const float* X, const float* y, 
     g->N = N;
     g->d = d;
     g->D = d <= 16 ? 16 : (d <= 32 ? 32 : 64);
-    std::vector<float> xp((size_t)N * g->D, 0.0f);
-    const float* xh = X;
-    std::vector<float> xcopy;
-    if (is_device_ptr(X)) {
-        xcopy.resize((size_t)N * d);
-        BH_HIP(hipMemcpy(xcopy.data(), X, xcopy.size() * 4, hipMemcpyDeviceToHost));
-        xh = xcopy.data();
-    }
-    for (uint64_t i = 0; i < N; ++i)
-        std::memcpy(&xp[(size_t)i * g->D], xh + (size_t)i * d, (size_t)d * 4);
-    BH_TRY(g->Xf.alloc(xp.size() * 4));
-    BH_HIP(hipMemcpy(g->Xf.p, xp.data(), xp.size() * 4, hipMemcpyHostToDevice));
-    BH_TRY(g->y.alloc((size_t)N * 4));
-    BH_HIP(hipMemcpy(g->y.p, y, (size_t)N * 4, hipMemcpyDefault));
+    DevIn dx, dy;
+    BH_TRY(dx.init(X, (size_t)N * d * 4, ctx->stream));
+    BH_TRY(dy.init(y, (size_t)N * 4, ctx->stream));
+    BH_TRY(g->Xf.alloc(bh::glm_gauss_x_floats(N, g->D) * 4));
+    BH_TRY(g->y.alloc(bh::glm_gauss_y_floats(N) * 4));
+    BH_HIP(bh::launch_glm_gauss_pack(ctx->stream, dx.as<float>(), dy.as<float>(), N, d, g->D,
+                                     g->Xf.as<float>(), g->y.as<float>()));
+    BH_TRY(sync(ctx->stream));
     const double c[4] = {(double)N, 0.5 * (double)N * std::log(2.0 * M_PI),
                          1.0 / ((double)beta_sd * beta_sd),
                          1.0 / ((double)log_sigma_sd * log_sigma_sd)};

@@ -266,86 +266,119 @@ glm_logistic_fp64_kernel(const __bf16* __restrict__ X, unsigned long long N,
 // range r and point k (coefficients b_k = the first d of its DIM = d + 1
 // coordinates, row stride pstride),
 //   partial[r][k] = sum_{i in r} (y_i - x_i . b_k)^2,
-// X fp32 N x D (columns past d zero), y fp32.  The plain fp32 kernel: PPT
-// points per thread (their coefficients in registers), tiles of 32 rows of
-// X and y in LDS read as broadcasts, each read feeding every point's fma;
-// fp32 residuals, squares summed four rows at a time into a double.
-template <int D, int PPT>
+// X fp32 with D = 16, 32 or 64 columns (zero past d), y fp32.
+//
+// X is kept in the order the fp32 matrix cores read it (v_mfma_f32_16x16x4:
+// lane l holds row l % 16, feature l / 16 of four): for each 16-row block and
+// 16-feature chunk, lane l's features l / 16, l / 16 + 4, + 8, + 12 one after
+// the other, so that a chunk is one 16-byte load per lane and 1 KB of
+// consecutive bytes per wave.  Rows past N are zero, and so is y.
+__device__ __forceinline__ size_t gauss_frag_at(unsigned long long row, unsigned j, unsigned D) {
+    return (((row / 16) * (D / 16) + j / 16) * 64 + (j % 4) * 16 + row % 16) * 4 + j % 16 / 4;
+}
+
 __global__ void __launch_bounds__(256)
-glm_gauss_fp32_kernel(const float* __restrict__ X, const float* __restrict__ yv,
-                      unsigned long long N, const float* __restrict__ P, unsigned pstride,
-                      unsigned d, unsigned n, unsigned groups, unsigned nranges,
-                      unsigned long long rows_per_range, double* __restrict__ partial) {
-    constexpr int TR = 32;
-    __shared__ float4 xs[TR * D / 4];
-    __shared__ float ys[TR];
+glm_gauss_pack_kernel(const float* __restrict__ X, const float* __restrict__ y,
+                      unsigned long long N, unsigned d, unsigned D, float* __restrict__ Xf,
+                      float* __restrict__ yf) {
+    const unsigned long long rows = ((N + 15) / 16 + 1) * 16;
+    const unsigned long long i = (unsigned long long)blockIdx.x * 256 + threadIdx.x;
+    if (i >= rows * D) return;
+    const unsigned long long row = i / D;
+    const unsigned j = (unsigned)(i % D);
+    Xf[gauss_frag_at(row, j, D)] = row < N && j < d ? X[row * d + j] : 0.0f;
+    if (j == 0) yf[row] = row < N ? y[row] : 0.0f;
+}
+
+// The fp32 kernel, on the matrix cores: U = X.B in 16 x 16 tiles of rows and
+// points.  The instruction rounds after every product of a point's sum, in
+// feature order (checked against fma chains on the device), so a residual is
+// the same bits as a chain of fma; a lane's four accumulators are four
+// consecutive rows of one point, whose squares are summed in fp32 in row
+// order and then added to a double.  A block of 4 waves owns 256 points, 64
+// per wave as four column blocks whose coefficients stay in registers; the
+// next row block is loaded while one is multiplied.  The products alone bound
+// it: 100,000 x 16 rows x 4096 points take 119 us (87 at the 150 TFLOP/s
+// the instruction reaches by itself; residuals, squares and sums overlap with
+// it but for 14 us), 167 us as fma chains on the vector units.
+template <int D>
+__global__ void __launch_bounds__(256)
+glm_gauss_mfma_kernel(const f32x4* __restrict__ Xf, const f32x4* __restrict__ yf, unsigned nblocks,
+                      const float* __restrict__ P, unsigned pstride, unsigned d, unsigned n,
+                      unsigned groups, unsigned nranges, unsigned blocks_per_range,
+                      double* __restrict__ partial) {
+    constexpr int KC = D / 16, CB = 4;
     unsigned group, range;
     glm_tile(groups, group, range);
     if (range >= nranges) return;
-    // PPT points per thread, 256 apart: each broadcast read of a row feeds
-    // every point's fma
-    const unsigned k = group * (256u * PPT) + threadIdx.x;
-    float b[PPT][D];
+    const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const unsigned lr = lane & 15u, lg = lane >> 4;
+    const unsigned w0 = group * 256u + wave * 64u;
+    float b[CB][D / 4];
 #pragma unroll
-    for (int p = 0; p < PPT; ++p)
+    for (int wb = 0; wb < CB; ++wb)
 #pragma unroll
-        for (int j = 0; j < D; ++j)
-            b[p][j] = (unsigned)j < d ? P[(size_t)(k + 256u * p) * pstride + j] : 0.0f;
-    const unsigned long long r0 = (unsigned long long)range * rows_per_range;
-    unsigned long long r1 = r0 + rows_per_range;
-    if (r1 > N) r1 = N;
-    double acc[PPT];
-#pragma unroll
-    for (int p = 0; p < PPT; ++p) acc[p] = 0.0;
-    for (unsigned long long rb = r0; rb < r1; rb += TR) {
-        __syncthreads();
-        for (unsigned e = threadIdx.x; e < TR * D / 4; e += 256) {
-            const unsigned long long row = rb + (4 * e) / D;
-            xs[e] = row < r1 ? *reinterpret_cast<const float4*>(X + rb * D + 4 * e)
-                             : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        for (int q = 0; q < D / 4; ++q) {
+            const unsigned j = 4 * q + lg;
+            b[wb][q] = j < d ? P[(size_t)(w0 + wb * 16 + lr) * pstride + j] : 0.0f;
         }
-        if (threadIdx.x < TR) ys[threadIdx.x] = rb + threadIdx.x < r1 ? yv[rb + threadIdx.x] : 0.0f;
-        __syncthreads();
-        // rows past r1 are zero with y = 0: residual 0
-        for (int r = 0; r < TR; r += 4) {
-            float s4[PPT];
+    const unsigned b0 = range * blocks_per_range;
+    const unsigned b1 = b0 >= nblocks ? b0 : (nblocks - b0 < blocks_per_range ? nblocks : b0 + blocks_per_range);
+    double acc[CB] = {0.0, 0.0, 0.0, 0.0};
+    if (b0 < b1) {
+        const f32x4* xp = Xf + (size_t)b0 * KC * 64 + lane;
+        const f32x4* yp = yf + (size_t)b0 * 4 + lg;
+        f32x4 a[KC], y = *yp;
 #pragma unroll
-            for (int p = 0; p < PPT; ++p) s4[p] = 0.0f;
+        for (int kc = 0; kc < KC; ++kc) a[kc] = xp[kc * 64];
+        for (unsigned blk = b0; blk < b1; ++blk) {
+            // the next block's rows (one block of zeros follows the last),
+            // kept ahead of this one's products
+            xp += KC * 64;
+            yp += 4;
+            f32x4 an[KC];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                float t[PPT];
+            for (int kc = 0; kc < KC; ++kc) an[kc] = xp[kc * 64];
+            const f32x4 yn = *yp;
+            __builtin_amdgcn_sched_barrier(0);
+            f32x4 c[CB];
 #pragma unroll
-                for (int p = 0; p < PPT; ++p) t[p] = 0.0f;
+            for (int q = 0; q < D / 4; ++q)
 #pragma unroll
-                for (int j4 = 0; j4 < D / 4; ++j4) {
-                    const float4 x = xs[(r + i) * (D / 4) + j4];
+                for (int wb = 0; wb < CB; ++wb)
+                    c[wb] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                        a[q / 4][q % 4], b[wb][q],
+                        q == 0 ? f32x4{0.0f, 0.0f, 0.0f, 0.0f} : c[wb], 0, 0, 0);
 #pragma unroll
-                    for (int p = 0; p < PPT; ++p) {
-                        t[p] = __builtin_fmaf(x.x, b[p][4 * j4 + 0], t[p]);
-                        t[p] = __builtin_fmaf(x.y, b[p][4 * j4 + 1], t[p]);
-                        t[p] = __builtin_fmaf(x.z, b[p][4 * j4 + 2], t[p]);
-                        t[p] = __builtin_fmaf(x.w, b[p][4 * j4 + 3], t[p]);
-                    }
+            for (int wb = 0; wb < CB; ++wb) {
+                float s4 = 0.0f;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float res = y[i] - c[wb][i];
+                    s4 = __builtin_fmaf(res, res, s4);
                 }
-#pragma unroll
-                for (int p = 0; p < PPT; ++p) {
-                    const float res = ys[r + i] - t[p];
-                    s4[p] = __builtin_fmaf(res, res, s4[p]);
-                }
+                acc[wb] += (double)s4;
             }
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int p = 0; p < PPT; ++p) acc[p] += (double)s4[p];
+            for (int kc = 0; kc < KC; ++kc) a[kc] = an[kc];
+            y = yn;
         }
     }
 #pragma unroll
-    for (int p = 0; p < PPT; ++p) partial[(size_t)range * n + k + 256u * p] = acc[p];
+    for (int wb = 0; wb < CB; ++wb) {
+        double v = acc[wb];
+        v += __shfl_xor(v, 16, 64);
+        v += __shfl_xor(v, 32, 64);
+        if (lg == 0) partial[(size_t)range * n + w0 + wb * 16 + lr] = v;
+    }
 }
 
 // fp64 reference of the same sums: exact products of fp32 data and
 // coefficients, double residuals and squares.
 template <int D>
 __global__ void __launch_bounds__(256)
-glm_gauss_fp64_kernel(const float* __restrict__ X, const float* __restrict__ yv,
+glm_gauss_fp64_kernel(const float* __restrict__ Xf, const float* __restrict__ yv,
                       unsigned long long N, const float* __restrict__ P, unsigned pstride,
                       unsigned d, unsigned n, unsigned groups, unsigned nranges,
                       unsigned long long rows_per_range, double* __restrict__ partial) {
@@ -367,7 +400,7 @@ glm_gauss_fp64_kernel(const float* __restrict__ X, const float* __restrict__ yv,
         __syncthreads();
         for (unsigned e = threadIdx.x; e < TR * D; e += 256) {
             const unsigned long long row = rb + e / D;
-            xs[e] = row < r1 ? (double)X[rb * D + e] : 0.0;
+            xs[e] = row < r1 ? (double)Xf[gauss_frag_at(row, e % D, D)] : 0.0;
         }
         if (threadIdx.x < TR) ys[threadIdx.x] = rb + threadIdx.x < r1 ? (double)yv[rb + threadIdx.x] : 0.0;
         __syncthreads();
@@ -940,6 +973,23 @@ unsigned glm_blocks_per_cu(int precision, unsigned d) {
     return (unsigned)blocks;
 }
 
+unsigned glm_gauss_blocks_per_cu(int precision, unsigned D) {
+    const void* k;
+    if (precision == kGlmFp64)
+        k = D == 64   ? (const void*)glm_gauss_fp64_kernel<64>
+            : D == 32 ? (const void*)glm_gauss_fp64_kernel<32>
+                      : (const void*)glm_gauss_fp64_kernel<16>;
+    else
+        k = D == 64   ? (const void*)glm_gauss_mfma_kernel<64>
+            : D == 32 ? (const void*)glm_gauss_mfma_kernel<32>
+                      : (const void*)glm_gauss_mfma_kernel<16>;
+    int blocks = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k, 256, 0) != hipSuccess ||
+        blocks < 1)
+        return 1;
+    return (unsigned)blocks;
+}
+
 hipError_t launch_glm_logistic(int precision, hipStream_t s, const void* X, unsigned long long N,
                                unsigned d, const float* P, const void* ys, unsigned n,
                                unsigned nranges, unsigned long long rows_per_range, float yscale,
@@ -1047,11 +1097,17 @@ hipError_t launch_glm_x_to_f16(hipStream_t s, const void* X, unsigned long long 
     return hipGetLastError();
 }
 
-// Points per thread of the fp32 linear-regression kernel: 2 for up to 32
-// features (4 points at 16 features measured no faster, 2 at 64 spill) when
-// n divides into whole work-groups of 512 points.
-unsigned glm_gauss_points_per_thread(int precision, unsigned D, unsigned n) {
-    return precision == kGlmFp32 && D <= 32 && n % 512 == 0 ? 2u : 1u;
+// whole 16-row blocks and one more, which the kernel reads ahead into
+static size_t gauss_rows(unsigned long long N) { return (size_t)((N + 15) / 16 + 1) * 16; }
+size_t glm_gauss_x_floats(unsigned long long N, unsigned D) { return gauss_rows(N) * D; }
+size_t glm_gauss_y_floats(unsigned long long N) { return gauss_rows(N); }
+
+hipError_t launch_glm_gauss_pack(hipStream_t s, const float* X, const float* y,
+                                 unsigned long long N, unsigned d, unsigned D, float* Xf,
+                                 float* yf) {
+    const unsigned long long items = glm_gauss_x_floats(N, D);
+    glm_gauss_pack_kernel<<<(unsigned)((items + 255) / 256), 256, 0, s>>>(X, y, N, d, D, Xf, yf);
+    return hipGetLastError();
 }
 
 template <int D>
@@ -1062,15 +1118,11 @@ hipError_t launch_gauss_d(int precision, hipStream_t s, const float* X, const fl
     const unsigned groups = n / 256;
     const unsigned blocks = groups * nranges;
     if (precision == kGlmFp32) {
-        if (glm_gauss_points_per_thread(precision, D, n) == 2) {
-            if constexpr (D <= 32)
-                glm_gauss_fp32_kernel<D, 2><<<blocks / 2, 256, 0, s>>>(
-                    X, yv, N, P, pstride, d, n, groups / 2, nranges, rows_per_range, partial);
-        } else {
-            glm_gauss_fp32_kernel<D, 1><<<blocks, 256, 0, s>>>(X, yv, N, P, pstride, d, n,
-                                                               groups, nranges, rows_per_range,
-                                                               partial);
-        }
+        if (rows_per_range % 16) return hipErrorInvalidValue;
+        glm_gauss_mfma_kernel<D><<<blocks, 256, 0, s>>>(
+            reinterpret_cast<const f32x4*>(X), reinterpret_cast<const f32x4*>(yv),
+            (unsigned)((N + 15) / 16), P, pstride, d, n, groups, nranges,
+            (unsigned)(rows_per_range / 16), partial);
     } else if (precision == kGlmFp64) {
         glm_gauss_fp64_kernel<D><<<blocks, 256, 0, s>>>(X, yv, N, P, pstride, d, n, groups,
                                                         nranges, rows_per_range, partial);

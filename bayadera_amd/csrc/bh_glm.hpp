@@ -15,12 +15,11 @@ constexpr int kGlmFp16 = 5;
 bool glm_supported_dim(unsigned d);
 // the number of points n of a launch must be a multiple of this
 unsigned glm_point_quantum(int precision);
-// points per thread of the linear-regression likelihood kernel for n points
-// of D padded features (1 or 2); its work-groups take 256 times as many
-unsigned glm_gauss_points_per_thread(int precision, unsigned D, unsigned n);
 // work-groups of the logistic likelihood kernel of a precision that one
 // compute unit holds at once (the device's occupancy for its registers)
 unsigned glm_blocks_per_cu(int precision, unsigned d);
+// the same of the linear-regression kernel of a precision
+unsigned glm_gauss_blocks_per_cu(int precision, unsigned D);
 // partial[r][k] for r < nranges (a multiple of 8), k < n; X bf16 N x d
 // (fp16 for kGlmFp16x2), P fp32 n x d (fp32/fp64 kernels), ys the 16-bit
 // split of yscale*P (NS x n x d, MFMA kernels; fp16 terms for kGlmFp16x2).
@@ -78,9 +77,18 @@ hipError_t launch_glm_hess(hipStream_t s, const void* X, unsigned long long N, u
 hipError_t launch_glm_fp64_list(hipStream_t s, const void* X, unsigned long long N, unsigned d,
                                 const double* pts, const unsigned* count, unsigned lmax,
                                 unsigned nranges, double* partial64);
-// Linear regression sums of squared residuals (fp32 or fp64 kernels): X fp32
-// N x D (D = 16, 32 or 64, columns past d zero), points P with row stride
-// pstride whose first d coordinates are the coefficients.
+// Linear regression data in the kernels' order (glm_gauss_x_floats and
+// glm_gauss_y_floats floats, whole 16-row blocks and one more, zero past N
+// and d): X fp32
+// N x d row-major, D = 16, 32 or 64 >= d.
+size_t glm_gauss_x_floats(unsigned long long N, unsigned D);
+size_t glm_gauss_y_floats(unsigned long long N);
+hipError_t launch_glm_gauss_pack(hipStream_t s, const float* X, const float* y,
+                                 unsigned long long N, unsigned d, unsigned D, float* Xf,
+                                 float* yf);
+// Linear regression sums of squared residuals (fp32 or fp64 kernels) over the
+// packed X and y; points P with row stride pstride whose first d coordinates
+// are the coefficients; rows_per_range a multiple of 16.
 hipError_t launch_glm_gauss(int precision, hipStream_t s, const float* X, const float* yv,
                             unsigned long long N, unsigned D, const float* P, unsigned pstride,
                             unsigned d, unsigned n, unsigned nranges,
