@@ -589,10 +589,11 @@ int run_resident(bh_stretch* s, bool accu, uint32_t seed_odd, uint32_t seed_even
 // ---------------------------------------------------------------- GLM
 constexpr double kLn2 = 0.69314718055994530942;
 constexpr float kLog2e = 1.44269504088896340736f;
-// threads per walker of bh_glm_propose and bh_glm_screen (their
-// BH_GLM_TPW, BH_GLM_STPW)
+// threads per walker of bh_glm_propose (its BH_GLM_TPW)
 constexpr unsigned kGlmProposeThreads = 16;
-constexpr unsigned kGlmScreenThreads = 8;
+// points per work-group of bh_glm_screen and bh_glm_logpost (the likelihood
+// kernels' points come in multiples of 256)
+constexpr unsigned kGlmLogpostPoints = 16;
 // steps between refreshes of the split precisions' correction gradient and
 // Hessian (the ensemble's reference point moves little in 16 steps, and
 // both are always taken at the same point; the correction needs g0 to
@@ -717,7 +718,7 @@ int glm_logpost_points(bh_stretch* s, const float* P, unsigned n, double* lp) {
     const double* pc = partial;
     const double* cc = corr;
     void* a[] = {&P, &n, &pc, &nr, &lin, &scale, &pp, &lp, &cc};
-    return launch(f->glm_logpost, (n + s->wgs - 1) / s->wgs, s->wgs, 0, s->stream, a);
+    return launch(f->glm_logpost, n / kGlmLogpostPoints, s->wgs, 0, s->stream, a);
 }
 
 // One GLM half-step: proposals, the likelihood contraction, the accept test.
@@ -792,7 +793,7 @@ int glm_half(bh_stretch* s, bool first, unsigned seed, unsigned oe, unsigned ste
         const float* gsc = gscale;
         void* sa[] = {&Yc, &zc, &u2c, &pc, &nranges, &lin, &scale, &pp, &lpc, &beta, &K, &guard,
                       &flag, &list, &gcount, &lmax, &Xc, &pts64, &lpy, &cc, &gsc};
-        BH_TRY(launch(f->glm_screen, K * kGlmScreenThreads / s->wgs, s->wgs, 0, s->stream, sa));
+        BH_TRY(launch(f->glm_screen, K / kGlmLogpostPoints, s->wgs, 0, s->stream, sa));
         double* part64 = s->gpart64.as<double>();
         BH_HIP(bh::launch_glm_fp64_list(s->stream, g.X.p, g.N, g.d, pts64, gcount, lmax,
                                         guard_ranges(K), part64));

@@ -1418,6 +1418,32 @@ __device__ __forceinline__ double bh_glm_logpost_sum(const float (&y)[DIM], doub
 #endif
 }
 
+// p[0] + p[stride] + ..., n values in this order.  The chain is one thread's
+// and each load some 0.7 us away, so the time is the number of rounds of
+// loads: 32 in flight, then 8 (a small logistic regression has 768 ranges, 96
+// per thread with 8 threads to a walker).
+__device__ __forceinline__ double bh_strided_sum(const double* __restrict__ p, size_t stride,
+                                                 unsigned n) {
+    double s = 0.0;
+    unsigned r = 0;
+    for (; r + 32 <= n; r += 32) {
+        double v[32];
+#pragma unroll
+        for (int e = 0; e < 32; ++e) v[e] = p[(size_t)(r + e) * stride];
+#pragma unroll
+        for (int e = 0; e < 32; ++e) s += v[e];
+    }
+    for (; r + 8 <= n; r += 8) {
+        double v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = p[(size_t)(r + e) * stride];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s += v[e];
+    }
+    for (; r < n; ++r) s += p[(size_t)r * stride];
+    return s;
+}
+
 // The same from the per-range row sums of the likelihood kernel (the sum
 // over ranges runs in range order).
 __device__ __forceinline__ double bh_glm_logpost(const float (&y)[DIM], unsigned k, unsigned n,
@@ -1425,17 +1451,7 @@ __device__ __forceinline__ double bh_glm_logpost(const float (&y)[DIM], unsigned
                                                  unsigned nranges, const double* __restrict__ lin,
                                                  double scale, double prior_prec,
                                                  const double* __restrict__ corr) {
-    // in range order, eight loads in flight at a time
-    double s = 0.0;
-    unsigned r = 0;
-    for (; r + 8 <= nranges; r += 8) {
-        double v[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = partial[(size_t)(r + e) * n + k];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) s += v[e];
-    }
-    for (; r < nranges; ++r) s += partial[(size_t)r * n + k];
+    const double s = bh_strided_sum(partial + k, n, nranges);
     const double l = bh_glm_logpost_sum(y, s, lin, scale, prior_prec);
     return corr ? l + corr[k] : l;
 }
@@ -1461,17 +1477,95 @@ __device__ __forceinline__ double bh_wave_range_sum(const double* __restrict__ p
     return s;
 }
 
-// Initial log posteriors of n points.
+// The log posteriors of 16 consecutive points by one work-group, WGS/16
+// threads to a point: lane l of a wave takes point l % 16, so that a load of
+// the partial sums reads whole lines, and the ranges and coordinates go round
+// the point's threads (`sub` of BH_GLM_STPW).  With a point's threads side by
+// side in a wave instead, each load touched eight half-used lines on few
+// compute units: 14.4 us for 1024 points x 768 ranges, now 5.7.
+#define BH_GLM_STPW (WGS / 16)
+struct BhGlmLds {
+    double s[WGS / 64][3][16];
+    unsigned slot[16];
+};
+
+// The thread's point is k = base + lane % 16.  The result is in the first 16
+// threads of the work-group.
+__device__ __forceinline__ double bh_glm_logpost16(const float* __restrict__ P, unsigned k,
+                                                   unsigned n,
+                                                   const double* __restrict__ partial,
+                                                   unsigned nranges,
+                                                   const double* __restrict__ lin, double scale,
+                                                   double prior_prec,
+                                                   const double* __restrict__ corr,
+                                                   BhGlmLds& lds) {
+    const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const unsigned sub = threadIdx.x / 16;
+    // coordinates of the linear and quadratic terms, and their coefficients
+    // (linear regression: the coefficients' squares; log sigma by itself)
+#if BH_GLM_KIND == 2
+    constexpr unsigned QD = DIM - 1;
+    const float ls = P[(size_t)k * DIM + QD];
+#else
+    constexpr unsigned QD = DIM;
+#endif
+    constexpr unsigned SC = (QD + BH_GLM_STPW - 1) / BH_GLM_STPW;
+    float yc[SC];
+    double lc[SC];
+#pragma unroll
+    for (unsigned c = 0; c < SC; ++c) {
+        const unsigned i = sub + c * BH_GLM_STPW;
+        yc[c] = i < QD ? P[(size_t)k * DIM + i] : 0.0f;
+        lc[c] = 0.0;
+#if BH_GLM_KIND != 2
+        if (i < QD) lc[c] = lin[i];
+#endif
+    }
+    double v[3] = {0.0, 0.0, 0.0};  // row sum, linear and quadratic term
+    if (sub < nranges)
+        v[0] = bh_strided_sum(partial + (size_t)sub * n + k, (size_t)BH_GLM_STPW * n,
+                              (nranges - sub + BH_GLM_STPW - 1) / BH_GLM_STPW);
+#pragma unroll
+    for (unsigned c = 0; c < SC; ++c) {
+        const double y = (double)yc[c];
+        v[1] = __builtin_fma(lc[c], y, v[1]);
+        v[2] = __builtin_fma(y, y, v[2]);
+    }
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        v[j] += __shfl_xor(v[j], 16, 64);
+        v[j] += __shfl_xor(v[j], 32, 64);
+        if (lane < 16) lds.s[wave][j][lane] = v[j];
+    }
+    __syncthreads();
+    double lp = 0.0;
+    if (threadIdx.x < 16) {
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            v[j] = lds.s[0][j][lane];
+            for (unsigned w = 1; w < WGS / 64; ++w) v[j] += lds.s[w][j][lane];
+        }
+#if BH_GLM_KIND == 2
+        const double lsd = (double)ls;
+        lp = -lin[0] * lsd - lin[1] - 0.5 * exp(-2.0 * lsd) * v[0] -
+             0.5 * (lin[2] * v[2] + lin[3] * lsd * lsd);
+#else
+        lp = v[1] - scale * v[0] - 0.5 * prior_prec * v[2];
+#endif
+        if (corr) lp += corr[k];
+    }
+    return lp;
+}
+
+// Initial log posteriors of n points, 16 per work-group.
 extern "C" __global__ void __launch_bounds__(WGS)
 bh_glm_logpost(const float* __restrict__ P, unsigned n, const double* __restrict__ partial,
                unsigned nranges, const double* __restrict__ lin, double scale, double prior_prec,
                double* __restrict__ lp, const double* __restrict__ corr) {
-    const unsigned k = blockIdx.x * WGS + threadIdx.x;
-    if (k >= n) return;
-    float y[DIM];
-#pragma unroll
-    for (int i = 0; i < DIM; ++i) y[i] = P[(size_t)k * DIM + i];
-    lp[k] = bh_glm_logpost(y, k, n, partial, nranges, lin, scale, prior_prec, corr);
+    __shared__ BhGlmLds lds;
+    const unsigned k = blockIdx.x * 16 + (threadIdx.x & 15u);
+    const double v = bh_glm_logpost16(P, k, n, partial, nranges, lin, scale, prior_prec, corr, lds);
+    if (threadIdx.x < 16) lp[k] = v;
 }
 
 // The accept decision of stretch_move (amd-gcn-mcmc-stretch.cl:66-71): q =
@@ -1492,10 +1586,9 @@ __device__ __forceinline__ bool bh_glm_decide(double lpy, double lpx, float z, f
 // walkers, the rest counting as overflow; the engine passes lmax = K, so
 // none overflow) for an fp64 evaluation of lp(Y) and lp(X) and decided on
 // those.
-// BH_GLM_STPW threads per walker.
+// 16 walkers per work-group (bh_glm_logpost16).
 // flag[k]: 0 decided here, 3 listed (bh_glm_resolve turns it into 1 = reject
 // or 2 = accept).
-#define BH_GLM_STPW 8
 extern "C" __global__ void __launch_bounds__(WGS)
 bh_glm_screen(const float* __restrict__ Y, const float* __restrict__ zbuf,
               const float* __restrict__ u2buf, const double* __restrict__ partial,
@@ -1505,73 +1598,17 @@ bh_glm_screen(const float* __restrict__ Y, const float* __restrict__ zbuf,
               unsigned* __restrict__ count, unsigned lmax, const float* __restrict__ Xpos,
               double* __restrict__ pts64, double* __restrict__ lpy_out,
               const double* __restrict__ corr, const float* __restrict__ gscale) {
-    const unsigned gt = blockIdx.x * WGS + threadIdx.x;
-    const unsigned k = gt / BH_GLM_STPW, sub = gt % BH_GLM_STPW;
-    const unsigned base = (threadIdx.x & 63u) & ~(unsigned)(BH_GLM_STPW - 1);
-#if BH_GLM_KIND == 2
-    // (the guard is for logistic GLMs; this form is not launched)
-    double lpy = 0.0;
-    if (sub == 0) {
-        float y[DIM];
-#pragma unroll
-        for (int i = 0; i < DIM; ++i) y[i] = Y[(size_t)k * DIM + i];
-        lpy = bh_glm_logpost(y, k, K, partial, nranges, lin, scale, prior_prec, corr);
-    }
-#else
-    // the walker's BH_GLM_STPW threads (consecutive lanes) share its sums:
-    // row ranges sub, sub + STPW, ... (in that order, eight loads in
-    // flight) and coordinates likewise.  The thread's coordinates and the
-    // walker's scalars are loaded first, all together (where corr or gscale
-    // is absent the load reads lp or zbuf instead; the value is unused).
-    constexpr int SC = (DIM + BH_GLM_STPW - 1) / BH_GLM_STPW;
-    float ycv[SC];
-    double lcv[SC];
-#pragma unroll
-    for (int c = 0; c < SC; ++c) {
-        const unsigned i = sub + c * BH_GLM_STPW;
-        ycv[c] = i < DIM ? Y[(size_t)k * DIM + i] : 0.0f;
-        lcv[c] = i < DIM ? lin[i] : 0.0;
-    }
-    const float u2k = u2buf[k], zk = zbuf[k];
-    const double lpk = lp[k];
-    const double ck = (corr ? corr : lp)[k];
-    const float gsk = (gscale ? gscale : zbuf)[k];
-    double sm = 0.0, l = 0.0, q = 0.0;
-    unsigned r = sub;
-    for (; r + 7 * BH_GLM_STPW < nranges; r += 8 * BH_GLM_STPW) {
-        double v[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = partial[(size_t)(r + e * BH_GLM_STPW) * K + k];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) sm += v[e];
-    }
-    for (; r < nranges; r += BH_GLM_STPW) sm += partial[(size_t)r * K + k];
-#pragma unroll
-    for (int c = 0; c < SC; ++c) {
-        if (sub + c * BH_GLM_STPW < DIM) {
-            const double yi = (double)ycv[c];
-            l = __builtin_fma(lcv[c], yi, l);
-            q = __builtin_fma(yi, yi, q);
-        }
-    }
-#pragma unroll
-    for (int off = BH_GLM_STPW / 2; off >= 1; off >>= 1) {
-        sm += __shfl_xor(sm, off, 64);
-        l += __shfl_xor(l, off, 64);
-        q += __shfl_xor(q, off, 64);
-    }
-    double lpy = l - scale * sm - 0.5 * prior_prec * q;
-    if (corr) lpy += ck;
-#endif
-    // the walker's first thread decides or lists it; all its threads stage
-    // the listed points
-#if BH_GLM_KIND == 2
+    __shared__ BhGlmLds lds;
+    const unsigned kk = threadIdx.x & 15u, sub = threadIdx.x / 16;
+    const unsigned k = blockIdx.x * 16 + kk;
+    // the walker's scalars, ahead of the sums
     const float u2k = u2buf[k], zk = zbuf[k];
     const double lpk = lp[k];
     const float gsk = gscale ? gscale[k] : 1.0f;
-#endif
-    unsigned slot = 0xffffffffu;
-    if (sub == 0) {
+    const double lpy =
+        bh_glm_logpost16(Y, k, K, partial, nranges, lin, scale, prior_prec, corr, lds);
+    if (threadIdx.x < 16) {
+        unsigned slot = 0xffffffffu;
         lpy_out[k] = lpy;
         unsigned f = 0;
         if (__builtin_isfinite(lpy)) {
@@ -1591,8 +1628,10 @@ bh_glm_screen(const float* __restrict__ Y, const float* __restrict__ zbuf,
         // (1 reject, 2 accept; bh_glm_resolve decides the listed ones)
         if (f == 0) f = bh_glm_decide(lpy, lpk, zk, u2k, beta) ? 2u : 1u;
         flag[k] = f;
+        lds.slot[kk] = slot;
     }
-    slot = __shfl(slot, base, 64);
+    __syncthreads();
+    const unsigned slot = lds.slot[kk];
     if (slot != 0xffffffffu) {
         // the two points in double for the fp64 likelihood kernel: row 2i
         // the proposal, row 2i + 1 the current position
