@@ -1478,10 +1478,9 @@ int bh_dataset_variance_noalloc(bh_ctx* ctx, const float* data, uint32_t m, uint
     void* scr = nullptr;
     BH_HIP(bh::noalloc_scratch_init(ctx->device));
     BH_HIP(bh::noalloc_scratch(ctx->device, &scr));
-    // the same launches as bh_dataset_variance, with the partial sums and the
-    // row means in the device array instead of allocated buffers
-    float* mean = reinterpret_cast<float*>(static_cast<char*>(scr) + bh::kNoAllocPartialBytes);
-    BH_HIP(bh::launch_moments(ctx->stream, data, m, n, ld, mean, out, scr));
+    // the same launches as bh_dataset_variance, with the blocks' parts in the
+    // device array instead of allocated buffers
+    BH_HIP(bh::launch_moments(ctx->stream, data, m, n, ld, nullptr, out, scr));
     return sync(ctx->stream);
 }
 

@@ -4,10 +4,10 @@
 // accounting reductions and the autocorrelation estimator.
 //
 // Matrices are the reference's DIM x n column-major blocks (element (d, j)
-// at a[j*ld + d]).  The dataset kernels map a 256-thread block onto a tile of
-// TM rows x TN columns (TM*TN = 256, TM the next power of two >= m, capped at
-// 64 rows per pass), so every thread owns one row and consecutive threads
-// read consecutive addresses of a column.
+// at a[j*ld + d]).  The dataset kernels map a block onto a tile of TM rows x
+// TN columns (TM*TN its threads, TM the next power of two >= m, capped at 64
+// rows per pass), so every thread owns one row and consecutive threads read
+// consecutive addresses of a column.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -15,8 +15,8 @@
 #include "bh_kernels.hpp"
 #include "bh_philox.hpp"
 
-// The working memory of bh_dataset_variance_noalloc (partial sums and row
-// means), for callers that cannot allocate.  Each GPU holds its own copy at
+// The working memory of bh_dataset_variance_noalloc (the blocks' parts), for
+// callers that cannot allocate.  Each GPU holds its own copy at
 // its own address; host code reaches it only through the address that
 // noalloc_scratch_init looks up (the array's name is a host-side stand-in).
 static __device__ __align__(256) unsigned char scratch[bh::kNoAllocScratchBytes];
@@ -139,24 +139,45 @@ direct_sample_kernel(int kind, unsigned seed, float p0, float p1, unsigned quads
 __device__ __forceinline__ float ordered_min(float a, float b) { return b < a ? b : a; }
 __device__ __forceinline__ float ordered_max(float a, float b) { return b > a ? b : a; }
 
+// What the dataset kernels do with a thread's values: every column j of the
+// thread's row r with j = blockIdx * tn + cl + k * gridDim * tn, eight loads in
+// flight.  They are bound by HBM: 268 MB (2^24 x 4) in 39 to 44 us, 6.1 to 6.9
+// TB/s; with one load in flight 53 to 56 us, the histogram 88.
+template <class F>
+__device__ __forceinline__ void row_values(const float* __restrict__ a, unsigned long long n,
+                                           unsigned ld, unsigned r, unsigned tn, unsigned cl,
+                                           F&& use) {
+    constexpr unsigned U = 8;
+    const unsigned long long stride = (unsigned long long)gridDim.x * tn;
+    unsigned long long j = (unsigned long long)blockIdx.x * tn + cl;
+    const float* p = a + j * ld + r;
+    const size_t step = (size_t)stride * ld;
+    for (; j + (U - 1) * stride < n; j += U * stride) {
+        float x[U];
+#pragma unroll
+        for (unsigned u = 0; u < U; ++u) x[u] = p[u * step];
+        p += U * step;
+#pragma unroll
+        for (unsigned u = 0; u < U; ++u) use(x[u]);
+    }
+    for (; j < n; j += stride, p += step) use(*p);
+}
+
 // Per-block [min, max] of rows [r0, r0+tm) -> partial[(blk*m + r)*2 + {0,1}].
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(kDatasetThreads)
 minmax_partial_kernel(const float* __restrict__ a, unsigned m, unsigned long long n,
                       unsigned ld, unsigned r0, unsigned tm, float* __restrict__ partial) {
     const unsigned t = threadIdx.x;
-    const unsigned tn = 256 / tm;
+    const unsigned tn = kDatasetThreads / tm;
     const unsigned rl = t % tm, cl = t / tm;
     const unsigned r = r0 + rl;
     float lo = __builtin_inff(), hi = -__builtin_inff();
-    if (r < m) {
-        for (unsigned long long j = (unsigned long long)blockIdx.x * tn + cl; j < n;
-             j += (unsigned long long)gridDim.x * tn) {
-            const float x = a[j * ld + r];
+    if (r < m)
+        row_values(a, n, ld, r, tn, cl, [&](float x) {
             lo = ordered_min(lo, x);
             hi = ordered_max(hi, x);
-        }
-    }
-    __shared__ float slo[256], shi[256];
+        });
+    __shared__ float slo[kDatasetThreads], shi[kDatasetThreads];
     slo[t] = lo;
     shi[t] = hi;
     __syncthreads();
@@ -201,36 +222,58 @@ minmax_final_kernel(const float* __restrict__ partial, unsigned blocks, unsigned
 
 // bin = (uint)((x-lo)/(hi-lo)*bins) clamped to bins-1 (amd-gcn-estimate.cl:17-18);
 // v_cvt_u32_f32 saturates negative values and NaN to 0.
-__device__ __forceinline__ unsigned hist_bin(float x, float lo, float hi, unsigned bins) {
-    const float f = (x - lo) / (hi - lo) * (float)bins;
-    unsigned b = f > 0.0f ? (f >= 4294967296.0f ? 0xffffffffu : (unsigned)f) : 0u;
+__device__ __forceinline__ unsigned hist_clamp(float f, unsigned bins) {
+    const unsigned b = f > 0.0f ? (f >= 4294967296.0f ? 0xffffffffu : (unsigned)f) : 0u;
     return b < bins ? b : bins - 1;
+}
+__device__ __forceinline__ unsigned hist_bin(float x, float lo, float hi, unsigned bins) {
+    return hist_clamp((x - lo) / (hi - lo) * (float)bins, bins);
+}
+// The same bin with the row's width w = hi - lo divided by once: with y =
+// RN(1 / w), q = RN(a y) and the exact remainder r = a - q w, RN(q + r y) is
+// the correctly rounded quotient a / w (Markstein), as long as r is exact
+// (2^-60 <= w <= 2^60, and a quotient below 2^-24 is in bin 0 either way).
+// A quotient of 2 or more, also an infinite one whose remainder is not a
+// number, is in the last bin without the correction.
+__device__ __forceinline__ unsigned hist_bin_by(float x, float lo, float w, float y,
+                                                unsigned bins) {
+    const float a = x - lo;
+    float q = a * y;
+    const float c = __builtin_fmaf(__builtin_fmaf(-q, w, a), y, q);
+    q = q >= 2.0f ? q : c;
+    return hist_clamp(q * (float)bins, bins);
 }
 
 // LDS-privatised histogram of rows [r0, r0+tm): counts[r*bins + b] += n_rb.
 // Each block keeps tm x bins counters in LDS (ds_add_u32), then adds its
-// non-zero counters to global memory once.
-__global__ void __launch_bounds__(256)
+// non-zero counters to global memory once.  A division per value, 2048 blocks
+// adding their counters and one load in flight took 88 us for 2^24 x 4 values,
+// now 44.
+__global__ void __launch_bounds__(kDatasetThreads)
 histogram_kernel(const float* __restrict__ a, unsigned m, unsigned long long n, unsigned ld,
                  unsigned r0, unsigned tm, const float* __restrict__ limits, unsigned bins,
                  unsigned* __restrict__ counts) {
     extern __shared__ unsigned hist[];  // tm * bins
     const unsigned t = threadIdx.x;
-    const unsigned tn = 256 / tm;
+    const unsigned tn = kDatasetThreads / tm;
     const unsigned rl = t % tm, cl = t / tm;
     const unsigned r = r0 + rl;
-    for (unsigned i = t; i < tm * bins; i += 256) hist[i] = 0;
+    for (unsigned i = t; i < tm * bins; i += kDatasetThreads) hist[i] = 0;
     __syncthreads();
     if (r < m) {
-        const float lo = limits[2 * r], hi = limits[2 * r + 1];
+        const float lo = limits[2 * r], hi = limits[2 * r + 1], w = hi - lo;
         unsigned* h = hist + rl * bins;
-        for (unsigned long long j = (unsigned long long)blockIdx.x * tn + cl; j < n;
-             j += (unsigned long long)gridDim.x * tn) {
-            atomicAdd(&h[hist_bin(a[j * ld + r], lo, hi, bins)], 1u);
+        if (w >= 0x1p-60f && w <= 0x1p60f) {
+            const float y = 1.0f / w;
+            row_values(a, n, ld, r, tn, cl,
+                       [&](float x) { atomicAdd(&h[hist_bin_by(x, lo, w, y, bins)], 1u); });
+        } else {
+            row_values(a, n, ld, r, tn, cl,
+                       [&](float x) { atomicAdd(&h[hist_bin(x, lo, hi, bins)], 1u); });
         }
     }
     __syncthreads();
-    for (unsigned i = t; i < tm * bins; i += 256) {
+    for (unsigned i = t; i < tm * bins; i += kDatasetThreads) {
         const unsigned c = hist[i];
         const unsigned rr = r0 + i / bins;
         if (c && rr < m) atomicAdd(&counts[(size_t)rr * bins + (i % bins)], c);
@@ -274,55 +317,111 @@ histogram_finalize_kernel(const unsigned* __restrict__ counts, const float* __re
     ranks[(size_t)r * bins + lid] = vx;
 }
 
-// Row sums in double: pass 0 sums x, pass 1 sums (x - (float)mu)^2 with the
-// difference taken in float as variance_reduce does (amd-gcn-estimate.cl:146-157).
-__global__ void __launch_bounds__(256)
+// Mean and population variance of every row in one pass over the data, in
+// double (the reference's two passes round the mean and each difference to
+// float, amd-gcn-estimate.cl:146-157).  A block sums its values' differences d
+// from its own first value of the row, which are exact in double, and their
+// squares; it leaves its mean and the sum of squares about it.  The blocks'
+// parts are then combined about the mean of all (Chan, Golub, LeVeque).  With
+// a block's value as its origin, cancellation costs at most a factor of the
+// block's count of values: an origin far from the others is itself among the
+// values whose variance is taken.  partial[(blk*m + r)*3]: the block's mean of
+// row r, its sum of squares, its count.  With var 0 plain sums of the values:
+// partial[blk*m + r].
+template <int VAR>
+__global__ void __launch_bounds__(kDatasetThreads)
 moments_partial_kernel(const float* __restrict__ a, unsigned m, unsigned long long n,
-                       unsigned ld, unsigned r0, unsigned tm, const float* __restrict__ mu,
-                       double* __restrict__ partial) {
+                       unsigned ld, unsigned r0, unsigned tm, double* __restrict__ partial) {
     const unsigned t = threadIdx.x;
-    const unsigned tn = 256 / tm;
+    const unsigned tn = kDatasetThreads / tm;
     const unsigned rl = t % tm, cl = t / tm;
     const unsigned r = r0 + rl;
-    double s = 0.0;
+    double s1 = 0.0, s2 = 0.0, origin = 0.0;
+    unsigned long long count = 0;
     if (r < m) {
-        const float c = mu ? mu[r] : 0.0f;
-        for (unsigned long long j = (unsigned long long)blockIdx.x * tn + cl; j < n;
-             j += (unsigned long long)gridDim.x * tn) {
-            const float x = a[j * ld + r];
-            if (mu) {
-                const double d = (double)(x - c);
-                s = __builtin_fma(d, d, s);
-            } else {
-                s += (double)x;
-            }
+        if (VAR) {
+            // (blockIdx * tn < n: the launch has no block without columns)
+            origin = (double)a[(size_t)blockIdx.x * tn * ld + r];
+            row_values(a, n, ld, r, tn, cl, [&](float x) {
+                const double d = (double)x - origin;
+                s1 += d;
+                s2 = __builtin_fma(d, d, s2);
+                ++count;
+            });
+        } else {
+            row_values(a, n, ld, r, tn, cl, [&](float x) { s1 += (double)x; });
         }
     }
-    __shared__ double ss[256];
-    ss[t] = s;
+    __shared__ double ss[VAR ? 2 : 1][kDatasetThreads];
+    __shared__ unsigned long long sc[VAR ? kDatasetThreads : 1];
+    ss[0][t] = s1;
+    if (VAR) {
+        ss[VAR ? 1 : 0][t] = s2;
+        sc[VAR ? t : 0] = count;
+    }
     __syncthreads();
     for (unsigned k = tn / 2; k >= 1; k >>= 1) {
-        if (cl < k) ss[t] += ss[t + k * tm];
+        if (cl < k) {
+            ss[0][t] += ss[0][t + k * tm];
+            if (VAR) {
+                ss[VAR ? 1 : 0][t] += ss[VAR ? 1 : 0][t + k * tm];
+                sc[VAR ? t : 0] += sc[VAR ? t + k * tm : 0];
+            }
+        }
         __syncthreads();
     }
-    if (cl == 0 && r < m) partial[(size_t)blockIdx.x * m + r] = ss[t];
+    if (cl == 0 && r < m) {
+        if (VAR) {
+            double* o = partial + ((size_t)blockIdx.x * m + r) * 3;
+            const double c = (double)sc[VAR ? t : 0], mean = ss[0][t] / c;
+            o[0] = origin + mean;
+            o[1] = __builtin_fma(-mean, ss[0][t], ss[VAR ? 1 : 0][t]);
+            o[2] = c;
+        } else {
+            partial[(size_t)blockIdx.x * m + r] = ss[0][t];
+        }
+    }
 }
 
-// out[r] = (float)(sum of partials / n); also keeps the float mean for pass 1.
-__global__ void __launch_bounds__(256)
-moments_final_kernel(const double* __restrict__ partial, unsigned blocks, unsigned m,
-                     unsigned r0, double inv_n, float* __restrict__ out) {
-    const unsigned r = r0 + blockIdx.x;
-    double s = 0.0;
-    for (unsigned b = threadIdx.x; b < blocks; b += blockDim.x) s += partial[(size_t)b * m + r];
-    __shared__ double ss[256];
-    ss[threadIdx.x] = s;
+// Sum over the block's 256 threads, in all of them.
+__device__ __forceinline__ double block_sum256(double v, double* ss) {
     __syncthreads();
-    for (unsigned k = blockDim.x / 2; k >= 1; k >>= 1) {
+    ss[threadIdx.x] = v;
+    __syncthreads();
+    for (unsigned k = 128; k >= 1; k >>= 1) {
         if (threadIdx.x < k) ss[threadIdx.x] += ss[threadIdx.x + k];
         __syncthreads();
     }
-    if (threadIdx.x == 0) out[r] = (float)(ss[0] * inv_n);
+    return ss[0];
+}
+
+// out[r] = (float)(sum of partials / n), or the variance of the combined parts.
+template <int VAR>
+__global__ void __launch_bounds__(256)
+moments_final_kernel(const double* __restrict__ partial, unsigned blocks, unsigned m,
+                     unsigned r0, double inv_n, float* __restrict__ out) {
+    __shared__ double ss[256];
+    const unsigned r = r0 + blockIdx.x;
+    double s = 0.0;
+    if (!VAR) {
+        for (unsigned b = threadIdx.x; b < blocks; b += 256) s += partial[(size_t)b * m + r];
+        s = block_sum256(s, ss);
+        if (threadIdx.x == 0) out[r] = (float)(s * inv_n);
+        return;
+    }
+    for (unsigned b = threadIdx.x; b < blocks; b += 256) {
+        const double* p = partial + ((size_t)b * m + r) * 3;
+        s = __builtin_fma(p[0], p[2], s);
+    }
+    const double mean = block_sum256(s, ss) * inv_n;
+    double q = 0.0;
+    for (unsigned b = threadIdx.x; b < blocks; b += 256) {
+        const double* p = partial + ((size_t)b * m + r) * 3;
+        const double d = p[0] - mean;
+        q += __builtin_fma(d * d, p[2], p[1]);
+    }
+    q = block_sum256(q, ss) * inv_n;
+    if (threadIdx.x == 0) out[r] = (float)(q < 0.0 ? 0.0 : q);
 }
 
 // --------------------------------------------------------------------------
@@ -936,10 +1035,12 @@ static unsigned tile_rows(unsigned m) {
     return tm;
 }
 
-static unsigned blocks_for(unsigned long long n, unsigned tn, unsigned cap) {
-    unsigned long long b = (n + tn - 1) / tn;
-    if (b > cap) b = cap;
-    return b ? (unsigned)b : 1u;
+// blocks of a dataset kernel over n columns in tiles of tm rows: each with
+// columns of its own, a few rounds of its eight loads when there are enough
+static unsigned dataset_blocks(unsigned long long n, unsigned tm) {
+    const unsigned tn = kDatasetThreads / tm;
+    const unsigned long long b = (n + tn - 1) / tn;
+    return b < kMaxDatasetBlocks ? (unsigned)b : kMaxDatasetBlocks;
 }
 
 hipError_t launch_copy16(hipStream_t s, const void* src, void* dst, unsigned long long n16,
@@ -976,7 +1077,7 @@ hipError_t launch_direct_sample(hipStream_t s, int kind, unsigned seed, float p0
 
 size_t dataset_scratch_bytes(unsigned m, unsigned long long n) {
     (void)n;
-    return (size_t)kMaxDatasetBlocks * m * 2 * sizeof(double) + 64;
+    return (size_t)kMaxDatasetBlocks * m * 3 * sizeof(double) + 64;
 }
 
 hipError_t launch_min_max(hipStream_t s, const float* a, unsigned m, unsigned long long n,
@@ -985,8 +1086,8 @@ hipError_t launch_min_max(hipStream_t s, const float* a, unsigned m, unsigned lo
     for (unsigned r0 = 0; r0 < m; r0 += 64) {
         const unsigned rows = m - r0 < 64 ? m - r0 : 64;
         const unsigned tm = tile_rows(rows);
-        const unsigned blocks = blocks_for(n, 256 / tm, kMaxDatasetBlocks);
-        minmax_partial_kernel<<<blocks, 256, 0, s>>>(a, m, n, ld, r0, tm, partial);
+        const unsigned blocks = dataset_blocks(n, tm);
+        minmax_partial_kernel<<<blocks, kDatasetThreads, 0, s>>>(a, m, n, ld, r0, tm, partial);
         minmax_final_kernel<<<rows, 256, 0, s>>>(partial, blocks, m, r0, limits);
     }
     return hipGetLastError();
@@ -1000,9 +1101,10 @@ hipError_t launch_histogram(hipStream_t s, const float* a, unsigned m, unsigned 
     for (unsigned r0 = 0; r0 < m; r0 += per_pass) {
         const unsigned rows = m - r0 < per_pass ? m - r0 : per_pass;
         const unsigned tm = tile_rows(rows);
-        const unsigned blocks = blocks_for(n, 256 / tm, kMaxDatasetBlocks);
+        const unsigned blocks = dataset_blocks(n, tm);
         const size_t lds = (size_t)tm * bins * sizeof(unsigned);
-        histogram_kernel<<<blocks, 256, lds, s>>>(a, m, n, ld, r0, tm, limits, bins, counts);
+        histogram_kernel<<<blocks, kDatasetThreads, lds, s>>>(a, m, n, ld, r0, tm, limits, bins,
+                                                              counts);
     }
     return hipGetLastError();
 }
@@ -1018,15 +1120,18 @@ hipError_t launch_moments(hipStream_t s, const float* a, unsigned m, unsigned lo
                           unsigned ld, float* mean, float* var, void* scratch) {
     double* partial = (double*)scratch;
     const double inv_n = 1.0 / (double)n;
-    for (int pass = 0; pass < (var ? 2 : 1); ++pass) {
-        for (unsigned r0 = 0; r0 < m; r0 += 64) {
-            const unsigned rows = m - r0 < 64 ? m - r0 : 64;
-            const unsigned tm = tile_rows(rows);
-            const unsigned blocks = blocks_for(n, 256 / tm, kMaxDatasetBlocks);
-            moments_partial_kernel<<<blocks, 256, 0, s>>>(a, m, n, ld, r0, tm,
-                                                          pass ? mean : nullptr, partial);
-            moments_final_kernel<<<rows, 256, 0, s>>>(partial, blocks, m, r0, inv_n,
-                                                      pass ? var : mean);
+    for (unsigned r0 = 0; r0 < m; r0 += 64) {
+        const unsigned rows = m - r0 < 64 ? m - r0 : 64;
+        const unsigned tm = tile_rows(rows);
+        const unsigned blocks = dataset_blocks(n, tm);
+        if (var) {
+            moments_partial_kernel<1>
+                <<<blocks, kDatasetThreads, 0, s>>>(a, m, n, ld, r0, tm, partial);
+            moments_final_kernel<1><<<rows, 256, 0, s>>>(partial, blocks, m, r0, inv_n, var);
+        } else {
+            moments_partial_kernel<0>
+                <<<blocks, kDatasetThreads, 0, s>>>(a, m, n, ld, r0, tm, partial);
+            moments_final_kernel<0><<<rows, 256, 0, s>>>(partial, blocks, m, r0, inv_n, mean);
         }
     }
     return hipGetLastError();

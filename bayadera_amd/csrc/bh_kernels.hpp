@@ -4,18 +4,22 @@
 
 namespace bh {
 
-constexpr unsigned kMaxDatasetBlocks = 2048;  // 8 blocks per CU over 256 CUs
+// dataset kernels: threads per block, and blocks: two per CU over 256 CUs
+constexpr unsigned kDatasetThreads = 512;
+constexpr unsigned kMaxDatasetBlocks = 512;
 // largest work-group the context accepts (WGS); the reduction trees of acor and
 // the per-step means are sized for it
 constexpr unsigned kMaxGroupThreads = 1024;
 
 // bh_dataset_variance_noalloc: the rows one call may have, and the device
 // array (one per GPU, held until the process ends) that takes the place of
-// the buffers bh_dataset_variance allocates: kMaxDatasetBlocks x rows double
-// partial sums, then the row means.
+// the buffers bh_dataset_variance allocates (4 MiB, of which the blocks' parts
+// of the rows take three doubles each).
 constexpr unsigned kNoAllocMaxRows = 256;
-constexpr size_t kNoAllocPartialBytes = (size_t)kMaxDatasetBlocks * kNoAllocMaxRows * sizeof(double);
-constexpr size_t kNoAllocScratchBytes = kNoAllocPartialBytes + kNoAllocMaxRows * sizeof(float);
+constexpr size_t kNoAllocScratchBytes = (size_t)4 << 20;
+static_assert((size_t)kMaxDatasetBlocks * kNoAllocMaxRows * 3 * sizeof(double) <=
+                  kNoAllocScratchBytes,
+              "the parts of every row");
 // Looks up the array's address on `device`, which must be the current
 // device; once per device, later calls return at once.
 hipError_t noalloc_scratch_init(int device);
@@ -39,6 +43,7 @@ hipError_t launch_histogram(hipStream_t s, const float* a, unsigned m, unsigned 
 hipError_t launch_histogram_finalize(hipStream_t s, const unsigned* counts, const float* limits,
                                      float alpha, unsigned m, unsigned bins, float* pdf,
                                      float* ranks);
+// the rows' means, or with var (mean is not written then) their variances
 hipError_t launch_moments(hipStream_t s, const float* a, unsigned m, unsigned long long n,
                           unsigned ld, float* mean, float* var, void* scratch);
 hipError_t launch_row_tree_sum(hipStream_t s, const float* a, unsigned rows, unsigned count,

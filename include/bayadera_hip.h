@@ -179,7 +179,7 @@ int bh_dataset_variance(bh_ctx* ctx, const float* data, uint32_t m, uint64_t n, 
  * it is for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  data and
  * out must be device pointers (nothing is staged: BH_ERR_ARG otherwise) and
- * m <= 256 (BH_ERR_ARG beyond).  The partial sums and row means live in one
+ * m <= 256 (BH_ERR_ARG beyond).  The partial sums live in one
  * static device array per GPU (4 MiB, held until the process ends) instead
  * of allocated buffers; the result equals bh_dataset_variance's bit for bit.
  * Every call on a GPU shares that GPU's array, so calls that overlap on one
