@@ -286,10 +286,11 @@ histogram_kernel(const float* __restrict__ a, unsigned m, unsigned long long n, 
 // by descending pdf; ties keep the network's positional order.
 __global__ void __launch_bounds__(1024)
 histogram_finalize_kernel(const unsigned* __restrict__ counts, const float* __restrict__ limits,
-                          float alpha, unsigned bins, float* __restrict__ pdf,
-                          float* __restrict__ ranks) {
+                          float alpha, unsigned bins, float* __restrict__ limits_out,
+                          float* __restrict__ pdf, float* __restrict__ ranks) {
     const unsigned r = blockIdx.x;
     const unsigned lid = threadIdx.x;
+    if (lid < 2) limits_out[2 * r + lid] = limits[2 * r + lid];
     __shared__ float ax[1024], ay[1024];
     const float p = alpha / (limits[2 * r + 1] - limits[2 * r]) * (float)counts[(size_t)r * bins + lid];
     pdf[(size_t)r * bins + lid] = p;
@@ -512,6 +513,28 @@ sum_f64_kernel(const double* __restrict__ v, unsigned n, double* __restrict__ ou
         __syncthreads();
     }
     if (threadIdx.x == 0) *out = ss[0];
+}
+
+// A batch's acceptance rates, means and population deviations from its sums;
+// dimensions past a problem's own are 0.
+__global__ void __launch_bounds__(256)
+batch_results_kernel(const unsigned long long* __restrict__ acc, const double* __restrict__ s1,
+                     const double* __restrict__ s2, unsigned step,
+                     const unsigned* __restrict__ dims, unsigned problems, unsigned max_dim,
+                     double count, double* __restrict__ rate, double* __restrict__ mean,
+                     double* __restrict__ sd) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (rate && i < problems) rate[i] = (double)acc[i] / count;
+    if (i >= (size_t)problems * max_dim) return;
+    const unsigned p = (unsigned)(i / max_dim);
+    double m = 0.0, v = 0.0;
+    if (i - (size_t)p * max_dim < dims[p]) {
+        m = s1[i * step] / count;
+        v = s2[i * step] / count - __dmul_rn(m, m);
+        v = v > 0.0 ? v : 0.0;
+    }
+    if (mean) mean[i] = m;
+    if (sd) sd[i] = sqrt(v);
 }
 
 // --------------------------------------------------------------------------
@@ -1110,9 +1133,10 @@ hipError_t launch_histogram(hipStream_t s, const float* a, unsigned m, unsigned 
 }
 
 hipError_t launch_histogram_finalize(hipStream_t s, const unsigned* counts, const float* limits,
-                                     float alpha, unsigned m, unsigned bins, float* pdf,
-                                     float* ranks) {
-    histogram_finalize_kernel<<<m, bins, 0, s>>>(counts, limits, alpha, bins, pdf, ranks);
+                                     float alpha, unsigned m, unsigned bins, float* limits_out,
+                                     float* pdf, float* ranks) {
+    histogram_finalize_kernel<<<m, bins, 0, s>>>(counts, limits, alpha, bins, limits_out, pdf,
+                                                 ranks);
     return hipGetLastError();
 }
 
@@ -1154,6 +1178,16 @@ hipError_t launch_sum_u32(hipStream_t s, const unsigned* v, unsigned n, unsigned
 
 hipError_t launch_sum_f64(hipStream_t s, const double* v, unsigned n, double* out) {
     sum_f64_kernel<<<1, 256, 0, s>>>(v, n, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_batch_results(hipStream_t s, const unsigned long long* acc, const double* s1,
+                                const double* s2, unsigned step, const unsigned* dims,
+                                unsigned problems, unsigned max_dim, double count, double* rate,
+                                double* mean, double* sd) {
+    const size_t n = (size_t)problems * max_dim;
+    batch_results_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(
+        acc, s1, s2, step, dims, problems, max_dim, count, rate, mean, sd);
     return hipGetLastError();
 }
 

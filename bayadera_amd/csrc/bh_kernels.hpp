@@ -41,8 +41,13 @@ hipError_t launch_min_max(hipStream_t s, const float* a, unsigned m, unsigned lo
 hipError_t launch_histogram(hipStream_t s, const float* a, unsigned m, unsigned long long n,
                             unsigned ld, const float* limits, unsigned bins, unsigned* counts);
 hipError_t launch_histogram_finalize(hipStream_t s, const unsigned* counts, const float* limits,
-                                     float alpha, unsigned m, unsigned bins, float* pdf,
-                                     float* ranks);
+                                     float alpha, unsigned m, unsigned bins, float* limits_out,
+                                     float* pdf, float* ranks);
+// step: the doubles from one sum to the next; rate, mean, sd may be null
+hipError_t launch_batch_results(hipStream_t s, const unsigned long long* acc, const double* s1,
+                                const double* s2, unsigned step, const unsigned* dims,
+                                unsigned problems, unsigned max_dim, double count, double* rate,
+                                double* mean, double* sd);
 // the rows' means, or with var (mean is not written then) their variances
 hipError_t launch_moments(hipStream_t s, const float* a, unsigned m, unsigned long long n,
                           unsigned ld, float* mean, float* var, void* scratch);
