@@ -433,6 +433,9 @@ struct bh_batch {
     struct Class {
         uint32_t begin, count, dim_hi;
         int gstate;  // BH_BATCH_STATE_LDS or BH_BATCH_STATE_GLOBAL
+        // the largest sum of a pair's dimensions (the i-th largest problem and
+        // the i-th smallest), and of a pair's dimensions rounded up to odd
+        uint32_t pair, pair_odd;
     };
     int gstate = BH_BATCH_STATE_LDS;  // placement of new classes
     std::vector<Class> classes;
@@ -2039,12 +2042,43 @@ int bh_stretch_glm_guard_stats(bh_stretch* s, uint64_t* listed, uint64_t* overfl
 
 // ------------------------------------------------------------------ batch
 // LDS of one work-group of bh_batch_run: the accounting (2 max_dim doubles,
-// 2 nb floats), the proposals (nb x dim_hi floats) and, with the state in
+// 2 nb floats), the proposals (nb x dim_hi floats, an odd stride with `pad` 1
+// where that fits) and, with the state in
 // LDS, the positions and log densities (W x dim_hi + W floats).
-static size_t batch_lds(const bh_batch* b, uint32_t dim_hi, uint32_t nb, int gstate) {
-    size_t floats = (size_t)2 * nb + (size_t)nb * dim_hi;
+static size_t batch_lds(const bh_batch* b, uint32_t dim_hi, uint32_t nb, int gstate,
+                        unsigned pad = 0) {
+    size_t floats = (size_t)2 * nb + (size_t)nb * (dim_hi | pad);
     if (gstate == BH_BATCH_STATE_LDS) floats += (size_t)b->W * dim_hi + b->W;
     return (size_t)2 * b->max_dim * sizeof(double) + floats * sizeof(float);
+}
+
+// The same for a work-group that runs a pair of problems of these summed
+// dimensions, each with a half of 2 nb threads.
+static size_t batch_pair_lds(const bh_batch* b, const bh_batch::Class& cl, unsigned pad) {
+    size_t floats = (size_t)4 * b->nb + (size_t)b->nb * (pad ? cl.pair_odd : cl.pair);
+    if (cl.gstate == BH_BATCH_STATE_LDS) floats += (size_t)b->W * cl.pair + 2 * (size_t)b->W;
+    return (size_t)4 * b->max_dim * sizeof(double) + floats * sizeof(float);
+}
+
+// A launch gives every work-group the LDS of its largest problem, which
+// bounds the waves in flight where the problems' dimensions differ (52
+// coordinates: five work-groups of two waves on a compute unit, its vector
+// units 60% busy).  Pairs of a large and a small problem take twice the mean
+// (4096 posteriors of 7 to 52 dimensions, 16 steps: 1.55 -> 1.23 ms).  Taken where the LDS and not the registers (1024 threads a compute
+// unit) is the bound, where pairs put more problems on a compute unit, and
+// where the problems go round more than once (with fewer, a pair would leave
+// compute units empty).
+static bool batch_paired(const bh_batch* b, const bh_batch::Class& cl, unsigned* pad,
+                         size_t* lds) {
+    const size_t cap = (size_t)b->lds_max;
+    *pad = batch_lds(b, cl.dim_hi, b->nb, cl.gstate, 1) <= cap ? 1u : 0u;
+    *lds = batch_lds(b, cl.dim_hi, b->nb, cl.gstate, *pad);
+    const size_t slots = cap / *lds, pair = batch_pair_lds(b, cl, 1);
+    if (2 * b->nb > 1024 || slots * b->nb >= 1024 || pair > cap) return false;
+    if (2 * (cap / pair) <= slots || cl.count <= slots * (size_t)b->ctx->cu) return false;
+    *pad = 1;
+    *lds = pair;
+    return true;
 }
 
 // Launch classes from dimension bounds (ascending; the last >= every dim):
@@ -2060,7 +2094,14 @@ static int batch_set_classes(bh_batch* b, const std::vector<uint32_t>& bounds) {
         const uint32_t begin = i;
         uint32_t hi = 0;
         while (i < b->problems && b->dims_h[ord[i]] <= bound) hi = std::max(hi, b->dims_h[ord[i++]]);
-        if (i > begin) b->classes.push_back({begin, i - begin, hi, b->gstate});
+        if (i == begin) continue;
+        bh_batch::Class cl{begin, i - begin, hi, b->gstate, 0, 0};
+        for (uint32_t k = 0; k < (cl.count + 1) / 2; ++k) {
+            const uint32_t lo = b->dims_h[ord[begin + k]], up = b->dims_h[ord[i - 1 - k]];
+            cl.pair = std::max(cl.pair, lo + up);
+            cl.pair_odd = std::max(cl.pair_odd, (lo | 1u) + (up | 1u));
+        }
+        b->classes.push_back(cl);
     }
     if (i != b->problems) return fail(BH_ERR_ARG, "class bounds do not cover every dimension");
     BH_HIP(hipMemcpyAsync(b->order.p, ord.data(), ord.size() * 4, hipMemcpyHostToDevice,
@@ -2218,15 +2259,16 @@ static int batch_steps(bh_batch* b, uint32_t seed0, uint64_t n, float a, int mod
         const unsigned* ord = b->order.as<unsigned>();
         for (size_t c = 0; c < b->classes.size(); ++c) {
             const auto& cl = b->classes[c];
-            unsigned base = cl.begin;
+            unsigned base = cl.begin, count = cl.count, nb = b->nb, pad = 0;
+            size_t lds = 0;
+            const bool paired = batch_paired(b, cl, &pad, &lds);
             void* args[] = {&seed0, &dims, &poff, &dlen, &plen, &params, &xs, &lf, &W, &a,
                             &step0, &chunk, &partner, &mode, &acc, &sums, &soff, &ser, &ord,
-                            &base};
+                            &base, &count, &nb, &pad};
             if (class_events) BH_HIP(hipEventRecord((*class_events)[c], b->stream));
             BH_HIP(hipModuleLaunchKernel(cl.gstate == BH_BATCH_STATE_GLOBAL ? b->run_g : b->run,
-                                         cl.count, 1, 1, b->nb, 1, 1,
-                                         (unsigned)batch_lds(b, cl.dim_hi, b->nb, cl.gstate),
-                                         b->stream, args, nullptr));
+                                         paired ? (count + 1) / 2 : count, 1, 1,
+                                         paired ? 2 * nb : nb, 1, 1, (unsigned)lds, b->stream, args, nullptr));
         }
         if (class_events) BH_HIP(hipEventRecord(class_events->back(), b->stream));
         b->bare_counter += chunk;

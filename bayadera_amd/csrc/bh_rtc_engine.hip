@@ -886,7 +886,20 @@ bh_trace_accu(const float* __restrict__ trace, unsigned K, unsigned step0,
 // (move-bare!, constants 3333/4444) with bare seed seed0 + 2b: the same
 // streams, moves and accept tests as a sampler created for that problem
 // alone.  Positions are packed with the problem's own dimension; a proposal
-// is built in the thread's LDS slot, where the model reads it.
+// is built in the thread's LDS slot, where the model reads it.  The records of
+// a wave's 64 walkers are read, and the accepted ones written, as one run of
+// floats, 64 a pass, and the partners' beside them: with each lane at its own
+// walker's record a load took 64 lines, and the L1's lookups bounded the
+// kernel.  16 accounted steps of 4096 posteriors of 7 to 52 dimensions, 256
+// walkers each: 2.0 -> 1.1 ms.  (Groups of 16 to 64 lanes at a record each
+// need fewer instructions a pass but leave lanes idle: 5% faster there, 6%
+// slower than a lane per record at 192 posteriors of up to 34 dimensions,
+// where this is 12% faster.)  What bounds it now is the vector instructions,
+// the model's half of them.  The slots' stride is odd where the LDS has the
+// room (ypad 1), so that the lanes' loads of one coordinate take different
+// banks.  A work-group of 2 nb threads runs two problems, the i-th largest and
+// the i-th smallest of its launch, in step (see batch_paired); the largest
+// problems start first.
 // State placement (gstate): 0 copies the problem's positions and log
 // densities into LDS for the call (partner reads from LDS; the LDS a
 // problem needs bounds how many share a CU), 1 works on them in place in
@@ -897,11 +910,66 @@ bh_trace_accu(const float* __restrict__ trace, unsigned K, unsigned step0,
 // pairs, P = nb / dim residues: a serial sum over walkers p, p + P, ..., then
 // the P partial sums in order).  With series non-null it also writes each
 // step's ensemble mean (that sum over W), problem b's n x dims[b] block
-// starting at series + soff[b].  Work-group i of a launch runs problem
-// order[base + i] (problems are launched in classes of similar dimension,
-// each with the LDS it needs).
-// LDS: 2*DIM doubles + 2*nb floats + nb*dim floats (+ W*dim + W floats for
-// gstate 0).
+// starting at series + soff[b].  A launch runs the problems
+// order[base .. base + count), ascending in dimension.
+// LDS of each problem: 2*DIM doubles + 2*nb floats + nb*ld floats (+ W*dim + W
+// floats for gstate 0).
+
+// The value of lane r4 / 4.
+__device__ __forceinline__ unsigned bh_lane(unsigned v, unsigned r4) {
+    return (unsigned)__builtin_amdgcn_ds_bpermute((int)r4, (int)v);
+}
+__device__ __forceinline__ float bh_lane(float v, unsigned r4) {
+    return __builtin_bit_cast(float, bh_lane(__builtin_bit_cast(unsigned, v), r4));
+}
+
+// A wave's 64 records of dim coordinates as one run of floats, 64 a pass: the
+// record (r4 / 4) and the coordinate (iy, in bytes, with the offset of the
+// wave's proposals in the LDS added) of a lane's element of a pass.
+struct BhRun {
+    unsigned r4, iy;
+    struct Steps {
+        unsigned dr4, di4, dim4, end;  // end: where iy is past a record
+    };
+    __device__ __forceinline__ void next(const Steps& s) {
+        iy += s.di4;
+        const bool past = iy >= s.end;
+        r4 += past ? s.dr4 + 4u : s.dr4;
+        iy -= past ? s.dim4 : 0u;
+    }
+};
+
+struct BhTrue {
+    static constexpr bool v = true;
+};
+struct BhFalse {
+    static constexpr bool v = false;
+};
+
+// A place in the LDS as a byte offset, and the float at one.
+__device__ __forceinline__ unsigned bh_lds_offset(const float* p) {
+    return (unsigned)(size_t)(__attribute__((address_space(3))) const float*)p;
+}
+__device__ __forceinline__ float& bh_lds(unsigned bytes) {
+    return *(float*)(__attribute__((address_space(3))) float*)(size_t)bytes;
+}
+
+// The float at a byte offset of 32 bits (one address register on a scalar base).
+__device__ __forceinline__ float& bh_at(float* p, unsigned bytes) {
+    return *reinterpret_cast<float*>(reinterpret_cast<char*>(p) + bytes);
+}
+__device__ __forceinline__ float bh_at(const float* p, unsigned bytes) {
+    return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(p) + bytes);
+}
+
+// A wave's LDS stores before, its other lanes' loads after (LDS operations of
+// a wave complete in order).
+__device__ __forceinline__ void bh_wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
 template <bool GSTATE>
 __device__ __forceinline__ void bh_batch_impl(
     unsigned seed0, const unsigned* __restrict__ dims, const unsigned long long* __restrict__ poff,
@@ -910,22 +978,31 @@ __device__ __forceinline__ void bh_batch_impl(
     unsigned W, float a, unsigned step0, unsigned nsteps, int partner, int mode,
     unsigned long long* __restrict__ accept, double* __restrict__ sums,
     const unsigned long long* __restrict__ soff, float* __restrict__ series,
-    const unsigned* __restrict__ order, unsigned base) {
+    const unsigned* __restrict__ order, unsigned base, unsigned count, unsigned nb,
+    unsigned ypad) {
     extern __shared__ double lds_d[];
-    const unsigned b = order[base + blockIdx.x];
+    // the work-group's blockIdx-th largest problem, and in its second half (if
+    // it has one) the blockIdx-th smallest
+    const unsigned half = (unsigned)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >= nb));
+    const unsigned big = order[base + count - 1u - blockIdx.x];
+    const unsigned b = half ? order[base + blockIdx.x] : big;
     const unsigned dim = dims[b];
-    const unsigned K = W / 2;
-    const unsigned t = threadIdx.x, nb = blockDim.x;
+    const bool idle = half && b == big;  // the middle one of an odd count
+    const unsigned K = idle ? 0u : W / 2;
+    const unsigned t = threadIdx.x - half * nb;
     const float* prm = params + poff[b];
     const unsigned data_len = dlen[b], params_len = plen[b];
     float* gx = xs + (size_t)b * W * DIM;  // problem slot: W x DIM floats, packed by dim
     float* gl = logfn + (size_t)b * W;
+    const unsigned dim0 = half ? dims[big] : 0;  // the first half's share of the LDS
     double* acc1 = lds_d;                  // DIM
+    if (half)
+        acc1 += 2 * DIM + (2 * nb + nb * (dim0 | ypad) + (GSTATE ? 0 : W * dim0 + W)) / 2;
     double* acc2 = acc1 + DIM;             // DIM
     float* red = reinterpret_cast<float*>(acc2 + DIM);  // 2 * nb
     float* sx;                             // W * dim
     float* sl;                             // W
-    float* yb;                             // nb * dim
+    float* yb;                             // nb * ld
     if constexpr (GSTATE) {
         sx = gx;
         sl = gl;
@@ -944,7 +1021,18 @@ __device__ __forceinline__ void bh_batch_impl(
     const float inv_a = 1.0f / a;
     const float ca = a - 2.0f + inv_a;
     const float cb = 2.0f * (1.0f - inv_a);
-    float* y = yb + (size_t)t * dim;
+    const unsigned ld = dim | ypad;  // odd if the LDS has the room
+    const unsigned lane = t & 63u;
+    float* yw = yb + (size_t)(t - lane) * ld;  // the wave's proposals
+    const float* y = yw + lane * ld;
+    constexpr int N = 8;  // passes in flight
+    const unsigned yw4 = (unsigned)__builtin_amdgcn_readfirstlane((int)bh_lds_offset(yw));
+    const unsigned sx4 = GSTATE ? 0u : bh_lds_offset(sx), dim4 = 4 * dim;
+    const BhRun run0{4 * (lane / dim), yw4 + 4 * (lane % dim)};
+    const BhRun::Steps steps{4 * (64u / dim), 4 * (64u % dim), dim4, yw4 + dim4};
+    // the problem's slot as a buffer of its own size
+    const __amdgpu_buffer_rsrc_t xbuf =
+        __builtin_amdgcn_make_buffer_rsrc(gx, 0, (int)(W * dim4), 0x00020000);
     const unsigned P = dim <= nb ? nb / dim : 1u;
     for (unsigned st = 0; st < nsteps; ++st) {
         const unsigned step = step0 + st;
@@ -957,78 +1045,152 @@ __device__ __forceinline__ void bh_batch_impl(
                     bh_u32x4{k, step, h ? 4444u : 3333u, BH_CTR3}, seed + (unsigned)h,
                     BH_KEY1_STRETCH));
                 const float z = __builtin_fmaf(ca * u.y, u.y, cb * u.y) + inv_a;
-                const float* xk = X + (size_t)k * dim;
                 // partner element i at S[(e + i) mod K*dim] (FLAT) or
-                // S[j*dim + i] (WALKER); eight coordinates' loads in flight
-                const unsigned total = K * dim;
+                // S[j*dim + i] (WALKER); e in bytes
+                const unsigned total = 4 * K * dim;
                 unsigned e;
                 if (partner == BH_PARTNER_FLAT) {
                     e = (unsigned)((u.x * (float)K) * (float)dim);
-                    if (e >= total) e -= total;
+                    if (e >= K * dim) e -= K * dim;
                 } else {
                     unsigned j = (unsigned)(u.x * (float)K);
                     j = j < K ? j : K - 1;
-                    e = j * dim;  // e + i < total for i < dim
+                    e = j * dim;  // e + i < K * dim for i < dim
                 }
-                unsigned i = 0;
-                for (; i + 8 <= dim; i += 8) {
-                    float xa[8], sa[8];
+                e *= 4;
+                // the wave's records (a scalar base, byte offsets below)
+                float* xw = X + (size_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(k - lane)) * dim;
+                const float lk = L[k];
+                e -= yw4;  // + iy: the coordinate's place
+                BhRun at = run0;
+                // N passes from the j-th, all of them in the records (FULL)
+                const auto propose = [&](unsigned j, auto FULL) {
+                    float xa[N], sa[N], zr[N];
+                    unsigned ec[N], yo[N];
 #pragma unroll
-                    for (int c = 0; c < 8; ++c) {
-                        unsigned ec = e + c;
-                        if (ec >= total) ec -= total;
-                        xa[c] = xk[i + c];
-                        sa[c] = S[ec];
+                    for (int c = 0; c < N; ++c) {
+                        ec[c] = bh_lane(e, at.r4) + at.iy;
+                        zr[c] = bh_lane(z, at.r4);
+                        yo[c] = __umul24(at.r4, ld) + at.iy;
+                        at.next(steps);
                     }
 #pragma unroll
-                    for (int c = 0; c < 8; ++c) y[i + c] = __builtin_fmaf(z, xa[c] - sa[c], sa[c]);
-                    e += 8;
-                    if (e >= total) e -= total;
-                }
-                for (; i < dim; ++i) {
-                    const float xj = S[e];
-                    y[i] = __builtin_fmaf(z, xk[i] - xj, xj);
-                    e = (e + 1 == total) ? 0u : e + 1;
-                }
+                    for (int c = 0; c < N; ++c) {
+                        // (a pass past the records loads from within them)
+                        xa[c] = bh_at(xw + 64 * (FULL.v || j + c < dim ? j + c : j), 4 * lane);
+                        // past the end: from the start (the smaller, unsigned)
+                        sa[c] = bh_at(S, ec[c] - total < ec[c] ? ec[c] - total : ec[c]);
+                    }
+#pragma unroll
+                    for (int c = 0; c < N; ++c)
+                        if (FULL.v || j + c < dim)
+                            bh_lds(yo[c]) = __builtin_fmaf(zr[c], xa[c] - sa[c], sa[c]);
+                };
+                unsigned j = 0;
+                for (; j + N <= dim; j += N) propose(j, BhTrue{});
+                if (j < dim) propose(j, BhFalse{});
+                bh_wave_sync();
                 const float ly = LOGFN(data_len, params_len, prm, dim, y);
                 float zp = 1.0f;
+#pragma unroll 4
                 for (unsigned i = 1; i < dim; ++i) zp *= z;
-                const float q = __builtin_isfinite(ly) ? zp * expf(ly - L[k]) : 0.0f;
-                if (u.z <= q) {
-                    for (unsigned i = 0; i < dim; ++i) X[(size_t)k * dim + i] = y[i];
+                const float q = __builtin_isfinite(ly) ? zp * expf(ly - lk) : 0.0f;
+                const bool accepted = u.z <= q;
+                if (accepted) {
                     L[k] = ly;
                     nacc += 1;
                 }
+                bh_wave_sync();
+                if (__builtin_amdgcn_ballot_w64(accepted) != 0) {
+                    // no branch: what did not move is stored past the buffer's
+                    // end, which the hardware drops, or (LDS) onto the
+                    // proposal itself
+                    const unsigned keep = accepted ? 0u : 0x80000000u;
+                    const unsigned xo = (unsigned)(xw - sx) * 4;
+                    at = run0;
+                    const auto move = [&](unsigned j, auto FULL) {
+                        float ya[N];
+                        unsigned kept[N], yo[N];
+#pragma unroll
+                        for (int c = 0; c < N; ++c) {
+                            kept[c] = bh_lane(keep, at.r4);
+                            yo[c] = __umul24(at.r4, ld) + at.iy;
+                            at.next(steps);
+                        }
+#pragma unroll
+                        for (int c = 0; c < N; ++c)
+                            ya[c] = bh_lds(FULL.v || j + c < dim ? yo[c] : yo[0]);
+#pragma unroll
+                        for (int c = 0; c < N; ++c)
+                            if (FULL.v || j + c < dim) {
+                                if constexpr (GSTATE)
+                                    __builtin_amdgcn_raw_buffer_store_b32(
+                                        __builtin_bit_cast(unsigned, ya[c]), xbuf,
+                                        4 * lane | kept[c], (int)(xo + 256 * (j + c)), 0);
+                                else
+                                    bh_lds(kept[c] ? yo[c]
+                                                   : sx4 + xo + 256 * (j + c) + 4 * lane) = ya[c];
+                            }
+                    };
+                    unsigned j = 0;
+                    for (; j + N <= dim; j += N) move(j, BhTrue{});
+                    if (j < dim) move(j, BhFalse{});
+                }
+                bh_wave_sync();
             }
             __syncthreads();
         }
         if (mode == 1) {
             if (dim <= nb) {
-                if (t < P * dim) {
+                if (t < P * dim && !idle) {
                     const unsigned d = t % dim, p = t / dim;
                     float s1 = 0.0f, s2 = 0.0f;
-                    unsigned w = p;
-                    // walkers p, p + P, ... in order, eight loads in flight
-                    for (; w + 7 * P < W; w += 8 * P) {
-                        float xv[8];
+                    // walkers p, p + P, ... in order, N loads in flight
+                    const unsigned wstep = 4 * P * dim, wend = 4 * W * dim;
+                    unsigned wo = 4 * (p * dim + d);
+                    for (; wo + (N - 1) * wstep < wend; wo += N * wstep) {
+                        float xv[N];
 #pragma unroll
-                        for (int c = 0; c < 8; ++c) xv[c] = sx[(size_t)(w + c * P) * dim + d];
+                        for (int c = 0; c < N; ++c) xv[c] = bh_at(sx, wo + c * wstep);
 #pragma unroll
-                        for (int c = 0; c < 8; ++c) {
+                        for (int c = 0; c < N; ++c) {
                             s1 += xv[c];
                             s2 = __builtin_fmaf(xv[c], xv[c], s2);
                         }
                     }
-                    for (; w < W; w += P) {
-                        const float x = sx[(size_t)w * dim + d];
-                        s1 += x;
-                        s2 = __builtin_fmaf(x, x, s2);
+                    if (wo < wend) {
+                        float xv[N];
+#pragma unroll
+                        for (int c = 0; c < N; ++c)
+                            xv[c] = bh_at(sx, wo + c * wstep < wend ? wo + c * wstep : wo);
+#pragma unroll
+                        for (int c = 0; c < N; ++c)
+                            if (wo + c * wstep < wend) {
+                                s1 += xv[c];
+                                s2 = __builtin_fmaf(xv[c], xv[c], s2);
+                            }
                     }
                     red[t] = s1;
                     red[nb + t] = s2;
                 }
-                __syncthreads();
-                if (t < dim) {
+            } else {
+                for (unsigned d = t; d < dim && !idle; d += nb) {
+                    float s1 = 0.0f, s2 = 0.0f;
+                    for (unsigned w = 0; w < W; ++w) {
+                        const float x = sx[(size_t)w * dim + d];
+                        s1 += x;
+                        s2 = __builtin_fmaf(x, x, s2);
+                    }
+                    acc1[d] += (double)s1;
+                    acc2[d] += (double)s2;
+                    if (series) series[soff[b] + (size_t)st * dim + d] = s1 / (float)W;
+                }
+            }
+            // the next step's first half writes accepted proposals into sx,
+            // which these sums read
+            __syncthreads();
+            if (dim <= nb) {
+                if (t < dim && !idle) {
                     float s1 = 0.0f, s2 = 0.0f;
                     for (unsigned p = 0; p < P; ++p) {
                         s1 += red[p * dim + t];
@@ -1040,25 +1202,10 @@ __device__ __forceinline__ void bh_batch_impl(
                 }
                 // red is written again only after the next step's two
                 // half-step barriers
-            } else {
-                for (unsigned d = t; d < dim; d += nb) {
-                    float s1 = 0.0f, s2 = 0.0f;
-                    for (unsigned w = 0; w < W; ++w) {
-                        const float x = sx[(size_t)w * dim + d];
-                        s1 += x;
-                        s2 = __builtin_fmaf(x, x, s2);
-                    }
-                    acc1[d] += (double)s1;
-                    acc2[d] += (double)s2;
-                    if (series) series[soff[b] + (size_t)st * dim + d] = s1 / (float)W;
-                }
-                // the next step's first half writes accepted proposals into
-                // sx, which these sums read
-                __syncthreads();
             }
         }
     }
-    if constexpr (!GSTATE) {
+    if (!GSTATE && !idle) {
         for (unsigned i = t; i < W * dim; i += nb) gx[i] = sx[i];
         for (unsigned i = t; i < W; i += nb) gl[i] = sl[i];
     }
@@ -1071,8 +1218,8 @@ __device__ __forceinline__ void bh_batch_impl(
         if (t < r) ra[t] += ra[t + r];
         __syncthreads();
     }
-    if (t == 0) accept[b] += ra[0];
-    if (mode == 1) {
+    if (t == 0 && !idle) accept[b] += ra[0];
+    if (mode == 1 && !idle) {
         for (unsigned i = t; i < dim; i += nb) {
             sums[((size_t)b * DIM + i) * 2] += acc1[i];
             sums[((size_t)b * DIM + i) * 2 + 1] += acc2[i];
@@ -1090,9 +1237,11 @@ __device__ __forceinline__ void bh_batch_impl(
         float* __restrict__ xs, float* __restrict__ logfn, unsigned W, float a, unsigned step0,   \
         unsigned nsteps, int partner, int mode, unsigned long long* __restrict__ accept,          \
         double* __restrict__ sums, const unsigned long long* __restrict__ soff,                   \
-        float* __restrict__ series, const unsigned* __restrict__ order, unsigned base) {          \
+        float* __restrict__ series, const unsigned* __restrict__ order, unsigned base,            \
+        unsigned count, unsigned nb, unsigned ypad) {                                             \
         bh_batch_impl<GSTATE>(seed0, dims, poff, dlen, plen, params, xs, logfn, W, a, step0,      \
-                              nsteps, partner, mode, accept, sums, soff, series, order, base);    \
+                              nsteps, partner, mode, accept, sums, soff, series, order, base,     \
+                              count, nb, ypad);                                                   \
     }
 BH_BATCH_RUN_KERNEL(bh_batch_run, false)
 BH_BATCH_RUN_KERNEL(bh_batch_run_g, true)
