@@ -388,18 +388,24 @@ const double* glm_lin(const GlmData& g, int prec) {
     return (prec == BH_GLM_FP64 ? g.lin : g.lin_half).as<double>();
 }
 
+// How a likelihood launch divides the rows: `runs` runs of `rpr` rows, shared
+// between `nranges` work-group ranges.
+struct GlmRows {
+    unsigned nranges, runs;
+    unsigned long long rpr;
+};
+
 // The likelihood contraction of n points P (row stride = the walker
 // dimension) into partial[nranges][n].
 int glm_contract(const GlmData& g, int prec, hipStream_t st, const float* P, unsigned pstride,
-                 const void* ys, unsigned n, unsigned nranges, unsigned long long rpr,
-                 float yscale, double* partial) {
+                 const void* ys, unsigned n, const GlmRows& r, float yscale, double* partial) {
     if (g.kind == BH_GLM_GAUSSIAN) {
         BH_HIP(bh::launch_glm_gauss(prec, st, g.Xf.as<float>(), g.y.as<float>(), g.N, g.D, P,
-                                    pstride, g.d, n, nranges, rpr, partial));
+                                    pstride, g.d, n, r.nranges, r.rpr, partial));
     } else {
         const void* X = (prec == BH_GLM_FP16X2 || prec == BH_GLM_FP16) ? g.X16.p : g.X.p;
-        BH_HIP(bh::launch_glm_logistic(prec, st, X, g.N, g.d, P, ys, n, nranges, rpr, yscale,
-                                       partial));
+        BH_HIP(bh::launch_glm_logistic(prec, st, X, g.N, g.d, P, ys, n, r.nranges, r.rpr,
+                                       r.runs, yscale, partial));
     }
     return BH_OK;
 }
@@ -509,6 +515,8 @@ constexpr uint32_t kResidentAnyDensity = 1024;
 constexpr uint64_t kResidentData = 100000;
 constexpr uint64_t kResidentParams = 1000000;
 
+// runs of rows shorter than this are shared out (see glm_rows)
+constexpr unsigned kGlmShortRun = 512;
 // rounds of work-groups per logistic likelihood launch
 constexpr unsigned kGlmRounds = 4;
 // and per linear-regression launch
@@ -765,18 +773,31 @@ int glm_prepare(bh_stretch_factory* f, int prec) {
     return BH_OK;
 }
 
+// Work-groups per compute unit that the runs of rows of a matrix-core launch
+// are cut for.  A constant, not the occupancy of the kernel as it is compiled:
+// the runs decide how the float sums round.
+unsigned glm_run_blocks(int prec, unsigned d) {
+    switch (prec) {
+    case BH_GLM_BF16:
+    case BH_GLM_FP16: return d == 64 ? 4 : 6;
+    case BH_GLM_FP16X2: return d == 64 ? 3 : 4;
+    default: return d == 64 ? 2 : 4;  // BH_GLM_BF16X3
+    }
+}
+
 // row ranges of one likelihood launch over n points: a multiple of 8.  The
-// logistic kernels get whole rounds of work-groups (the compute units times
-// the work-groups one holds at once for the kernel's registers): a partial
-// last round leaves compute units idle; a few rounds of smaller ranges even
-// out the ranges' finishing times.
+// logistic kernels get whole rounds of work-groups: a partial last round
+// leaves compute units idle; a few rounds of smaller ranges even out the
+// ranges' finishing times.  (The matrix-core kernels' ranges are the runs of
+// rows that glm_rows shares out.)
 unsigned glm_ranges(const bh_ctx* c, const GlmData& g, int prec, unsigned n) {
     const unsigned groups = std::max(n / bh::glm_point_quantum(prec), 1u);
     if (!g.bpc[prec])
         g.bpc[prec] = g.kind == BH_GLM_GAUSSIAN ? bh::glm_gauss_blocks_per_cu(prec, g.D)
                                                 : bh::glm_blocks_per_cu(prec, g.d);
     const unsigned rounds = g.kind == BH_GLM_GAUSSIAN ? kGaussRounds : kGlmRounds;
-    const unsigned blocks = rounds * g.bpc[prec] * (unsigned)c->cu;
+    const bool mfma = g.kind == BH_GLM_LOGISTIC && prec != BH_GLM_FP64 && prec != BH_GLM_FP32;
+    const unsigned blocks = rounds * (mfma ? glm_run_blocks(prec, g.d) : g.bpc[prec]) * (unsigned)c->cu;
     unsigned r = (blocks + groups - 1) / groups;
     r = (r + 7) / 8 * 8;
     const unsigned long long max_r = std::max(8ull, (g.N / 64 + 7) / 8 * 8);
@@ -784,13 +805,32 @@ unsigned glm_ranges(const bh_ctx* c, const GlmData& g, int prec, unsigned n) {
     return std::max(r, 8u);
 }
 
+// The rows of a launch over n points.  glm_ranges' ranges fix the runs of rows
+// whose terms are summed in floats; where they are short, the work-groups of
+// one round share them out, so that each loads its points' fragments once (the
+// latency of those loads is that of some 100 rows' work) and the sums after it
+// have a quarter of the partials to read: 50,021 x 32, 1024 points, runs of 80
+// rows 16.5 -> 14.3 us and a half-step 5 us less; steps of 30,239 x 32, runs
+// of 96, 11% less, of 298,857 x 64, runs of 448, 0.5%.  Long runs keep their
+// four rounds, which even out the work-groups' finishing times: 1M x 64, runs
+// of 10,432, one round 29.3 ms, four 27.0.
+GlmRows glm_rows(const bh_ctx* c, const GlmData& g, int prec, unsigned n) {
+    const unsigned nranges = glm_ranges(c, g, prec, n);
+    GlmRows r{nranges, nranges, ((g.N + nranges - 1) / nranges + 15) / 16 * 16};
+    if (g.kind != BH_GLM_LOGISTIC || prec == BH_GLM_FP64 || prec == BH_GLM_FP32) return r;
+    r.runs = (unsigned)((g.N + r.rpr - 1) / r.rpr);
+    const unsigned groups = std::max(n / bh::glm_point_quantum(prec), 1u);
+    const unsigned slots = g.bpc[prec] * (unsigned)c->cu / groups / 8 * 8;
+    if (r.rpr < kGlmShortRun && slots > 0 && slots < r.runs) r.nranges = slots;
+    return r;
+}
+
 // log posteriors of n points P (device, n x d) into lp (double, device).
 int glm_logpost_points(bh_stretch* s, const float* P, unsigned n, double* lp) {
     bh_stretch_factory* f = s->f;
     const GlmData& g = *f->glm;
     const int prec = s->glm_prec;
-    const unsigned nranges = glm_ranges(s->ctx, g, prec, n);
-    const unsigned long long rpr = ((g.N + nranges - 1) / nranges + 15) / 16 * 16;
+    const GlmRows rows = glm_rows(s->ctx, g, prec, n);
     int nsplit = glm_nsplit(prec);
     int f16 = glm_f16(prec);
     float yscale = kLog2e;
@@ -807,11 +847,11 @@ int glm_logpost_points(bh_stretch* s, const float* P, unsigned n, double* lp) {
         BH_TRY(launch(f->glm_split, (n + s->wgs - 1) / s->wgs, s->wgs, 0, s->stream, a));
     }
     double* partial = s->gpartial.as<double>();
-    BH_TRY(glm_contract(g, prec, s->stream, P, s->dim, ys, n, nranges, rpr, yscale, partial));
+    BH_TRY(glm_contract(g, prec, s->stream, P, s->dim, ys, n, rows, yscale, partial));
     const double* lin = glm_lin(g, prec);
     double scale = prec == BH_GLM_FP64 ? 1.0 : kLn2;
     double pp = g.prior_prec;
-    unsigned nr = nranges;
+    unsigned nr = rows.nranges;
     const double* pc = partial;
     const double* cc = corr;
     void* a[] = {&P, &n, &pc, &nr, &lin, &scale, &pp, &lp, &cc};
@@ -859,12 +899,11 @@ int glm_half(bh_stretch* s, bool first, unsigned seed, unsigned oe, unsigned ste
     void* pa[] = {&seed, &oe, &S, &Xc, &a, &step, &K, &partner, &Y, &z, &u2, &ys, &yscale, &nsplit,
                   &f16, &gcount, &g0, &lnscale, &corr, &H0, &bref, &gscale};
     BH_TRY(launch(f->glm_propose, K * kGlmProposeThreads / s->wgs, s->wgs, 0, s->stream, pa));
-    unsigned nranges = glm_ranges(s->ctx, g, prec, K);
-    const unsigned long long rpr = ((g.N + nranges - 1) / nranges + 15) / 16 * 16;
+    const GlmRows rows = glm_rows(s->ctx, g, prec, K);
+    unsigned nranges = rows.nranges;
     double* partial = s->gpartial.as<double>();
     BH_TRY(ktimed(s, [&]() -> int {
-        BH_TRY(glm_contract(g, prec, s->stream, Y, s->dim, ys, K, nranges, rpr, yscale,
-                            partial));
+        BH_TRY(glm_contract(g, prec, s->stream, Y, s->dim, ys, K, rows, yscale, partial));
         return BH_OK;
     }));
     const double* lin = glm_lin(g, prec);

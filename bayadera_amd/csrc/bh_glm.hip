@@ -103,7 +103,7 @@ struct Frag16 {
 template <int D, int NS, class T, class V>
 __global__ void __launch_bounds__(256)
 glm_logistic_mfma_kernel(const T* __restrict__ X, unsigned N, const T* __restrict__ ys, unsigned n,
-                         unsigned groups, unsigned nranges, unsigned rows_per_range,
+                         unsigned groups, unsigned nranges, unsigned rows_per_range, unsigned runs,
                          double* __restrict__ partial) {
     constexpr int KC = D / 32;
     const unsigned lane = threadIdx.x & 63u;
@@ -124,10 +124,14 @@ glm_logistic_mfma_kernel(const T* __restrict__ X, unsigned N, const T* __restric
                 bfrag[wb][kc][s] = *reinterpret_cast<const V*>(
                     ys + ((size_t)s * n + w0 + wb * 16 + lr) * D + kc * 32 + lg * 8);
 
-    const unsigned r0 = range * rows_per_range;
-    const unsigned r1 = (r0 >= N) ? r0 : ((N - r0 < rows_per_range) ? N : r0 + rows_per_range);
     double acc[4] = {0.0, 0.0, 0.0, 0.0};
-    if (r0 < r1) {
+    // `runs` runs of rows over the ranges, the first ranges one more
+    const unsigned each = runs / nranges, more = runs % nranges;
+    const unsigned q0 = range * each + (range < more ? range : more);
+    const unsigned q1 = q0 + each + (range < more ? 1u : 0u);
+    for (unsigned q = q0; q < q1; ++q) {
+        const unsigned r0 = q * rows_per_range;
+        const unsigned r1 = N - r0 < rows_per_range ? N : r0 + rows_per_range;
         if constexpr (__is_same(T, _Float16))
             glm_mfma_rows<D, NS, 4>(Frag16<D, T, V>{X, lr, lg}, bfrag, r0, r1, lg, acc);
         else
@@ -881,7 +885,7 @@ glm_lin_final_kernel(const double* __restrict__ part, unsigned chunks, unsigned 
 template <int D>
 static hipError_t launch_d(int precision, hipStream_t s, const void* Xv, unsigned long long N,
                            const float* P, const void* ysv, unsigned n, unsigned nranges,
-                           unsigned long long rpr, float yscale, double* partial) {
+                           unsigned long long rpr, unsigned runs, float yscale, double* partial) {
     const __bf16* X = static_cast<const __bf16*>(Xv);
     const __bf16* ys = static_cast<const __bf16*>(ysv);
     const _Float16* X16 = static_cast<const _Float16*>(Xv);
@@ -890,25 +894,25 @@ static hipError_t launch_d(int precision, hipStream_t s, const void* Xv, unsigne
     case kGlmBf16: {
         const unsigned groups = n / 256;
         glm_logistic_mfma_kernel<D, 1, __bf16, bf16x8><<<groups * nranges, 256, 0, s>>>(
-            X, (unsigned)N, ys, n, groups, nranges, (unsigned)rpr, partial);
+            X, (unsigned)N, ys, n, groups, nranges, (unsigned)rpr, runs, partial);
         break;
     }
     case kGlmBf16x3: {
         const unsigned groups = n / 256;
         glm_logistic_mfma_kernel<D, 3, __bf16, bf16x8><<<groups * nranges, 256, 0, s>>>(
-            X, (unsigned)N, ys, n, groups, nranges, (unsigned)rpr, partial);
+            X, (unsigned)N, ys, n, groups, nranges, (unsigned)rpr, runs, partial);
         break;
     }
     case kGlmFp16x2: {
         const unsigned groups = n / 256;
         glm_logistic_mfma_kernel<D, 2, _Float16, f16x8><<<groups * nranges, 256, 0, s>>>(
-            X16, (unsigned)N, ys16, n, groups, nranges, (unsigned)rpr, partial);
+            X16, (unsigned)N, ys16, n, groups, nranges, (unsigned)rpr, runs, partial);
         break;
     }
     case kGlmFp16: {
         const unsigned groups = n / 256;
         glm_logistic_mfma_kernel<D, 1, _Float16, f16x8><<<groups * nranges, 256, 0, s>>>(
-            X16, (unsigned)N, ys16, n, groups, nranges, (unsigned)rpr, partial);
+            X16, (unsigned)N, ys16, n, groups, nranges, (unsigned)rpr, runs, partial);
         break;
     }
     case kGlmFp32: {
@@ -992,10 +996,14 @@ unsigned glm_gauss_blocks_per_cu(int precision, unsigned D) {
 
 hipError_t launch_glm_logistic(int precision, hipStream_t s, const void* X, unsigned long long N,
                                unsigned d, const float* P, const void* ys, unsigned n,
-                               unsigned nranges, unsigned long long rows_per_range, float yscale,
-                               double* partial) {
-    if (d == 64) return launch_d<64>(precision, s, X, N, P, ys, n, nranges, rows_per_range, yscale, partial);
-    if (d == 32) return launch_d<32>(precision, s, X, N, P, ys, n, nranges, rows_per_range, yscale, partial);
+                               unsigned nranges, unsigned long long rows_per_range, unsigned runs,
+                               float yscale, double* partial) {
+    if (d == 64)
+        return launch_d<64>(precision, s, X, N, P, ys, n, nranges, rows_per_range, runs, yscale,
+                            partial);
+    if (d == 32)
+        return launch_d<32>(precision, s, X, N, P, ys, n, nranges, rows_per_range, runs, yscale,
+                            partial);
     return hipErrorInvalidValue;
 }
 

@@ -25,7 +25,8 @@ unsigned glm_gauss_blocks_per_cu(int precision, unsigned D);
 // split of yscale*P (NS x n x d, MFMA kernels; fp16 terms for kGlmFp16x2).
 hipError_t launch_glm_logistic(int precision, hipStream_t s, const void* X, unsigned long long N,
                                unsigned d, const float* P, const void* ys, unsigned n,
-                               unsigned nranges, unsigned long long rows_per_range, float yscale,
+                               unsigned nranges, unsigned long long rows_per_range, unsigned runs,
+                               float yscale,
                                double* partial);
 // Issue-rate kernels (which = 0: v_exp_f32, 1: v_fma_f32, 8 x iters
 // operations per thread; 2: v_mfma_f32_16x16x32_f16, 8 x iters per wave),

@@ -1569,8 +1569,7 @@ __device__ __forceinline__ double bh_glm_logpost_sum(const float (&y)[DIM], doub
 
 // p[0] + p[stride] + ..., n values in this order.  The chain is one thread's
 // and each load some 0.7 us away, so the time is the number of rounds of
-// loads: 32 in flight, then 8 (a small logistic regression has 768 ranges, 96
-// per thread with 8 threads to a walker).
+// loads: 32 in flight, then 8, also for the last few.
 __device__ __forceinline__ double bh_strided_sum(const double* __restrict__ p, size_t stride,
                                                  unsigned n) {
     double s = 0.0;
@@ -1582,14 +1581,14 @@ __device__ __forceinline__ double bh_strided_sum(const double* __restrict__ p, s
 #pragma unroll
         for (int e = 0; e < 32; ++e) s += v[e];
     }
-    for (; r + 8 <= n; r += 8) {
+    for (; r < n; r += 8) {
+        // past the end the first of the eight again, not added
         double v[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = p[(size_t)(r + e) * stride];
+        for (unsigned e = 0; e < 8; ++e) v[e] = p[(size_t)(r + e < n ? r + e : r) * stride];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) s += v[e];
+        for (unsigned e = 0; e < 8; ++e) s = r + e < n ? s + v[e] : s;
     }
-    for (; r < n; ++r) s += p[(size_t)r * stride];
     return s;
 }
 
