@@ -1181,14 +1181,15 @@ int acor_device(bh_ctx* c, Call& call, std::vector<float>& h, float* d_series, u
     return BH_OK;
 }
 
-// Limits (when asked for) and counts of a matrix; d_limits and d_counts in
-// device memory.
+// Counts of a matrix, added to d_counts; with compute_limits its limits first,
+// and the counts from zero.  d_limits and d_counts in device memory.
 int histogram_device(bh_ctx* c, Call& call, const float* d_a, uint32_t m, uint64_t n,
                      uint32_t ld, float* d_limits, unsigned* d_counts, bool compute_limits) {
     if (compute_limits) {
         char* scratch;
         BH_TRY(call.dev(bh::dataset_scratch_bytes(m, n), &scratch));
-        BH_HIP(bh::launch_min_max(call.stream, d_a, m, n, ld, d_limits, scratch));
+        BH_HIP(bh::launch_min_max(call.stream, d_a, m, n, ld, d_limits, d_counts, c->wgs,
+                                  scratch));
     }
     BH_HIP(bh::launch_histogram(call.stream, d_a, m, n, ld, d_limits, c->wgs, d_counts));
     return BH_OK;
@@ -1224,8 +1225,8 @@ int batch_results(Call& call, const unsigned long long* acc, const double* s1, c
     return call.finish();
 }
 
-// A histogram call: counts cleared, `fill` (limits and counts), then pdf and
-// ranks of `total` values, and the results.
+// A histogram call: `fill` (limits, and counts from zero), then pdf and ranks
+// of `total` values, and the results.
 template <class F>
 int histogram_call(Call& call, uint32_t m, uint32_t bins, double total, float* limits,
                    float* pdf, float* bin_ranks, F&& fill) {
@@ -1236,7 +1237,6 @@ int histogram_call(Call& call, uint32_t m, uint32_t bins, double total, float* l
     BH_TRY(call.out(limits, (size_t)2 * m, &l));
     BH_TRY(call.out(pdf, (size_t)bins * m, &p));
     BH_TRY(call.out(bin_ranks, (size_t)bins * m, &r));
-    BH_HIP(hipMemsetAsync(counts, 0, (size_t)m * bins * sizeof(unsigned), call.stream));
     BH_TRY(fill(d_limits, counts));
     // alpha = WGS / n as the reference's float (amd_gcn.clj:206)
     const float alpha = (float)((double)bins / total);

@@ -36,8 +36,10 @@ hipError_t launch_uniform_sample(hipStream_t s, unsigned seed, float lo, float h
 hipError_t launch_direct_sample(hipStream_t s, int kind, unsigned seed, float p0, float p1,
                                 unsigned quads, float* x);
 size_t dataset_scratch_bytes(unsigned m, unsigned long long n);
+// limits of every row; clears its `bins` counters
 hipError_t launch_min_max(hipStream_t s, const float* a, unsigned m, unsigned long long n,
-                          unsigned ld, float* limits, void* scratch);
+                          unsigned ld, float* limits, unsigned* counts, unsigned bins,
+                          void* scratch);
 hipError_t launch_histogram(hipStream_t s, const float* a, unsigned m, unsigned long long n,
                             unsigned ld, const float* limits, unsigned bins, unsigned* counts);
 hipError_t launch_histogram_finalize(hipStream_t s, const unsigned* counts, const float* limits,
