@@ -2553,12 +2553,40 @@ bool gb_mfma(int prec) {
     return prec == BH_GLM_BF16 || prec == BH_GLM_BF16X3 || prec == BH_GLM_FP16X2;
 }
 
-// The contraction units of every problem: its rows in pieces of the tile's
-// unit rows of its stride class, the units of one stride in problem order,
-// global unit ids in problem order (ubeg[p] the first of problem p).
+// The rows of a contraction unit: the class's unit rows (whose runs of rows fix
+// the float sums), or a piece of them of whole 64-row runs where those make
+// fewer than 16 work-groups to a compute unit, the number of work-groups a
+// multiple of the compute units.  64 problems of 800,000 rows in all, 1024
+// points: 340 and 115 units x 4 groups for 1024 and 768 resident work-groups,
+// 129 + 63 us; in pieces of 192 to 576 rows 107 + 42, 12 half-steps
+// 2740 -> 2150.  Pieces below 256 rows wait for their points' fragments as
+// long as they work (192: no faster; 384: 13% slower where the rows are few).
+constexpr unsigned kGbMinPiece = 256, kGbCuWorkGroups = 16;
+unsigned gb_piece_rows(const bh_glm_batch* b, int cls) {
+    const unsigned ur = b->unit_rows[cls];
+    unsigned long long rows = 0;
+    for (uint32_t p = 0; p < b->P; ++p)
+        if ((b->dims_h[p] <= 32 ? 0 : 1) == cls) rows += b->rows_h[p];
+    // 256-point groups, also with 512 points to a work-group: the same units,
+    // and so the same sums, for both
+    const unsigned long long groups = std::max(b->K / 256u, 1u);
+    const unsigned long long work = rows * groups, cu = (unsigned long long)b->ctx->cu;
+    const unsigned long long each = std::clamp<unsigned long long>(
+        work / (kGbMinPiece * cu), 1, kGbCuWorkGroups);
+    const unsigned long long piece = (work / (each * cu) + 63) / 64 * 64;
+    return (unsigned)std::min<unsigned long long>(std::max<unsigned long long>(piece, kGbMinPiece),
+                                                  ur);
+}
+
+// The contraction units of every problem: its rows in runs of the tile's unit
+// rows of its stride class, a run in pieces (gb_piece_rows); the units of one
+// stride in problem order, global unit ids in problem order (ubeg[p] the first
+// of problem p).
 int gb_build_units(bh_glm_batch* b) {
     std::vector<uint32_t> u32, u64, ub(b->P + 1);
     uint32_t uid = 0;
+    unsigned piece[2];
+    for (int cls = 0; cls < 2; ++cls) piece[cls] = gb_piece_rows(b, cls);
     for (uint32_t p = 0; p < b->P; ++p) {
         const int cls = b->dims_h[p] <= 32 ? 0 : 1;
         const unsigned long long N = b->rows_h[p], ur = b->unit_rows[cls];
@@ -2566,7 +2594,13 @@ int gb_build_units(bh_glm_batch* b) {
         ub[p] = uid;
         for (unsigned long long r0 = 0; r0 < N; r0 += ur) {
             const unsigned long long r1 = std::min<unsigned long long>(N, r0 + ur);
-            dst.insert(dst.end(), {p, (uint32_t)r0, (uint32_t)r1, uid++});
+            // (the last piece takes what would be less than half of one)
+            for (unsigned long long q = r0; q < r1;) {
+                const bool more = r1 - q >= piece[cls] + piece[cls] / 2;
+                const unsigned long long e = more ? q + piece[cls] : r1;
+                dst.insert(dst.end(), {more ? p | bh::kGbMore : p, (uint32_t)q, (uint32_t)e, uid++});
+                q = e;
+            }
         }
     }
     ub[b->P] = uid;

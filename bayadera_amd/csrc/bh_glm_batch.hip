@@ -338,8 +338,9 @@ __device__ __forceinline__ bool gb_tile(unsigned nunits, unsigned groups, unsign
     return u < nunits;
 }
 
-// MFMA contraction of the units of one row stride D (units: {problem, r0,
-// r1, global unit}); partial[unit][point] as the single-posterior kernel
+// MFMA contraction of the units of one row stride D (units: {problem | kGbMore
+// for a piece that is not the last of its run of rows, r0, r1, global unit});
+// partial[unit][point] as the single-posterior kernel
 // (log2 units, |u|/2 + log2(1 + 2^-|u|) summed over the unit's rows).  Each
 // wave holds the B fragments of CB 16-point column blocks (a block of four
 // waves: 64 CB points); CB and the unit rows are the tile shape the batch's
@@ -354,7 +355,7 @@ gb_mfma_kernel(const unsigned char* __restrict__ X8, const unsigned long long* _
     unsigned ui, g;
     if (!gb_tile(nunits, groups, ui, g)) return;
     const uint4 unit = units[ui];
-    const unsigned p = unit.x;
+    const unsigned p = unit.x & ~kGbMore;
     const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const unsigned lr = lane & 15u, lg = lane >> 4;
     const unsigned w0 = g * (64u * CB) + wave * (16u * CB);
@@ -373,7 +374,7 @@ gb_mfma_kernel(const unsigned char* __restrict__ X8, const unsigned long long* _
     for (int wb = 0; wb < CB; ++wb) acc[wb] = 0.0;
     if (unit.y < unit.z)
         glm_mfma_rows<D, NS, CB>(Fp8Rows<D, V>{X8 + xoff[p], lr, lg}, bfrag, unit.y, unit.z, lg,
-                                 acc);
+                                 acc, unit.x & kGbMore);
 #pragma unroll
     for (int wb = 0; wb < CB; ++wb) {
         double v = acc[wb];
@@ -396,7 +397,7 @@ gb_fp32_kernel(const unsigned char* __restrict__ X8, const unsigned long long* _
     unsigned ui, g;
     if (!gb_tile(nunits, groups, ui, g)) return;
     const uint4 unit = units[ui];
-    const unsigned p = unit.x;
+    const unsigned p = unit.x & ~kGbMore;
     const unsigned k = g * 256u + threadIdx.x;
     float y[D];
 #pragma unroll
@@ -449,7 +450,7 @@ gb_fp64_kernel(const unsigned char* __restrict__ X8, const unsigned long long* _
     unsigned ui, g;
     if (!gb_tile(nunits, groups, ui, g)) return;
     const uint4 unit = units[ui];
-    const unsigned p = unit.x;
+    const unsigned p = unit.x & ~kGbMore;
     const unsigned k = g * 256u + threadIdx.x;
     double y[D];
 #pragma unroll
@@ -479,6 +480,30 @@ gb_fp64_kernel(const unsigned char* __restrict__ X8, const unsigned long long* _
     partial[(size_t)unit.w * n + k] = acc;
 }
 
+// partial[u * n] over the units ub .. ue in this order, 32 loads in flight
+// (one thread's chain: its time is the number of rounds of loads), the last
+// ones eight at a time with the first of the eight for those past the end.
+__device__ __forceinline__ double gb_unit_sum(const double* __restrict__ partial, unsigned n,
+                                              unsigned ub, unsigned ue) {
+    double s = 0.0;
+    unsigned u = ub;
+    for (; u + 32 <= ue; u += 32) {
+        double v[32];
+#pragma unroll
+        for (int e = 0; e < 32; ++e) v[e] = partial[(size_t)(u + e) * n];
+#pragma unroll
+        for (int e = 0; e < 32; ++e) s += v[e];
+    }
+    for (; u < ue; u += 8) {
+        double v[8];
+#pragma unroll
+        for (unsigned e = 0; e < 8; ++e) v[e] = partial[(size_t)(u + e < ue ? u + e : u) * n];
+#pragma unroll
+        for (unsigned e = 0; e < 8; ++e) s = u + e < ue ? s + v[e] : s;
+    }
+    return s;
+}
+
 // lp of point k of problem p from its units' partial sums (in unit order):
 // lin.y - scale * s - |y|^2 / (2 s0^2), in double.
 __device__ __forceinline__ double gb_logpost(const float* __restrict__ y, unsigned d,
@@ -486,18 +511,7 @@ __device__ __forceinline__ double gb_logpost(const float* __restrict__ y, unsign
                                              unsigned ue, unsigned n, unsigned k,
                                              const double* __restrict__ lin, double scale,
                                              double prior_prec) {
-    // the units' partial sums in unit order, loaded eight at a time so the
-    // loads are in flight together
-    double s = 0.0;
-    unsigned u = ub;
-    for (; u + 8 <= ue; u += 8) {
-        double v[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = partial[(size_t)(u + e) * n + k];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) s += v[e];
-    }
-    for (; u < ue; ++u) s += partial[(size_t)u * n + k];
+    const double s = gb_unit_sum(partial + k, n, ub, ue);
     double l = 0.0, q = 0.0;
     for (unsigned i = 0; i < d; ++i) {
         l = __builtin_fma(lin[i], (double)y[i], l);
@@ -558,18 +572,7 @@ __device__ __forceinline__ void gb_accept_one(int half, unsigned p, unsigned k, 
     if (threadIdx.x < D) lin_s[threadIdx.x] = lin[(size_t)p * kGbD + threadIdx.x];
     __syncthreads();
     const float4* y4 = reinterpret_cast<const float4*>(Y + ((size_t)p * K + k) * kGbD);
-    // lp(Y): the units' partial sums in unit order, eight loads in flight
-    double s = 0.0;
-    unsigned u = ubeg[p];
-    const unsigned ue = ubeg[p + 1];
-    for (; u + 8 <= ue; u += 8) {
-        double v[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = partial[(size_t)(u + e) * K + k];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) s += v[e];
-    }
-    for (; u < ue; ++u) s += partial[(size_t)u * K + k];
+    const double s = gb_unit_sum(partial + k, K, ubeg[p], ubeg[p + 1]);
     double l = 0.0, q = 0.0;
 #pragma unroll 4
     for (int c = 0; c < D / 4; ++c) {

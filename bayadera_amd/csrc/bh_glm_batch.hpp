@@ -11,6 +11,8 @@ namespace bh {
 // rows of one unit of the batched contraction (a multiple of 16) until the
 // batch's tile shapes are set or autotuned
 constexpr unsigned kGbUnitRows = 2048;
+// a unit's problem word: the rows go on in the next unit
+constexpr unsigned kGbMore = 0x80000000u;
 
 // f16 = 0: the fp32 path's decoding; 1: the fp16 matrix-core path's.
 hipError_t launch_gb_fp8_decode(hipStream_t s, const void* in, float* out, unsigned long long n,

@@ -183,11 +183,14 @@ __device__ __forceinline__ void glm_epilogue_second(const f32x4 (&c)[CB], double
 // (ld.full(rb, a): all 16 rows valid; ld.masked(rb, r1, a): rows >= r1 read
 // as zeros; Loader::vec is the operand type).  acc[wb] accumulates this
 // lane's four rows of column block wb.  CB = 4 (64 points per wave) or 8.
+// more: the range is a piece of a longer one, whole runs of four blocks, and
+// its last four are a run like the others.
 template <int D, int NS, int CB, class Loader>
 __device__ __forceinline__ void glm_mfma_rows(const Loader& ld,
                                               const typename Loader::vec (&bfrag)[CB][D / 32][NS],
                                               unsigned r0,
-                                              unsigned r1, unsigned lg, double (&acc)[CB]) {
+                                              unsigned r1, unsigned lg, double (&acc)[CB],
+                                              bool more = false) {
     constexpr int KC = D / 32;
     const unsigned rfull = r0 + (r1 - r0) / 16 * 16;
     f32x4 c0[CB], c1[CB];
@@ -217,6 +220,15 @@ __device__ __forceinline__ void glm_mfma_rows(const Loader& ld,
             glm_mfma_overlap<D, NS, 2, CB>(a1, bfrag, c1, c0, acc, st);
             ld.full(clamp(rb + 64), a1);
             glm_mfma_overlap<D, NS, 1, CB>(a0, bfrag, c0, c1, acc, st);
+        }
+        if (more) {
+            ld.full(clamp(rb + 16), a0);
+            glm_mfma_overlap<D, NS, 0, CB>(a1, bfrag, c1, c0, acc, st);
+            ld.full(clamp(rb + 32), a1);
+            glm_mfma_overlap<D, NS, 2, CB>(a0, bfrag, c0, c1, acc, st);
+            glm_mfma_overlap<D, NS, 2, CB>(a1, bfrag, c1, c0, acc, st);
+            glm_epilogue_second(c1, acc, st);
+            return;
         }
         // pairs of blocks (rb - 16, rb): the first's epilogue runs with the
         // products of rb, the second's with those of rb + 16
