@@ -211,7 +211,10 @@ __device__ __forceinline__ void glm_mfma_rows(const Loader& ld,
         GlmEpiState<CB> st;
         unsigned rb = r0 + 16;
         // runs of four blocks rb - 16 .. rb + 32 (products of rb .. rb + 48)
-        for (; rb + 48 < rfull; rb += 64) {
+        // (with `more` the last run too: the products beside its last epilogue
+        // are those of a block again, not used)
+        const unsigned rruns = more ? rfull + 16 : rfull;
+        for (; rb + 48 < rruns; rb += 64) {
             ld.full(clamp(rb + 16), a0);
             glm_mfma_overlap<D, NS, 0, CB>(a1, bfrag, c1, c0, acc, st);
             ld.full(clamp(rb + 32), a1);
@@ -220,15 +223,6 @@ __device__ __forceinline__ void glm_mfma_rows(const Loader& ld,
             glm_mfma_overlap<D, NS, 2, CB>(a1, bfrag, c1, c0, acc, st);
             ld.full(clamp(rb + 64), a1);
             glm_mfma_overlap<D, NS, 1, CB>(a0, bfrag, c0, c1, acc, st);
-        }
-        if (more) {
-            ld.full(clamp(rb + 16), a0);
-            glm_mfma_overlap<D, NS, 0, CB>(a1, bfrag, c1, c0, acc, st);
-            ld.full(clamp(rb + 32), a1);
-            glm_mfma_overlap<D, NS, 2, CB>(a0, bfrag, c0, c1, acc, st);
-            glm_mfma_overlap<D, NS, 2, CB>(a1, bfrag, c1, c0, acc, st);
-            glm_epilogue_second(c1, acc, st);
-            return;
         }
         // pairs of blocks (rb - 16, rb): the first's epilogue runs with the
         // products of rb, the second's with those of rb + 16
@@ -241,7 +235,7 @@ __device__ __forceinline__ void glm_mfma_rows(const Loader& ld,
         if (rb < rfull) {
             glm_mfma_overlap<D, NS, 0, CB>(a1, bfrag, c1, c0, acc, st);
             glm_epilogue_second(c1, acc, st);
-        } else {
+        } else if (!more) {
             glm_epilogue(c0, acc);
         }
     }
