@@ -996,7 +996,7 @@ int glm_alloc(bh_stretch* s, unsigned n_points, unsigned k_half) {
 
 // One bare half-step pair (move-bare!, amd_gcn.clj:347-353): odd half with
 // seed and constant 3333, even half with seed+1 and 4444 (:547-550).
-int bare_pair(bh_stretch* s, float beta) {
+int bare_pair(bh_stretch* s, float beta, float* out = nullptr) {
     if (s->f->glm) {
         BH_TRY(glm_half(s, true, s->bare_seed, 3333, s->bare_counter, s->bare_a, beta, 0, 0));
         return glm_half(s, false, s->bare_seed + 1u, 4444, s->bare_counter, s->bare_a, beta, 0, 0);
@@ -1013,8 +1013,10 @@ int bare_pair(bh_stretch* s, float beta) {
     unsigned seed0 = s->bare_seed, seed1 = s->bare_seed + 1u, c0 = 3333, c1 = 4444;
     const float* S1 = x1;
     const float* S0 = x0;
-    void* a0[] = {&seed0, &c0, &data_len, &params_len, &params, &S1, &x0, &l0, &a, &beta, &step, &K, &partner};
-    void* a1[] = {&seed1, &c1, &data_len, &params_len, &params, &S0, &x1, &l1, &a, &beta, &step, &K, &partner};
+    float* o0 = out;
+    float* o1 = out ? out + (size_t)s->K * s->dim : nullptr;
+    void* a0[] = {&seed0, &c0, &data_len, &params_len, &params, &S1, &x0, &l0, &a, &beta, &step, &K, &partner, &o0};
+    void* a1[] = {&seed1, &c1, &data_len, &params_len, &params, &S0, &x1, &l1, &a, &beta, &step, &K, &partner, &o1};
     const unsigned grid = s->K / s->wgs;
     BH_TRY(ktimed(s, [&] { return launch(s->f->bare, grid, s->wgs, 0, s->stream, a0); }));
     BH_TRY(ktimed(s, [&] { return launch(s->f->bare, grid, s->wgs, 0, s->stream, a1); }));
@@ -3218,11 +3220,16 @@ int bh_stretch_sample(bh_stretch* s, float* out, uint64_t ncols) {
     } else {
         uint64_t ofst = 0;
         for (uint64_t i = 0; i < steps; ++i) {
-            BH_TRY(bare_pair(s, 1.0f));
-            s->bare_counter += 1;
             const uint64_t chunk = std::min(avail, req - ofst);
-            BH_HIP(hipMemcpyAsync(o + ofst, s->xs.p, chunk * sizeof(float),
-                                  hipMemcpyDeviceToDevice, s->stream));
+            // a whole ensemble is written by its moves (in 16-byte pieces), a
+            // part of one copied
+            const bool by_moves = !s->f->glm && chunk == avail &&
+                                  reinterpret_cast<uintptr_t>(o + ofst) % 16 == 0;
+            BH_TRY(bare_pair(s, 1.0f, by_moves ? o + ofst : nullptr));
+            s->bare_counter += 1;
+            if (!by_moves)
+                BH_HIP(hipMemcpyAsync(o + ofst, s->xs.p, chunk * sizeof(float),
+                                      hipMemcpyDeviceToDevice, s->stream));
             ofst += chunk;
         }
     }

@@ -370,7 +370,8 @@ __device__ __forceinline__ void bh_stretch_half_staged(unsigned seed, unsigned o
                                                        float* __restrict__ logfn_X, float a,
                                                        float beta, unsigned step, unsigned K,
                                                        unsigned* __restrict__ accept,
-                                                       float* __restrict__ means) {
+                                                       float* __restrict__ means,
+                                                       float* __restrict__ out) {
     typedef float bh_f4 __attribute__((ext_vector_type(4)));
     constexpr int ST = kBhStageStride;
     constexpr bool V4 = DIM % 4 == 0;                     // records as 16-byte pieces
@@ -472,6 +473,9 @@ __device__ __forceinline__ void bh_stretch_half_staged(unsigned seed, unsigned o
             tile[t * ST + i] = y[i];
         }
         __builtin_nontemporal_store(ly, logfn_X + k);
+    } else if (out) {
+#pragma unroll
+        for (int i = 0; i < DIM; ++i) tile[t * ST + i] = xk[i];
     }
     const unsigned long long m = __ballot(accepted);
     if ((t & 63u) == 0) acc_mask[t >> 6] = m;
@@ -490,6 +494,20 @@ __device__ __forceinline__ void bh_stretch_half_staged(unsigned seed, unsigned o
             }
         }
     }
+    if (out) {
+        float* ob = out + (size_t)blockIdx.x * WGS * DIM;
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            const unsigned g = i * WGS + t, w = g / NP, c = g % NP;
+            if constexpr (V4) {
+                bh_f4* q = reinterpret_cast<bh_f4*>(__builtin_assume_aligned(ob, 16));
+                __builtin_nontemporal_store(*reinterpret_cast<const bh_f4*>(&tile[w * ST + 4 * c]),
+                                            q + g);
+            } else {
+                __builtin_nontemporal_store(tile[w * ST + c], ob + g);
+            }
+        }
+    }
     if (ACCU)
         bh_accu(xk, accepted, blockIdx.x, gridDim.x, step, accept, means, old, bh_accu_lds());
 }
@@ -502,10 +520,11 @@ __device__ __forceinline__ void bh_stretch_half(unsigned seed, unsigned odd_or_e
                                                 float* __restrict__ logfn_X, float a, float beta,
                                                 unsigned step, unsigned K,
                                                 unsigned* __restrict__ accept,
-                                                float* __restrict__ means) {
+                                                float* __restrict__ means,
+                                                float* __restrict__ out) {
     if constexpr (kBhStage) {
         bh_stretch_half_staged<ACCU, PARTNER>(seed, odd_or_even, data_len, params_len, params, S,
-                                              X, logfn_X, a, beta, step, K, accept, means);
+                                              X, logfn_X, a, beta, step, K, accept, means, out);
         return;
     } else {
         const unsigned k = blockIdx.x * WGS + threadIdx.x;
@@ -521,23 +540,28 @@ __device__ __forceinline__ void bh_stretch_half(unsigned seed, unsigned odd_or_e
             bh_store_walker_nt(xp, xk);
             __builtin_nontemporal_store(lx, logfn_X + k);
         }
+        if (out) bh_store_walker_nt(out + (size_t)k * DIM, xk);
         if (ACCU)
             bh_accu(xk, accepted, blockIdx.x, gridDim.x, step, accept, means, old, bh_accu_lds());
     }
 }
 
+// With `out` the half's records after the move go there too: a sample of an
+// ensemble is written by its last step instead of being copied from it (2^21
+// x 16 walkers a half: the copy read and wrote 2 x 134 MB, 100 us for both
+// halves; writing alone 43).
 extern "C" __global__ void __launch_bounds__(WGS)
 bh_stretch_move_bare(unsigned seed, unsigned odd_or_even, unsigned data_len, unsigned params_len,
                      const float* __restrict__ params, const float* __restrict__ S,
                      float* __restrict__ X, float* __restrict__ logfn_X, float a, float beta,
-                     unsigned step, unsigned K, int partner) {
+                     unsigned step, unsigned K, int partner, float* __restrict__ out) {
     if (partner == BH_PARTNER_FLAT)
         bh_stretch_half<false, BH_PARTNER_FLAT>(seed, odd_or_even, data_len, params_len, params, S,
-                                                X, logfn_X, a, beta, step, K, nullptr, nullptr);
+                                                X, logfn_X, a, beta, step, K, nullptr, nullptr, out);
     else
         bh_stretch_half<false, BH_PARTNER_WALKER>(seed, odd_or_even, data_len, params_len, params,
                                                   S, X, logfn_X, a, beta, step, K, nullptr,
-                                                  nullptr);
+                                                  nullptr, out);
 }
 
 extern "C" __global__ void __launch_bounds__(WGS)
@@ -549,10 +573,10 @@ bh_stretch_move_accu(unsigned seed, unsigned odd_or_even, unsigned data_len,
                      int partner) {
     if (partner == BH_PARTNER_FLAT)
         bh_stretch_half<true, BH_PARTNER_FLAT>(seed, odd_or_even, data_len, params_len, params, S,
-                                               X, logfn_X, a, 1.0f, step, K, accept, means);
+                                               X, logfn_X, a, 1.0f, step, K, accept, means, nullptr);
     else
         bh_stretch_half<true, BH_PARTNER_WALKER>(seed, odd_or_even, data_len, params_len, params,
-                                                 S, X, logfn_X, a, 1.0f, step, K, accept, means);
+                                                 S, X, logfn_X, a, 1.0f, step, K, accept, means, nullptr);
 }
 
 #endif  // !BH_RESIDENT && !BH_BATCH
