@@ -87,6 +87,11 @@ struct DevBuf {
         bytes = n;
         return BH_OK;
     }
+    void drop() {
+        if (p) (void)hipFree(p);
+        p = nullptr;
+        bytes = 0;
+    }
     template <class T>
     T* as() const {
         return static_cast<T*>(p);
@@ -414,7 +419,7 @@ struct bh_stretch_factory {
     bh_ctx* ctx = nullptr;
     uint32_t dim = 0, params_len = 0;
     Module mod;
-    hipFunction_t logfn = nullptr, bare = nullptr, accu = nullptr;
+    hipFunction_t logfn = nullptr, bare = nullptr, accu = nullptr, found = nullptr;
     // the resident steps' kernels, compiled for the first sampler that takes them
     std::string source, logfn_name;
     std::mutex resident_mu;
@@ -461,6 +466,7 @@ struct bh_stretch {
     uint32_t dim = 0, W = 0, K = 0, wgs = 0, groups = 0;
     uint32_t params_count = 0, data_len = 0, params_len = 0;
     DevBuf xs, logfn, params, accept, means_acc;
+    DevBuf fentries, fpos, fstarts, fg;  // partners found beforehand (see found_alloc)
     DevBuf rdraws, rtrace, rsink;  // a chunk of resident steps' draws and positions
     uint64_t means_cap = 0;
     uint32_t bare_seed = 0, move_seed = 0, bare_counter = 0, move_counter = 0;
@@ -994,6 +1000,38 @@ int glm_alloc(bh_stretch* s, unsigned n_points, unsigned k_half) {
     return BH_OK;
 }
 
+// Whether a sampler's half-steps look their partners up beforehand
+// (partner_sort_kernel), and its buffers for that: 12 + 4 dim bytes for each
+// walker of a half, made with the sampler.  Where the memory is short the moves
+// read their partners themselves, as any other ensemble's.  A half-step, us,
+// direct against sort (half a step's) + read + move:
+//   dim 1, halves of 2^21   27    11 + 14 + 12     2^22   64   15 + 17 + 19
+//                    2^23  149    22 + 32 + 34     2^24  323   43 + 84 + 63
+//   dim 2, halves of 2^21   38    15 + 11 + 21     2^22   81   16 + 22 + 23
+//                    2^24  351    43 + 189 + 92
+// so the line is 2^22 walkers; past 2^25 floats a tile has less than a sector
+// of entries in a region.
+constexpr uint32_t kFoundMin = 1u << 22;
+constexpr unsigned kFoundThreads = 1024;  // of bh_stretch_move_found
+bh::PartnerPlan found_plan(const bh_stretch* s) {
+    return bh::PartnerPlan{s->K, s->dim, s->fentries.as<unsigned>(), s->fpos.as<unsigned short>(),
+                           s->fstarts.as<unsigned>(), s->fg.as<float>()};
+}
+
+void found_alloc(bh_stretch* s) {
+    if (s->f->glm || s->dim > bh::kPartnerMaxDim || s->K < kFoundMin) return;
+    const bh::PartnerPlan p = found_plan(s);
+    const size_t K = s->K, starts = (size_t)p.tiles() * (p.regions() + 1);
+    if (p.regions() > bh::kPartnerRegions) return;
+    if (s->fentries.alloc(2 * K * sizeof(unsigned)) != BH_OK ||
+        s->fpos.alloc(2 * K * sizeof(unsigned short)) != BH_OK ||
+        s->fstarts.alloc(2 * starts * sizeof(unsigned)) != BH_OK ||
+        s->fg.alloc(K * s->dim * sizeof(float)) != BH_OK) {
+        (void)hipGetLastError();
+        for (DevBuf* b : {&s->fentries, &s->fpos, &s->fstarts, &s->fg}) b->drop();
+    }
+}
+
 // One bare half-step pair (move-bare!, amd_gcn.clj:347-353): odd half with
 // seed and constant 3333, even half with seed+1 and 4444 (:547-550).
 int bare_pair(bh_stretch* s, float beta, float* out = nullptr) {
@@ -1018,6 +1056,24 @@ int bare_pair(bh_stretch* s, float beta, float* out = nullptr) {
     void* a0[] = {&seed0, &c0, &data_len, &params_len, &params, &S1, &x0, &l0, &a, &beta, &step, &K, &partner, &o0};
     void* a1[] = {&seed1, &c1, &data_len, &params_len, &params, &S0, &x1, &l1, &a, &beta, &step, &K, &partner, &o1};
     const unsigned grid = s->K / s->wgs;
+    if (s->fg.p) {
+        const bh::PartnerPlan p = found_plan(s);
+        const float* found = p.g;
+        const unsigned short *pos0 = p.pos, *pos1 = p.pos + K;
+        void* f0[] = {&seed0, &c0, &data_len, &params_len, &params, &found, &pos0, &x0, &l0, &a, &beta, &step, &K, &o0};
+        void* f1[] = {&seed1, &c1, &data_len, &params_len, &params, &found, &pos1, &x1, &l1, &a, &beta, &step, &K, &o1};
+        BH_TRY(ktimed(s, [&]() -> int {
+            const unsigned seeds[2] = {seed0, seed1}, consts[2] = {c0, c1};
+            BH_HIP(bh::launch_partner_sort(s->stream, p, partner == BH_PARTNER_WALKER, seeds, consts,
+                                           step));
+            BH_HIP(bh::launch_partner_read(s->stream, p, 0, S1));
+            return launch(s->f->found, p.tiles(), kFoundThreads, 0, s->stream, f0);
+        }));
+        return ktimed(s, [&]() -> int {
+            BH_HIP(bh::launch_partner_read(s->stream, p, 1, S0));
+            return launch(s->f->found, p.tiles(), kFoundThreads, 0, s->stream, f1);
+        });
+    }
     BH_TRY(ktimed(s, [&] { return launch(s->f->bare, grid, s->wgs, 0, s->stream, a0); }));
     BH_TRY(ktimed(s, [&] { return launch(s->f->bare, grid, s->wgs, 0, s->stream, a1); }));
     return BH_OK;
@@ -1770,6 +1826,7 @@ int bh_stretch_factory_create(bh_ctx* ctx, const char* source, const char* logfn
     BH_TRY(f->mod.fn("bh_logfn", &f->logfn));
     BH_TRY(f->mod.fn("bh_stretch_move_bare", &f->bare));
     BH_TRY(f->mod.fn("bh_stretch_move_accu", &f->accu));
+    if (dim <= bh::kPartnerMaxDim) BH_TRY(f->mod.fn("bh_stretch_move_found", &f->found));
     f->source = source;
     f->logfn_name = logfn_name;
     *out = f.release();
@@ -1956,6 +2013,7 @@ int bh_stretch_create(bh_stretch_factory* f, uint32_t seed, uint32_t walkers,
     BH_TRY(s->xs.alloc((size_t)walkers * f->dim * sizeof(float)));
     BH_TRY(s->logfn.alloc((size_t)walkers * sizeof(float)));
     BH_TRY(s->params.alloc((size_t)std::max(params_count, 1u) * sizeof(float)));
+    found_alloc(s.get());
     BH_HIP(hipMemsetAsync(s->xs.p, 0, (size_t)walkers * f->dim * sizeof(float), s->stream));
     BH_HIP(hipMemsetAsync(s->logfn.p, 0, (size_t)walkers * sizeof(float), s->stream));
     if (params_count)

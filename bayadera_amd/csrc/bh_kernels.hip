@@ -1082,6 +1082,143 @@ copy16_kernel(const bh_copy_f4* __restrict__ src, bh_copy_f4* __restrict__ dst,
 }
 
 // --------------------------------------------------------------------------
+// Partners of a half-step found beforehand
+// --------------------------------------------------------------------------
+// A half-step of a large ensemble of small records is bound by its partners:
+// each is a line from memory (5.2e10 a second) for 4 or 8 bytes of it.  They
+// are sorted by region first, and read from LDS.
+//
+// Sorting: a work-group takes a tile's draws (the Philox words of the move, of
+// which only the partner's counts here), counts them by region in LDS and puts
+// each partner's first element at its place.  The order inside a region is
+// whatever the counters gave; nothing depends on it.  Draws don't depend on
+// positions, so one launch sorts for both half-steps of a step: 2 x 2^23 draws
+// in 43 us against 27 for 2^23.
+constexpr unsigned kPartnerThreads = 1024;
+__global__ void __launch_bounds__(kPartnerThreads)
+    partner_sort_kernel(unsigned K, unsigned dim, int partner_walker, uint2 seeds, uint2 odd_even,
+                        unsigned step, unsigned bits, unsigned regions,
+                        unsigned* __restrict__ entries, unsigned short* __restrict__ pos,
+                        unsigned* __restrict__ starts) {
+    const unsigned seed = blockIdx.y ? seeds.y : seeds.x;
+    const unsigned odd_or_even = blockIdx.y ? odd_even.y : odd_even.x;
+    entries += (size_t)blockIdx.y * K;
+    pos += (size_t)blockIdx.y * K;
+    starts += (size_t)blockIdx.y * gridDim.x * (regions + 1);
+    constexpr unsigned N = kPartnerTile / kPartnerThreads;
+    static_assert(kPartnerRegions == kPartnerThreads, "a thread per region");
+    __shared__ unsigned count[kPartnerRegions], first[kPartnerRegions], waves[kPartnerThreads / 64];
+    __shared__ unsigned sorted[kPartnerTile];
+    const unsigned t = threadIdx.x, tile = blockIdx.x * kPartnerTile;
+    const unsigned n = K - tile < kPartnerTile ? K - tile : kPartnerTile;
+    count[t] = 0;
+    __syncthreads();
+    unsigned e[N], rank[N];
+#pragma unroll
+    for (unsigned i = 0; i < N; ++i) {
+        const unsigned w = i * kPartnerThreads + t;
+        const bh_u32x4 r = bh_philox4x32_10(bh_u32x4{tile + w, step, odd_or_even, BH_CTR3}, seed,
+                                            BH_KEY1_STRETCH);
+        const float u = bh_u01(r.x);
+        if (partner_walker) {
+            unsigned j = (unsigned)(u * (float)K);
+            j = j < K ? j : K - 1;
+            e[i] = j * dim;
+        } else {
+            e[i] = (unsigned)((u * (float)K) * (float)dim);
+            if (e[i] >= K * dim) e[i] -= K * dim;
+        }
+        if (w < n) rank[i] = atomicAdd(&count[e[i] >> bits], 1u);
+    }
+    __syncthreads();
+    const unsigned own = count[t];
+    unsigned s = own;
+#pragma unroll
+    for (unsigned i = 1; i < 64; i *= 2) {
+        const unsigned v = __shfl_up(s, i);
+        if ((t & 63u) >= i) s += v;
+    }
+    if ((t & 63u) == 63u) waves[t >> 6] = s;
+    __syncthreads();
+    for (unsigned w = 0; w < (t >> 6); ++w) s += waves[w];
+    first[t] = s - own;
+    const unsigned tiles = gridDim.x;
+    if (t < regions) starts[(size_t)t * tiles + blockIdx.x] = s - own;
+    if (t == 0) starts[(size_t)regions * tiles + blockIdx.x] = n;
+    __syncthreads();
+#pragma unroll
+    for (unsigned i = 0; i < N; ++i) {
+        const unsigned w = i * kPartnerThreads + t;
+        if (w < n) {
+            const unsigned at = first[e[i] >> bits] + rank[i];
+            sorted[at] = e[i];
+            pos[tile + w] = (unsigned short)at;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (unsigned i = 0; i < N; ++i) {
+        const unsigned w = i * kPartnerThreads + t;
+        if (w < n) entries[tile + w] = sorted[w];
+    }
+}
+
+// Reading: a work-group's region of S lies in LDS (and the floats that a record
+// starting at its end runs on to); `lanes` lanes take a tile's entries of it,
+// and four tiles at a time so that the loads of eight groups of entries are in
+// flight.
+template <unsigned DIM>
+__global__ void __launch_bounds__(kPartnerThreads)
+    partner_read_kernel(const unsigned* __restrict__ entries, const unsigned* __restrict__ starts,
+                        unsigned bits, unsigned lanes, unsigned tiles,
+                        const float* __restrict__ S, unsigned total, float* __restrict__ g) {
+    constexpr unsigned NS = 4, NU = 2;
+    extern __shared__ __attribute__((aligned(16))) float region[];
+    const unsigned t = threadIdx.x, r0 = blockIdx.x << bits;
+    const unsigned n = total - r0 < (1u << bits) ? total - r0 : 1u << bits;
+    // total is a multiple of 4 (K is one of 64), and so is n
+    for (unsigned i = t * 4; i < n; i += kPartnerThreads * 4)
+        *reinterpret_cast<float4*>(region + i) = *reinterpret_cast<const float4*>(S + r0 + i);
+    if (t < DIM - 1) region[n + t] = S[r0 + n == total ? t : r0 + n + t];
+    const unsigned* row = starts + (size_t)blockIdx.x * tiles;
+    const unsigned lane = t & (lanes - 1), groups = kPartnerThreads / lanes;
+    __syncthreads();
+    for (unsigned t0 = t / lanes; t0 < tiles; t0 += NS * groups) {
+        unsigned at[NS], end[NS], longest = 0;
+#pragma unroll
+        for (unsigned c = 0; c < NS; ++c) {
+            const unsigned tile = t0 + c * groups;
+            const bool has = tile < tiles;
+            const unsigned lo = has ? row[tile] : 0, hi = has ? row[tiles + tile] : 0;
+            at[c] = tile * kPartnerTile + lo;
+            end[c] = tile * kPartnerTile + hi;
+            longest = longest > hi - lo ? longest : hi - lo;
+        }
+        for (unsigned i0 = lane; i0 < longest; i0 += lanes * NU) {
+            unsigned e[NS][NU];
+#pragma unroll
+            for (unsigned c = 0; c < NS; ++c)
+#pragma unroll
+                for (unsigned j = 0; j < NU; ++j) {
+                    const unsigned i = at[c] + i0 + lanes * j;
+                    e[c][j] = i < end[c] ? entries[i] : r0;
+                }
+#pragma unroll
+            for (unsigned c = 0; c < NS; ++c)
+#pragma unroll
+                for (unsigned j = 0; j < NU; ++j) {
+                    const unsigned i = at[c] + i0 + lanes * j;
+                    if (i < end[c])
+#pragma unroll
+                        for (unsigned d = 0; d < DIM; ++d)
+                            __builtin_nontemporal_store(region[e[c][j] - r0 + d],
+                                                        g + (size_t)i * DIM + d);
+                }
+        }
+    }
+}
+
+// --------------------------------------------------------------------------
 // Host-side launchers (all on the caller's stream)
 // --------------------------------------------------------------------------
 static unsigned tile_rows(unsigned m) {
@@ -1108,6 +1245,33 @@ hipError_t launch_copy16(hipStream_t s, const void* src, void* dst, unsigned lon
     else
         copy16_kernel<false><<<(unsigned)blocks, 256, 0, s>>>(
             static_cast<const bh_copy_f4*>(src), static_cast<bh_copy_f4*>(dst), n16);
+    return hipGetLastError();
+}
+
+hipError_t launch_partner_sort(hipStream_t s, const PartnerPlan& p, int partner_walker,
+                               const unsigned seeds[2], const unsigned odd_even[2],
+                               unsigned step) {
+    partner_sort_kernel<<<dim3(p.tiles(), 2), kPartnerThreads, 0, s>>>(
+        p.K, p.dim, partner_walker, make_uint2(seeds[0], seeds[1]),
+        make_uint2(odd_even[0], odd_even[1]), step, p.bits(), p.regions(), p.entries, p.pos,
+        p.starts);
+    return hipGetLastError();
+}
+
+hipError_t launch_partner_read(hipStream_t s, const PartnerPlan& p, int half, const float* S) {
+    const unsigned regions = p.regions(), tiles = p.tiles();
+    // twice the lanes cover a tile's entries of a region but for rare ones
+    unsigned lanes = 64;
+    while (lanes > 8 && lanes * regions > kPartnerTile) lanes /= 2;
+    const unsigned* entries = p.entries + (size_t)half * p.K;
+    const unsigned* starts = p.starts + (size_t)half * tiles * (regions + 1);
+    const size_t lds = ((size_t)4 << p.bits()) + 16;
+    if (p.dim == 1)
+        partner_read_kernel<1><<<regions, kPartnerThreads, lds, s>>>(entries, starts, p.bits(), lanes,
+                                                                     tiles, S, p.K, p.g);
+    else
+        partner_read_kernel<2><<<regions, kPartnerThreads, lds, s>>>(entries, starts, p.bits(), lanes,
+                                                                     tiles, S, 2 * p.K, p.g);
     return hipGetLastError();
 }
 

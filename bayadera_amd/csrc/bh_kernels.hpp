@@ -29,6 +29,33 @@ hipError_t noalloc_scratch(int device, void** ptr);
 // dst[i] = src[i] for n16 16-byte pieces (nt: non-temporal loads and stores)
 hipError_t launch_copy16(hipStream_t s, const void* src, void* dst, unsigned long long n16,
                          bool nt);
+// The partners of a step found beforehand, for halves S (K walkers of dim floats)
+// past what the L2s hold: tiles of kPartnerTile walkers are sorted by the region
+// of S their partner starts in (for both half-steps at once), a work-group with
+// a region in LDS writes all tiles' partners from it in that order, and the move
+// of a tile finds walker k's at its pos[k].
+constexpr unsigned kPartnerTile = 8192;
+constexpr unsigned kPartnerRegions = 1024;  // at most
+constexpr unsigned kPartnerMaxDim = 2;
+struct PartnerPlan {
+    unsigned K, dim;
+    unsigned* entries;    // [2][K] the tiles' partners' first elements, by region
+    unsigned short* pos;  // [2][K] a walker's place in its tile's entries
+    unsigned* starts;     // [2][regions + 1][tiles] a region's first entry in a tile
+    float* g;             // [K][dim] the partners' records, in the order of entries
+
+    unsigned long long floats() const { return (unsigned long long)K * dim; }
+    unsigned tiles() const { return (K + kPartnerTile - 1) / kPartnerTile; }
+    // floats of a region: 64 KiB, two work-groups to a compute unit, while that
+    // makes 256 of them and a tile's entries of one a line; then 128 KiB (2^23
+    // floats: 32 us to read against 43)
+    unsigned bits() const { return floats() <= (1ull << 22) ? 14 : 15; }
+    unsigned regions() const { return (unsigned)((floats() + (1ull << bits()) - 1) >> bits()); }
+};
+hipError_t launch_partner_sort(hipStream_t s, const PartnerPlan& p, int partner_walker,
+                               const unsigned seeds[2], const unsigned odd_even[2], unsigned step);
+// of half-step `half`, from the half S
+hipError_t launch_partner_read(hipStream_t s, const PartnerPlan& p, int half, const float* S);
 hipError_t launch_init_walkers(hipStream_t s, unsigned seed, const float* limits, unsigned dim,
                                unsigned walkers, float* xs);
 hipError_t launch_uniform_sample(hipStream_t s, unsigned seed, float lo, float hi, unsigned quads,

@@ -252,6 +252,21 @@ __device__ __forceinline__ void bh_accu(const float (&xk)[DIM], bool accepted, u
 
 #ifdef LOGFN
 
+// The accept test of a proposal (:66-76).
+__device__ __forceinline__ bool bh_accept(const float (&y)[DIM], float z, float u2, float beta,
+                                          float (&xk)[DIM], float& lx, unsigned data_len,
+                                          unsigned params_len, const float* params) {
+    const float ly = LOGFN(data_len, params_len, params, DIM, y);
+    const float q = __builtin_isfinite(ly) ? bh_zpow(z) * expf(beta * (ly - lx)) : 0.0f;
+    const bool accepted = u2 <= q;
+    if (accepted) {
+#pragma unroll
+        for (int i = 0; i < DIM; ++i) xk[i] = y[i];
+        lx = ly;
+    }
+    return accepted;
+}
+
 // One walker's stretch move (amd-gcn-mcmc-stretch.cl:31-81).
 //   counter {k, step, odd_or_even, 0xbeeff00d}, key {seed, 0xdecafbad}
 //   z  = fma((a-2+1/a)*u1, u1, (2(1-1/a))*u1) + 1/a                     (:53-54)
@@ -271,15 +286,7 @@ __device__ __forceinline__ bool bh_stretch_walker(unsigned k, unsigned K, unsign
     float y[DIM];
     float z;
     const float u2 = bh_propose<PARTNER>(k, K, seed, odd_or_even, step, a, S, xk, y, z);
-    const float ly = LOGFN(data_len, params_len, params, DIM, y);
-    const float q = __builtin_isfinite(ly) ? bh_zpow(z) * expf(beta * (ly - lx)) : 0.0f;
-    const bool accepted = u2 <= q;
-    if (accepted) {
-#pragma unroll
-        for (int i = 0; i < DIM; ++i) xk[i] = y[i];
-        lx = ly;
-    }
-    return accepted;
+    return bh_accept(y, z, u2, beta, xk, lx, data_len, params_len, params);
 }
 
 // The modules of a model: its per-half-step kernels, and on their own (a user's
@@ -580,6 +587,66 @@ bh_stretch_move_accu(unsigned seed, unsigned odd_or_even, unsigned data_len,
         bh_stretch_half<true, BH_PARTNER_WALKER>(seed, odd_or_even, data_len, params_len, params,
                                                  S, X, logfn_X, a, 1.0f, step, K, accept, means, nullptr);
 }
+
+#if DIM <= 2
+// A half-step whose partners were found beforehand (see partner_sort_kernel in
+// bh_kernels.hip): a work-group takes a tile of kBhFoundTile walkers, puts the
+// tile's partners in LDS as they come (found) and reads walker k's at pos[k].
+// Its arithmetic is bh_stretch_move_bare's.  Bound by its traffic: 34 us for 2^23
+// walkers of one coordinate, 185 MB, 5.4 TB/s; reading the partners from memory
+// by pos takes 42 to 60, a line's lookup in the L2 each.  Tiles of 16384 take 36,
+// and leave records of two coordinates one work-group to a compute unit.
+constexpr unsigned kBhFoundTile = 8192, kBhFoundThreads = 1024;
+extern "C" __global__ void __launch_bounds__(kBhFoundThreads)
+bh_stretch_move_found(unsigned seed, unsigned odd_or_even, unsigned data_len, unsigned params_len,
+                      const float* __restrict__ params, const float* __restrict__ found,
+                      const unsigned short* __restrict__ pos, float* __restrict__ X,
+                      float* __restrict__ logfn_X, float a, float beta, unsigned step, unsigned K,
+                      float* __restrict__ out) {
+    __shared__ __attribute__((aligned(16))) float partners[kBhFoundTile * DIM];
+    const unsigned t = threadIdx.x, tile = blockIdx.x * kBhFoundTile;
+    const unsigned n = K - tile < kBhFoundTile ? K - tile : kBhFoundTile;
+    // the next walker's record, log density and place are read ahead
+    float nx[DIM], nl = 0.0f;
+    unsigned np = 0;
+    const auto load = [&](unsigned w) {
+        if (w < n) {
+            const unsigned k = tile + w;
+            bh_load_walker_nt(X + (size_t)k * DIM, nx);
+            nl = __builtin_nontemporal_load(logfn_X + k);
+            np = __builtin_nontemporal_load(pos + k);
+        }
+    };
+    load(t);
+    {
+        typedef float bh_f4 __attribute__((ext_vector_type(4)));
+        const bh_f4* q = reinterpret_cast<const bh_f4*>(found + (size_t)tile * DIM);
+        for (unsigned i = t; i < n * DIM / 4; i += kBhFoundThreads)
+            reinterpret_cast<bh_f4*>(partners)[i] = __builtin_nontemporal_load(q + i);
+    }
+    __syncthreads();
+    for (unsigned w = t; w < n; w += kBhFoundThreads) {
+        const unsigned k = tile + w;
+        float xk[DIM], lx = nl, y[DIM], z;
+        const unsigned p = np;
+#pragma unroll
+        for (int i = 0; i < DIM; ++i) xk[i] = nx[i];
+        load(w + kBhFoundThreads);
+        unsigned e;
+        const float u2 =
+            bh_stretch_draw<BH_PARTNER_WALKER>(k, K, seed, odd_or_even, step, a, z, e);
+#pragma unroll
+        for (int i = 0; i < DIM; ++i) {
+            const float xj = partners[p * DIM + i];
+            y[i] = __builtin_fmaf(z, xk[i] - xj, xj);
+        }
+        bh_accept(y, z, u2, beta, xk, lx, data_len, params_len, params);
+        bh_store_walker_nt(X + (size_t)k * DIM, xk);
+        __builtin_nontemporal_store(lx, logfn_X + k);
+        if (out) bh_store_walker_nt(out + (size_t)k * DIM, xk);
+    }
+}
+#endif
 
 #endif  // !BH_RESIDENT && !BH_BATCH
 
