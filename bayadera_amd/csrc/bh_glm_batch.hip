@@ -141,7 +141,7 @@ gb_init_kernel(unsigned seed, const unsigned* __restrict__ dims,
     }
 }
 
-// Writes r * t (t = log2(e) * column scale) as fp32 and as nsplit 16-bit
+// Writes r * t (t = log2(e) * column scale) as fp32 (nsplit 0) or as nsplit 16-bit
 // terms (bf16; or fp16 of r * t * 2^8 when f16 is set; hi, mid, lo), for
 // point k of problem p: the first D of its 64 slots (D = 32 or 64, the
 // problem's row stride, all that the contraction kernels read; slots from
@@ -154,9 +154,11 @@ __device__ __forceinline__ void gb_store_point(float (&r)[D], const float* __res
                                                void* __restrict__ ysplit, int nsplit, int f16) {
 #pragma unroll
     for (int i = 0; i < D; ++i) r[i] = (unsigned)i < d ? r[i] * t[i] : 0.0f;
-    float4* o = reinterpret_cast<float4*>(ysc + ((size_t)p * n + k) * kGbD);
+    if (nsplit == 0) {
+        float4* o = reinterpret_cast<float4*>(ysc + ((size_t)p * n + k) * kGbD);
 #pragma unroll
-    for (int c = 0; c < D / 4; ++c) o[c] = make_float4(r[4 * c], r[4 * c + 1], r[4 * c + 2], r[4 * c + 3]);
+        for (int c = 0; c < D / 4; ++c) o[c] = make_float4(r[4 * c], r[4 * c + 1], r[4 * c + 2], r[4 * c + 3]);
+    }
     if (f16) {
 #pragma unroll
         for (int i = 0; i < D; ++i) r[i] *= kGbF16Up;
@@ -221,7 +223,9 @@ gb_points_kernel(const float* __restrict__ xs, const unsigned* __restrict__ dims
         gb_points_one<64>(x, t, d, P, p, n, k, ysc, ysplit, nsplit, f16);
 }
 
-// The proposals of a block's 256 walkers from their partners (indices jl,
+constexpr unsigned kGbProposeWalkers = 64;  // of a block
+
+// The proposals of a block's walkers from their partners (indices jl,
 // stretch factors zl), one 16-byte piece per thread: D/4 consecutive threads
 // take one walker's record, so the block reads and writes its records, and
 // each partner's, as consecutive pieces: Y = fma(z, X - S, S) (zero beyond
@@ -238,15 +242,22 @@ __device__ __forceinline__ void gb_propose_pieces(const float* __restrict__ X,
                                                   int f16) {
     typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
     typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-    constexpr unsigned T = D / 4, WP = 256 / T;
+    constexpr unsigned T = D / 4, WP = 256 / T, N = kGbProposeWalkers / WP;
     const unsigned c = threadIdx.x % T;
     const float4 tv = reinterpret_cast<const float4*>(t)[c];
     const float ta[4] = {tv.x, tv.y, tv.z, tv.w};
-    for (unsigned it = 0; it < T; ++it) {
+    float4 xs[N], ss[N];
+#pragma unroll
+    for (unsigned it = 0; it < N; ++it) {
+        const unsigned w = it * WP + threadIdx.x / T;
+        xs[it] = reinterpret_cast<const float4*>(X + (size_t)(kb + w) * kGbD)[c];
+        ss[it] = reinterpret_cast<const float4*>(S + (size_t)jl[w] * kGbD)[c];
+    }
+#pragma unroll
+    for (unsigned it = 0; it < N; ++it) {
         const unsigned w = it * WP + threadIdx.x / T;
         const unsigned k = kb + w;
-        const float4 xv = reinterpret_cast<const float4*>(X + (size_t)k * kGbD)[c];
-        const float4 sv = reinterpret_cast<const float4*>(S + (size_t)jl[w] * kGbD)[c];
+        const float4 xv = xs[it], sv = ss[it];
         const float z = zl[w];
         const float xa[4] = {xv.x, xv.y, xv.z, xv.w};
         const float sa[4] = {sv.x, sv.y, sv.z, sv.w};
@@ -259,7 +270,8 @@ __device__ __forceinline__ void gb_propose_pieces(const float* __restrict__ X,
         }
         const size_t row = ((size_t)p * K + k) * kGbD;
         reinterpret_cast<float4*>(Y + row)[c] = make_float4(y[0], y[1], y[2], y[3]);
-        reinterpret_cast<float4*>(ysc + row)[c] = make_float4(r[0], r[1], r[2], r[3]);
+        if (nsplit == 0)
+            reinterpret_cast<float4*>(ysc + row)[c] = make_float4(r[0], r[1], r[2], r[3]);
         if (f16) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) r[e] *= kGbF16Up;
@@ -291,34 +303,40 @@ __device__ __forceinline__ void gb_propose_pieces(const float* __restrict__ X,
 // amd-gcn-mcmc-stretch.cl:31-65 with whole-walker partners): problem p uses
 // seed seed0 + 2p (+1 for the second half) and counter word `oe`.  Each
 // thread draws one walker's uniforms; the records are then built piece by
-// piece (gb_propose_pieces).
+// piece (gb_propose_pieces).  A block takes 64 walkers, so that a thread has its
+// two or four pieces in flight at once and small batches fill the device: 64
+// problems of 1024 points of 8 to 64 dimensions 13.6 us with 256 walkers a
+// block, 9.9 with 64, and 8.5 without the scaled points in fp32, which only the
+// fp32 contraction reads (ysc).
 __global__ void __launch_bounds__(256)
 gb_propose_kernel(unsigned seed0, int half, unsigned oe, unsigned step, float a,
                   const unsigned* __restrict__ dims, const float* __restrict__ tscale,
                   const float* __restrict__ xs, unsigned P, unsigned K, float* __restrict__ Y,
                   float* __restrict__ zbuf, float* __restrict__ u2buf, float* __restrict__ ysc,
                   void* __restrict__ ysplit, int nsplit, int f16) {
-    __shared__ unsigned jl[256];
-    __shared__ float zl[256];
+    __shared__ unsigned jl[kGbProposeWalkers];
+    __shared__ float zl[kGbProposeWalkers];
     const unsigned p = blockIdx.y;
-    const unsigned kb = blockIdx.x * 256;
-    const unsigned k = kb + threadIdx.x;
+    const unsigned kb = blockIdx.x * kGbProposeWalkers;
     const unsigned d = dims[p];
     const float* X = xs + ((size_t)p * 2 * K + (half ? K : 0)) * kGbD;
     const float* S = xs + ((size_t)p * 2 * K + (half ? 0 : K)) * kGbD;
-    const bh_f32x4 u = bh_u01x4(bh_philox4x32_10(bh_u32x4{k, step, oe, BH_CTR3},
-                                                 seed0 + 2u * p + (half ? 1u : 0u),
-                                                 BH_KEY1_STRETCH));
-    const float inv_a = 1.0f / a;
-    const float ca = a - 2.0f + inv_a;
-    const float cb = 2.0f * (1.0f - inv_a);
-    const float z = __builtin_fmaf(ca * u.y, u.y, cb * u.y) + inv_a;
-    unsigned j = (unsigned)(u.x * (float)K);
-    j = j < K ? j : K - 1;
-    jl[threadIdx.x] = j;
-    zl[threadIdx.x] = z;
-    zbuf[(size_t)p * K + k] = z;
-    u2buf[(size_t)p * K + k] = u.z;
+    if (threadIdx.x < kGbProposeWalkers) {
+        const unsigned k = kb + threadIdx.x;
+        const bh_f32x4 u = bh_u01x4(bh_philox4x32_10(bh_u32x4{k, step, oe, BH_CTR3},
+                                                     seed0 + 2u * p + (half ? 1u : 0u),
+                                                     BH_KEY1_STRETCH));
+        const float inv_a = 1.0f / a;
+        const float ca = a - 2.0f + inv_a;
+        const float cb = 2.0f * (1.0f - inv_a);
+        const float z = __builtin_fmaf(ca * u.y, u.y, cb * u.y) + inv_a;
+        unsigned j = (unsigned)(u.x * (float)K);
+        j = j < K ? j : K - 1;
+        jl[threadIdx.x] = j;
+        zl[threadIdx.x] = z;
+        zbuf[(size_t)p * K + k] = z;
+        u2buf[(size_t)p * K + k] = u.z;
+    }
     __syncthreads();
     const float* t = tscale + (size_t)p * kGbD;
     if (d <= 32)
@@ -537,20 +555,29 @@ gb_logpost_kernel(const float* __restrict__ xs, const unsigned* __restrict__ dim
 // d <= D), in 16-byte accesses over the first D slots of its proposal and
 // position (the slots from d on are zeros in both, and so are the linear
 // coefficients there).
-// Sum over the wave for lane 0 in the butterfly's pairing (lane t adds
-// lane t + i, i = 32, 16, 8, 4, 2, 1): v_permlane32_swap / v_permlane16_swap
-// bring lanes t + 32 / t + 16 to the low lanes (the builtins' second result),
-// DPP row_shl:i lane t + i within each 16-lane row.
-__device__ __forceinline__ float gb_wave_sum_lane0(float x) {
-    const unsigned u = __float_as_uint(x);
-    x = x + __uint_as_float(__builtin_amdgcn_permlane32_swap(u, u, false, false)[1]);
-    const unsigned u16 = __float_as_uint(x);
-    x = x + __uint_as_float(__builtin_amdgcn_permlane16_swap(u16, u16, false, false)[1]);
+// Sums over the wave of four values per lane in the tree's pairing (lane t adds
+// lane t + i, i = 32, 16, 8, 4, 2, 1), value `gb_wave_sums_at` of them in the
+// first lane of each row of 16.  v_permlane32_swap puts two values' halves side
+// by side, v_permlane16_swap two pairs' rows, so that one add takes a level of
+// two values; the levels inside a row (DPP row_shl:i) take four.
+__device__ __forceinline__ float gb_wave_sums(float x0, float x1, float x2, float x3) {
+    const auto add32 = [](float a, float b) {
+        const auto v = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+        return __uint_as_float(v[0]) + __uint_as_float(v[1]);
+    };
+    const auto v = __builtin_amdgcn_permlane16_swap(__float_as_uint(add32(x0, x1)),
+                                                    __float_as_uint(add32(x2, x3)), false, false);
+    float x = __uint_as_float(v[0]) + __uint_as_float(v[1]);
     x = x + __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(x), 0x108, 0xf, 0xf, false));
     x = x + __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(x), 0x104, 0xf, 0xf, false));
     x = x + __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(x), 0x102, 0xf, 0xf, false));
     x = x + __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(x), 0x101, 0xf, 0xf, false));
     return x;
+}
+// rows 0 .. 3 hold the values 0, 2, 1, 3
+__device__ __forceinline__ unsigned gb_wave_sums_at(unsigned lane) {
+    const unsigned row = lane >> 4;
+    return (row & 1u) * 2 + (row >> 1);
 }
 
 template <int D>
@@ -572,11 +599,21 @@ __device__ __forceinline__ void gb_accept_one(int half, unsigned p, unsigned k, 
     if (threadIdx.x < D) lin_s[threadIdx.x] = lin[(size_t)p * kGbD + threadIdx.x];
     __syncthreads();
     const float4* y4 = reinterpret_cast<const float4*>(Y + ((size_t)p * K + k) * kGbD);
+    const size_t w = (size_t)p * 2 * K + (half ? K : 0) + k;
+    const float z = zbuf[(size_t)p * K + k], u2 = u2buf[(size_t)p * K + k];
+    const double lpx = lp[w];
+    // the point in runs of eight loads, the first in flight with the units'
+    float4 yv[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) yv[i] = y4[i];
     const double s = gb_unit_sum(partial + k, K, ubeg[p], ubeg[p + 1]);
     double l = 0.0, q = 0.0;
-#pragma unroll 4
+#pragma unroll
     for (int c = 0; c < D / 4; ++c) {
-        const float4 v = y4[c];
+        if (c % 8 == 0 && c > 0)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) yv[i] = y4[c + i];
+        const float4 v = yv[c % 8];
         const float a[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -585,16 +622,14 @@ __device__ __forceinline__ void gb_accept_one(int half, unsigned p, unsigned k, 
         }
     }
     const double lpy = l - scale * s - 0.5 * prior_prec * q;
-    const size_t w = (size_t)p * 2 * K + (half ? K : 0) + k;
     float4* xk4 = reinterpret_cast<float4*>(xs + w * kGbD);
-    const float z = zbuf[(size_t)p * K + k];
     float zp = 1.0f;
     for (unsigned i = 0; i + 1 < d; ++i) zp *= z;
-    const float dl = (float)(lpy - lp[w]);
+    const float dl = (float)(lpy - lpx);
     const float qa = __builtin_isfinite(lpy) ? zp * expf(beta * dl) : 0.0f;
-    const bool accepted = u2buf[(size_t)p * K + k] <= qa;
+    const bool accepted = u2 <= qa;
     if (accepted) {
-#pragma unroll 4
+#pragma unroll 8
         for (int c = 0; c < D / 4; ++c) xk4[c] = y4[c];
         lp[w] = lpy;
     }
@@ -602,19 +637,22 @@ __device__ __forceinline__ void gb_accept_one(int half, unsigned p, unsigned k, 
     const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const unsigned long long ball = __ballot(accepted);
     if (lane == 0) cnt[wave] = (unsigned)__popcll(ball);
-    // the walker's coordinates after the move, four at a time, reduced over
-    // the wave coordinate by coordinate
+    // the walker's coordinates after the move, 32 loaded at a time (records are
+    // D floats), reduced over the wave four coordinates at a time
     const float4* src = accepted ? y4 : xk4;
-    for (unsigned c = 0; 4 * c < d; ++c) {
-        const float4 v = src[c];
-        const float a[4] = {v.x, v.y, v.z, v.w};
+    for (unsigned c0 = 0; 4 * c0 < d; c0 += 8) {
+        float4 v[8];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float s1 = gb_wave_sum_lane0(a[e]);
-            const float s2 = gb_wave_sum_lane0(a[e] * a[e]);
-            if (lane == 0 && 4 * c + e < d) {
-                red[0][wave][4 * c + e] = s1;
-                red[1][wave][4 * c + e] = s2;
+        for (unsigned i = 0; i < 8; ++i) v[i] = src[c0 + i];
+#pragma unroll
+        for (unsigned i = 0; i < 8; ++i) {
+            if (i % 4 == 0 && 4 * (c0 + i) >= d) break;
+            const float4 x = v[i];
+            const float s1 = gb_wave_sums(x.x, x.y, x.z, x.w);
+            const float s2 = gb_wave_sums(x.x * x.x, x.y * x.y, x.z * x.z, x.w * x.w);
+            if ((lane & 15u) == 0) {
+                red[0][wave][4 * (c0 + i) + gb_wave_sums_at(lane)] = s1;
+                red[1][wave][4 * (c0 + i) + gb_wave_sums_at(lane)] = s2;
             }
         }
     }
@@ -636,7 +674,9 @@ __device__ __forceinline__ void gb_accept_one(int half, unsigned p, unsigned k, 
 // the accounting: accepted walkers per problem (acc_cnt), and per 256-walker
 // block the sums of x and x^2 of every coordinate over the block's walkers
 // after the move (msum/msum2[p][slot][64], slot = half * K/256 + block of the
-// W/256 slots; a fixed shuffle-and-LDS tree).
+// W/256 slots; a fixed shuffle-and-LDS tree).  Bound by latency: its loads go
+// together, and four coordinates share a wave's adds (64 problems of 1024
+// points, accounted: 19.4 -> 12.3 us).
 __global__ void __launch_bounds__(256)
 gb_accept_kernel(int half, const unsigned* __restrict__ dims, const unsigned* __restrict__ ubeg,
                  const float* __restrict__ Y, const float* __restrict__ zbuf,
@@ -709,7 +749,7 @@ hipError_t launch_gb_propose(hipStream_t s, unsigned seed0, int half, unsigned o
                              float a, const unsigned* dims, const float* tscale, const float* xs,
                              unsigned P, unsigned K, float* Y, float* z, float* u2, float* ysc,
                              void* ysplit, int nsplit, int f16) {
-    gb_propose_kernel<<<dim3(K / 256, P), 256, 0, s>>>(seed0, half, oe, step, a, dims, tscale,
+    gb_propose_kernel<<<dim3(K / kGbProposeWalkers, P), 256, 0, s>>>(seed0, half, oe, step, a, dims, tscale,
                                                        xs, P, K, Y, z, u2, ysc, ysplit, nsplit,
                                                        f16);
     return hipGetLastError();
