@@ -479,11 +479,14 @@ __device__ __forceinline__ void bh_stretch_half_staged(unsigned seed, unsigned o
             xk[i] = y[i];
             tile[t * ST + i] = y[i];
         }
-        __builtin_nontemporal_store(ly, logfn_X + k);
+        lx = ly;
     } else if (out) {
 #pragma unroll
         for (int i = 0; i < DIM; ++i) tile[t * ST + i] = xk[i];
     }
+    // accepted or not: whole lines of 32 log densities take less than masked ones
+    // (2^21 x 16, us per half-step: 70.7 -> 69.7)
+    __builtin_nontemporal_store(lx, logfn_X + k);
     const unsigned long long m = __ballot(accepted);
     if ((t & 63u) == 0) acc_mask[t >> 6] = m;
     __syncthreads();
