@@ -20,6 +20,7 @@
 #include "bh_glm.hpp"
 #include "bh_glm_batch.hpp"
 #include "bh_kernels.hpp"
+#include "bh_pool.hpp"
 
 // Sources handed to hipRTC, embedded at build time as raw string literals.
 #include "bh_rtc_sources.inc"
@@ -68,6 +69,24 @@ bool is_device_ptr(const void* p) {
     return a.type == hipMemoryTypeDevice || a.type == hipMemoryTypeManaged;
 }
 
+struct HipMemory {
+    static int alloc(void** p, size_t bytes, bool pinned) {
+        const hipError_t e = pinned ? hipHostMalloc(p, bytes, hipHostMallocDefault)
+                                    : hipMalloc(p, bytes);
+        if (e == hipSuccess) return BH_OK;
+        (void)hipGetLastError();  // not the next launch's
+        *p = nullptr;
+        return fail(BH_ERR_HIP, "%zu bytes of %s memory: %s", bytes, pinned ? "pinned" : "device",
+                    hipGetErrorString(e));
+    }
+    static void release(void* p, bool pinned) {
+        if (pinned)
+            (void)hipHostFree(p);
+        else
+            (void)hipFree(p);
+    }
+};
+
 // Device buffer owned for the duration of a call.
 struct DevBuf {
     void* p = nullptr;
@@ -83,7 +102,7 @@ struct DevBuf {
         if (p) (void)hipFree(p);
         p = nullptr;
         bytes = 0;
-        BH_HIP(hipMalloc(&p, n ? n : 1));
+        BH_TRY(bh::alloc_or_reclaim<HipMemory>(&p, n ? n : 1, false));
         bytes = n;
         return BH_OK;
     }
@@ -98,70 +117,7 @@ struct DevBuf {
     }
 };
 
-// Device and pinned host memory that a context's calls use while they run.
-// A call used to allocate and free each of its buffers and to copy each result
-// down by itself (a copy to pageable memory costs ~9 us of the host's time, a
-// wait 11): draws, densities and estimates of 65,536 values took 247 us in six
-// calls of which the kernels are 75, and take 137 with this.  The blocks are
-// kept between calls, at most kDevMax + kPinMax bytes of them, and freed with
-// the context; a call holds its blocks until its stream is idle, so any call
-// on any stream of the context may use them next.
-struct Pool {
-    static constexpr size_t kDevMax = (size_t)64 << 20, kPinMax = (size_t)4 << 20;
-    struct Block {
-        void* p;
-        size_t bytes;
-        bool pinned;
-    };
-    std::mutex mu;
-    std::vector<Block> kept;
-    size_t kept_bytes[2] = {0, 0};
-    ~Pool() {
-        for (const Block& b : kept) release(b);
-    }
-    static void release(const Block& b) {
-        if (b.pinned)
-            (void)hipHostFree(b.p);
-        else
-            (void)hipFree(b.p);
-    }
-    int get(size_t bytes, bool pinned, Block* out) {
-        size_t want = bytes;  // a size that is kept: the next power of two
-        if (bytes <= (pinned ? kPinMax : kDevMax))
-            for (want = 4096; want < bytes;) want *= 2;
-        {
-            std::lock_guard<std::mutex> lk(mu);
-            for (size_t i = 0; i < kept.size(); ++i) {
-                if (kept[i].pinned != pinned || kept[i].bytes != want) continue;
-                *out = kept[i];
-                kept_bytes[pinned] -= want;
-                kept[i] = kept.back();
-                kept.pop_back();
-                return BH_OK;
-            }
-        }
-        Block b{nullptr, want, pinned};
-        if (pinned)
-            BH_HIP(hipHostMalloc(&b.p, want, hipHostMallocDefault));
-        else
-            BH_HIP(hipMalloc(&b.p, want));
-        *out = b;
-        return BH_OK;
-    }
-    void put(const Block& b) {
-        {
-            std::lock_guard<std::mutex> lk(mu);
-            if (kept.size() < kept.capacity() &&
-                kept_bytes[b.pinned] + b.bytes <= (b.pinned ? kPinMax : kDevMax)) {
-                kept_bytes[b.pinned] += b.bytes;
-                kept.push_back(b);
-                return;
-            }
-        }
-        release(b);
-    }
-    Pool() { kept.reserve(64); }
-};
+using Pool = bh::Pool<HipMemory>;
 
 // One call's buffers and results on its stream.  Inputs and outputs in device
 // memory are used in place.  A small result for the host is written by its
