@@ -732,7 +732,9 @@ __device__ __forceinline__ void bh_resident_accept(float* X, unsigned K, unsigne
 // the one load it needs instead of for all (which would be 0.7 us every
 // half-step).  For the same reason the loops have one way out, after whole
 // rounds of BH_RESIDENT_AHEAD; in what is past the last half-step nothing is
-// decided and the positions go to `sink` (K * DIM floats).
+// decided and the positions go to `sink` (K * DIM floats).  The draws there
+// were never made: the density, whose loops may depend on its argument, is
+// evaluated at a position of the other half instead (z = 0).
 #define BH_RESIDENT_AHEAD 4
 
 // nsteps steps with one walker of each half per thread (blockDim.x == K): the
@@ -790,11 +792,12 @@ __device__ __forceinline__ void bh_resident_one(
             asm volatile("" : "+v"(d[r]));
             float* X = sx + (h ? H : 0u);
             float sj[DIM], y[DIM];
+            const float z = live ? d[r].x : 0.0f;
             const float* S = sx + (h ? 0u : H) + (live ? __float_as_uint(d[r].y) : 0u);
 #pragma unroll
             for (int i = 0; i < DIM; ++i) sj[i] = S[i];
 #pragma unroll
-            for (int i = 0; i < DIM; ++i) y[i] = __builtin_fmaf(d[r].x, x[h][i] - sj[i], sj[i]);
+            for (int i = 0; i < DIM; ++i) y[i] = __builtin_fmaf(z, x[h][i] - sj[i], sj[i]);
             const float ly = LOGFN(data_len, params_len, params, DIM, y);
             // (u2 > 0: a log density that is not finite is never accepted)
             const float q = d[r].w * expf(b[r / NH] * (ly - lx[h]));
@@ -866,13 +869,14 @@ __device__ __forceinline__ void bh_resident_slots(
             asm volatile("" : "+v"(d[r]));
             float* X = sx + h * H;
             float xk[DIM], sj[DIM], y[DIM];
+            const float z = live ? d[r].x : 0.0f;
             const float* S = sx + (h ^ 1u) * H + (live ? __float_as_uint(d[r].y) : 0u);
 #pragma unroll
             for (int i = 0; i < DIM; ++i) sj[i] = S[i];
             bh_load_walker(X + k * DIM, xk);
             const float lx = sl[h * K + k];
 #pragma unroll
-            for (int i = 0; i < DIM; ++i) y[i] = __builtin_fmaf(d[r].x, xk[i] - sj[i], sj[i]);
+            for (int i = 0; i < DIM; ++i) y[i] = __builtin_fmaf(z, xk[i] - sj[i], sj[i]);
             const float ly = LOGFN(data_len, params_len, params, DIM, y);
             const float q = d[r].w * expf(b * (ly - lx));
             const bool acc = live && __builtin_isfinite(ly) && d[r].z <= q;
