@@ -423,7 +423,6 @@ struct bh_stretch {
     uint32_t params_count = 0, data_len = 0, params_len = 0;
     DevBuf xs, logfn, params, accept, means_acc;
     DevBuf fentries, fpos, fstarts, fg;  // partners found beforehand (see found_alloc)
-    DevBuf rdraws, rtrace, rsink;  // a chunk of resident steps' draws and positions
     uint64_t means_cap = 0;
     uint32_t bare_seed = 0, move_seed = 0, bare_counter = 0, move_counter = 0;
     uint64_t iter = 0;
@@ -564,8 +563,11 @@ bool resident_accepted(const bh_stretch* s) {
     return floats * 4 + (nb / 64) * 4 <= 64 * 1024;
 }
 
-// Draws and trace of one chunk of resident steps; kept by the sampler.  (Two
-// rounds of the kernel's four draws in flight lie past the last half-step.)
+// Draws and trace of one chunk of resident steps, blocks of the call: kept by
+// a sampler they were allocated anew for each one (burn-in, run and sample of
+// 1024 walkers x 4 on a fresh sampler 1990 us, on a used one 1290; now 1300 and
+// 1280).
+// (Two rounds of the kernel's four draws in flight lie past the last half-step.)
 constexpr uint32_t kResidentPad = 8;
 constexpr size_t kResidentWork = (size_t)16 << 20;
 constexpr uint32_t kResidentSteps = 16384;
@@ -602,9 +604,9 @@ int resident_module(bh_stretch_factory* f) {
 // nsteps resident steps: per chunk the draws, the steps and, with accu, the
 // accounting from their trace; with sample_out the positions after every
 // step go there (nsteps whole ensembles).
-int run_resident(bh_stretch* s, bool accu, uint32_t seed_odd, uint32_t seed_even, uint32_t c_odd,
-                 uint32_t c_even, float a, float beta, const float* d_betas, uint32_t step0,
-                 uint32_t nsteps, float* sample_out) {
+int run_resident(bh_stretch* s, Call& call, bool accu, uint32_t seed_odd, uint32_t seed_even,
+                 uint32_t c_odd, uint32_t c_even, float a, float beta, const float* d_betas,
+                 uint32_t step0, uint32_t nsteps, float* sample_out) {
     if (nsteps == 0) return BH_OK;
     BH_TRY(resident_module(s->f));
     const unsigned nb = resident_block(s), Kp = nb * resident_slots(s);
@@ -614,19 +616,19 @@ int run_resident(bh_stretch* s, bool accu, uint32_t seed_odd, uint32_t seed_even
     const uint32_t most = (uint32_t)std::min<size_t>(
         kResidentSteps, std::max<size_t>(1, kResidentWork / per_step));
     const uint32_t chunk = std::min(nsteps, most);
-    BH_TRY(s->rdraws.alloc(draw_bytes * chunk + (size_t)kResidentPad * nb * 16));
-    BH_TRY(s->rsink.alloc(step_floats / 2 * sizeof(float)));
-    if (accu) BH_TRY(s->rtrace.alloc(step_floats * sizeof(float) * chunk));
+    float4* draws;
+    float *sink, *rtrace = nullptr;
+    BH_TRY(call.dev((size_t)2 * chunk * Kp + (size_t)kResidentPad * nb, &draws));
+    BH_TRY(call.dev(step_floats / 2, &sink));
+    if (accu) BH_TRY(call.dev(step_floats * chunk, &rtrace));
     unsigned data_len = s->data_len, params_len = s->params_len, K = s->K;
     const float* params = s->params.as<float>();
     float* xs = s->xs.as<float>();
     float* lf = s->logfn.as<float>();
-    float4* draws = s->rdraws.as<float4>();
     const float4* drawsc = draws;
     int partner = s->partner;
     unsigned* acc = accu ? s->accept.as<unsigned>() : nullptr;
     float* means = s->means_acc.as<float>();
-    float* sink = s->rsink.as<float>();
     for (uint32_t done = 0; done < nsteps; done += chunk) {
         unsigned n = std::min(chunk, nsteps - done), step = step0 + done;
         unsigned kp = Kp;
@@ -635,7 +637,7 @@ int run_resident(bh_stretch* s, bool accu, uint32_t seed_odd, uint32_t seed_even
         BH_HIP(hipModuleLaunchKernel(s->f->draws, (K + 255) / 256, std::min(2 * n, 65535u), 1, 256,
                                      1, 1, 0, s->stream, da, nullptr));
         const float* betas = d_betas ? d_betas + done : nullptr;
-        float* out = accu ? s->rtrace.as<float>() : nullptr;
+        float* out = rtrace;
         if (sample_out) out = sample_out + step_floats * done;
         void* ra[] = {&drawsc, &data_len, &params_len, &params, &xs,  &lf, &K,
                       &beta,   &betas,    &n,          &acc,    &out, &sink};
@@ -644,7 +646,7 @@ int run_resident(bh_stretch* s, bool accu, uint32_t seed_odd, uint32_t seed_even
                           (unsigned)resident_lds(s), s->stream, ra);
         }));
         if (accu) {
-            const float* trace = s->rtrace.as<float>();
+            const float* trace = rtrace;
             void* ta[] = {&trace, &K, &step, &means};
             BH_HIP(hipModuleLaunchKernel(s->f->trace_accu, s->groups, n, 1, s->wgs, 1, 1, 0,
                                          s->stream, ta, nullptr));
@@ -1068,25 +1070,20 @@ int accu_pair(bh_stretch* s) {
 int bare_steps(bh_stretch* s, uint64_t n, const float* h_betas) {
     if (n == 0) return BH_OK;
     if (use_resident(s)) {
-        DevBuf d_betas;
-        const float* db = nullptr;
-        if (h_betas) {
-            BH_TRY(d_betas.alloc(n * sizeof(float)));
-            BH_HIP(hipMemcpyAsync(d_betas.p, h_betas, n * sizeof(float), hipMemcpyHostToDevice,
-                                  s->stream));
-            db = d_betas.as<float>();
-        }
         // the kernel's step counter is 32-bit, as the reference's (int-array)
         uint64_t done = 0;
         while (done < n) {
             const uint32_t chunk = (uint32_t)std::min<uint64_t>(n - done, 1u << 20);
-            BH_TRY(run_resident(s, false, s->bare_seed, s->bare_seed + 1u, 3333, 4444, s->bare_a,
-                                s->beta, db ? db + done : nullptr, s->bare_counter, chunk, nullptr));
+            Call call(s->ctx->pool, s->stream);
+            const float* db = nullptr;
+            if (h_betas) BH_TRY(call.in(h_betas + done, chunk, &db));
+            BH_TRY(run_resident(s, call, false, s->bare_seed, s->bare_seed + 1u, 3333, 4444,
+                                s->bare_a, s->beta, db, s->bare_counter, chunk, nullptr));
             s->bare_counter += chunk;
             done += chunk;
+            BH_TRY(call.finish());
         }
         if (h_betas) s->beta = h_betas[n - 1];
-        BH_TRY(sync(s->stream));
         return BH_OK;
     }
     for (uint64_t i = 0; i < n; ++i) {
@@ -1118,10 +1115,11 @@ int accu_steps(bh_stretch* s, uint64_t n) {
                     (unsigned long long)s->means_cap);
     if (n == 0) return BH_OK;
     if (use_resident(s)) {
-        BH_TRY(run_resident(s, true, s->move_seed, s->move_seed + 1u, 1111, 2222, s->accu_a, 1.0f,
-                            nullptr, s->move_counter, (uint32_t)n, nullptr));
+        Call call(s->ctx->pool, s->stream);
+        BH_TRY(run_resident(s, call, true, s->move_seed, s->move_seed + 1u, 1111, 2222, s->accu_a,
+                            1.0f, nullptr, s->move_counter, (uint32_t)n, nullptr));
         s->move_counter += (uint32_t)n;
-        return sync(s->stream);
+        return call.finish();
     }
     for (uint64_t i = 0; i < n; ++i) {
         BH_TRY(accu_pair(s));
@@ -3221,11 +3219,11 @@ int bh_stretch_sample(bh_stretch* s, float* out, uint64_t ncols) {
         // whole ensembles straight into the output; of a last part, its step
         // and a copy
         const uint32_t whole = (uint32_t)(req / avail);
-        BH_TRY(run_resident(s, false, s->bare_seed, s->bare_seed + 1u, 3333, 4444, s->bare_a, 1.0f,
-                            nullptr, s->bare_counter, whole, o));
+        BH_TRY(run_resident(s, call, false, s->bare_seed, s->bare_seed + 1u, 3333, 4444, s->bare_a,
+                            1.0f, nullptr, s->bare_counter, whole, o));
         if (whole < steps) {
-            BH_TRY(run_resident(s, false, s->bare_seed, s->bare_seed + 1u, 3333, 4444, s->bare_a,
-                                1.0f, nullptr, s->bare_counter + whole, 1, nullptr));
+            BH_TRY(run_resident(s, call, false, s->bare_seed, s->bare_seed + 1u, 3333, 4444,
+                                s->bare_a, 1.0f, nullptr, s->bare_counter + whole, 1, nullptr));
             BH_HIP(hipMemcpyAsync(o + (size_t)whole * avail, s->xs.p,
                                   (req - (size_t)whole * avail) * sizeof(float),
                                   hipMemcpyDeviceToDevice, s->stream));

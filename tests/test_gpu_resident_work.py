@@ -43,3 +43,29 @@ def test_density_past_the_last_half_step(wgs, walkers, steps):
     assert ms < 1.0, ms
     sf.release()
     fac.release()
+
+
+def test_fresh_samplers_share_the_chunk_buffers():
+    """A second sampler's job takes no device memory of its own: 1024 walkers x
+    4 draw 16 MiB and trace 8 MiB per chunk."""
+    import torch
+    fac = engine.HipBayaderaFactory(0, 256)
+    sf = fac.mcmc_factory(models.diag_gaussian_model(4))
+    params = np.array([0, 0, 0, 0, 1, 1, 1, 1], np.float32)
+
+    def sampler(seed):
+        return sf.create_sampler(seed, 1024, params).init_position(seed, [-2, 2] * 4)
+
+    def job(s):
+        s.burn_in(256, 2.0)
+        s.run_sampler(1024, 2.0)
+        s.sample(1 << 18, out=torch.empty(1 << 18, 4, device="cuda"))
+
+    first, second = sampler(1), sampler(2)
+    job(first)  # the context's buffers, and torch's block for the draws
+    second.init_move(2.0, 1024)  # the sums of this many steps are the sampler's own
+    before = torch.cuda.mem_get_info()[0]
+    job(second)
+    assert torch.cuda.mem_get_info()[0] == before
+    for h in (first, second, sf, fac):
+        h.release()
