@@ -285,13 +285,14 @@ __global__ void __launch_bounds__(256)
 glm_gauss_pack_kernel(const float* __restrict__ X, const float* __restrict__ y,
                       unsigned long long N, unsigned d, unsigned D, float* __restrict__ Xf,
                       float* __restrict__ yf) {
-    const unsigned long long rows = ((N + 15) / 16 + 1) * 16;
-    const unsigned long long i = (unsigned long long)blockIdx.x * 256 + threadIdx.x;
-    if (i >= rows * D) return;
-    const unsigned long long row = i / D;
-    const unsigned j = (unsigned)(i % D);
-    Xf[gauss_frag_at(row, j, D)] = row < N && j < d ? X[row * d + j] : 0.0f;
-    if (j == 0) yf[row] = row < N ? y[row] : 0.0f;
+    const unsigned long long items = ((N + 15) / 16 + 1) * 16 * D;
+    for (unsigned long long i = (unsigned long long)blockIdx.x * 256 + threadIdx.x; i < items;
+         i += (unsigned long long)gridDim.x * 256) {
+        const unsigned long long row = i / D;
+        const unsigned j = (unsigned)(i % D);
+        Xf[gauss_frag_at(row, j, D)] = row < N && j < d ? X[row * d + j] : 0.0f;
+        if (j == 0) yf[row] = row < N ? y[row] : 0.0f;
+    }
 }
 
 // The fp32 kernel, on the matrix cores: U = X.B in 16 x 16 tiles of rows and
@@ -1113,8 +1114,11 @@ size_t glm_gauss_y_floats(unsigned long long N) { return gauss_rows(N); }
 hipError_t launch_glm_gauss_pack(hipStream_t s, const float* X, const float* y,
                                  unsigned long long N, unsigned d, unsigned D, float* Xf,
                                  float* yf) {
-    const unsigned long long items = glm_gauss_x_floats(N, D);
-    glm_gauss_pack_kernel<<<(unsigned)((items + 255) / 256), 256, 0, s>>>(X, y, N, d, D, Xf, yf);
+    // (a grid takes less than 2^32 threads: from 67M rows of 64 columns on a
+    // thread has more than one float)
+    const unsigned long long blocks = (glm_gauss_x_floats(N, D) + 255) / 256;
+    glm_gauss_pack_kernel<<<(unsigned)(blocks < (1u << 22) ? blocks : 1u << 22), 256, 0, s>>>(
+        X, y, N, d, D, Xf, yf);
     return hipGetLastError();
 }
 
