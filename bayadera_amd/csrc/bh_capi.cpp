@@ -1887,6 +1887,9 @@ int bh_glm_gaussian_factory_create(bh_ctx* ctx, const float* X, const float* y, 
     g->N = N;
     g->d = d;
     g->D = d <= 16 ? 16 : (d <= 32 ? 32 : 64);
+    // data on the device may still be written by the default stream, which the
+    // context's does not wait for
+    if (is_device_ptr(X) || is_device_ptr(y)) BH_HIP(hipStreamSynchronize(nullptr));
     Call call(ctx->pool, ctx->stream);
     const float *dx, *dy;
     BH_TRY(call.in(X, (size_t)N * d, &dx));

@@ -1,4 +1,5 @@
-"""Linear regressions whose padded data is larger than 2^32 floats."""
+"""Linear regression data: larger than 2^32 padded floats, and in device memory
+that other work is still writing."""
 import numpy as np
 import pytest
 import torch
@@ -32,4 +33,27 @@ def test_rows_past_2p32_floats():
         assert abs(got[_lib.BH_GLM_FP64][k] - ref) <= 1e-12 * (abs(ref) + N)
         del r, e
     sf.release()
+    fac.release()
+
+
+def test_data_that_the_default_stream_is_writing():
+    """X and y on the device, written behind some 50 ms of other work: the same
+    log posteriors as from host copies, bit for bit."""
+    g = torch.Generator(device="cuda").manual_seed(3)
+    X = torch.randn(5000, 7, generator=g, device="cuda")
+    y = torch.randn(5000, generator=g, device="cuda")
+    pts = np.random.default_rng(4).standard_normal((40, 8)).astype(np.float32)
+    fac = engine.HipBayaderaFactory(0, 256)
+    out = []
+    for device in (False, True):
+        Xd, yd = torch.zeros_like(X), torch.zeros_like(y)
+        torch.cuda.synchronize()
+        torch.cuda._sleep(100_000_000)
+        Xd.copy_(X)
+        yd.copy_(y)
+        data = (Xd, yd) if device else (Xd.cpu().numpy(), yd.cpu().numpy())
+        sf = fac.mcmc_factory(models.GlmModel("gaussian", *data, 10.0))
+        out.append([sf.log_density(pts, p) for p in (_lib.BH_GLM_FP32, _lib.BH_GLM_FP64)])
+        sf.release()
+    assert np.array_equal(out[0], out[1])
     fac.release()
