@@ -549,10 +549,16 @@ __device__ __forceinline__ void bh_stretch_half(unsigned seed, unsigned odd_or_e
         // Accepted or not: a line holds several of these small records, so nearly
         // every line is written anyway, and whole ones take less than masked ones
         // (us per half-step, 2^23 x 1 158 -> 149, 2^22 x 4 101 -> 96, 2^21 x 7
-        // 118 -> 109; 2^15 x 7 the same).
-        bh_store_walker_nt(xp, xk);
+        // 118 -> 109; 2^15 x 7 the same).  A record of 8 coordinates or more that
+        // is too wide to stage fills lines of its own, of which few are accepted:
+        // those only (2^18 walkers x 48 coordinates 101 -> 62).
+        if (DIM < 8 || accepted) bh_store_walker_nt(xp, xk);
         __builtin_nontemporal_store(lx, logfn_X + k);
-        if (out) bh_store_walker_nt(out + (size_t)k * DIM, xk);
+        if (out) {
+            // (read again, and not held in registers while the density runs)
+            if (DIM >= 8 && !accepted) bh_load_walker_nt(xp, xk);
+            bh_store_walker_nt(out + (size_t)k * DIM, xk);
+        }
         if (ACCU)
             bh_accu(xk, accepted, blockIdx.x, gridDim.x, step, accept, means, old, bh_accu_lds());
     }

@@ -1,0 +1,37 @@
+"""Records too wide to stage in LDS: only those that moved are written."""
+import pytest
+
+from bayadera_amd import _lib, engine, models
+
+pytestmark = pytest.mark.gpu
+
+CONSTANT = """
+inline REAL constant_logpdf(const uint data_len, const uint params_len, const REAL* params, const uint dim,
+                            const REAL* x) {
+    return params[0];
+}
+"""
+
+
+@pytest.mark.parametrize("wgs,dim", [(256, 48), (512, 32)])
+def test_unmoved_records_are_not_written(wgs, dim):
+    """A log density of 0 everywhere accepts some 60% of the proposals, one of
+    minus infinity none: of three record's lengths (own, partner's, written) a
+    half-step then moves two.  The half-way point between those shares, 1 and
+    2 / 2.6 = 0.77, is 0.88."""
+    fac = engine.HipBayaderaFactory(0, wgs)
+    m = models.distribution_model(CONSTANT, "constant", dimension=dim, params_size=1)
+    sf = fac.mcmc_factory(m)
+    ms = []
+    for value in (0.0, float("-inf")):
+        s = sf.create_sampler(3, 1 << 19, [value]).set_exec(_lib.BH_EXEC_STEPWISE).set_timing(True)
+        s.init_position(4, [-1, 1] * dim)
+        runs = []
+        for _ in range(6):
+            s.burn_in(20, 2.0)
+            runs.append(s.last_gpu_ms())
+        ms.append(min(runs))
+        s.release()
+    assert ms[1] < 0.88 * ms[0], ms
+    sf.release()
+    fac.release()
