@@ -376,6 +376,9 @@ struct bh_stretch_factory {
     uint32_t dim = 0, params_len = 0;
     Module mod;
     hipFunction_t logfn = nullptr, bare = nullptr, accu = nullptr, found = nullptr;
+    // the bare half-step that writes a sample too, where that takes less than a
+    // copy of the ensemble (see sample_by_moves)
+    hipFunction_t bare_out = nullptr;
     // the resident steps' kernels, compiled for the first sampler that takes them
     std::string source, logfn_name;
     std::mutex resident_mu;
@@ -990,6 +993,27 @@ void found_alloc(bh_stretch* s) {
     }
 }
 
+// Which kernel writes a sample from the moves (bh_stretch_move_bare and its _out
+// form, whose conditions these are): none for records of 8 coordinates and more
+// that are not staged, nor where it holds half the work-groups of a compute unit
+// that the plain one does (2^19 walkers a half x 38, correlated Gaussian: 174 us,
+// 129 with a copy; x 44, two work-groups for three, 122 and 144).
+int sample_by_moves(bh_stretch_factory* f) {
+    const uint32_t d = f->dim, stride = d % 4 == 0 ? (d / 4 % 2 ? d : d + 4) : (d | 1u);
+    if (d <= 12) {
+        f->bare_out = f->bare;
+        return BH_OK;
+    }
+    if (f->ctx->wgs * stride * 4 > 49152) return BH_OK;
+    hipFunction_t own;
+    BH_TRY(f->mod.fn("bh_stretch_move_bare_out", &own));
+    int plain = 0, with = 0;
+    BH_HIP(hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&plain, f->bare, (int)f->ctx->wgs, 0));
+    BH_HIP(hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&with, own, (int)f->ctx->wgs, 0));
+    if (2 * with > plain) f->bare_out = own;
+    return BH_OK;
+}
+
 // One bare half-step pair (move-bare!, amd_gcn.clj:347-353): odd half with
 // seed and constant 3333, even half with seed+1 and 4444 (:547-550).
 int bare_pair(bh_stretch* s, float beta, float* out = nullptr) {
@@ -1032,8 +1056,9 @@ int bare_pair(bh_stretch* s, float beta, float* out = nullptr) {
             return launch(s->f->found, p.tiles(), kFoundThreads, 0, s->stream, f1);
         });
     }
-    BH_TRY(ktimed(s, [&] { return launch(s->f->bare, grid, s->wgs, 0, s->stream, a0); }));
-    BH_TRY(ktimed(s, [&] { return launch(s->f->bare, grid, s->wgs, 0, s->stream, a1); }));
+    const hipFunction_t move = out ? s->f->bare_out : s->f->bare;
+    BH_TRY(ktimed(s, [&] { return launch(move, grid, s->wgs, 0, s->stream, a0); }));
+    BH_TRY(ktimed(s, [&] { return launch(move, grid, s->wgs, 0, s->stream, a1); }));
     return BH_OK;
 }
 
@@ -1779,6 +1804,7 @@ int bh_stretch_factory_create(bh_ctx* ctx, const char* source, const char* logfn
     BH_TRY(f->mod.load(code));
     BH_TRY(f->mod.fn("bh_logfn", &f->logfn));
     BH_TRY(f->mod.fn("bh_stretch_move_bare", &f->bare));
+    BH_TRY(sample_by_moves(f.get()));
     BH_TRY(f->mod.fn("bh_stretch_move_accu", &f->accu));
     if (dim <= bh::kPartnerMaxDim) BH_TRY(f->mod.fn("bh_stretch_move_found", &f->found));
     f->source = source;
@@ -3238,7 +3264,7 @@ int bh_stretch_sample(bh_stretch* s, float* out, uint64_t ncols) {
             const uint64_t chunk = std::min(avail, req - ofst);
             // a whole ensemble is written by its moves (in 16-byte pieces), a
             // part of one copied
-            const bool by_moves = !s->f->glm && chunk == avail &&
+            const bool by_moves = s->f->bare_out && chunk == avail &&
                                   reinterpret_cast<uintptr_t>(o + ofst) % 16 == 0;
             BH_TRY(bare_pair(s, 1.0f, by_moves ? o + ofst : nullptr));
             s->bare_counter += 1;

@@ -348,11 +348,11 @@ __device__ __forceinline__ void bh_store_walker_nt(float* p, const float (&v)[DI
 // units (odd number of floats for DIM % 4 != 0) apart, so threads reading
 // consecutive rows hit distinct banks.  Arithmetic and results are those of
 // the thread-per-record path.
-constexpr int bh_stage_stride() {
-    return DIM % 4 == 0 ? ((DIM / 4) % 2 ? DIM : DIM + 4) : (DIM % 2 ? DIM : DIM + 1);
-}
-constexpr int kBhStageStride = bh_stage_stride();
-constexpr bool kBhStage = DIM >= 8 && WGS * kBhStageStride * 4 <= 49152;
+#define BH_STAGE_STRIDE \
+    (DIM % 4 == 0 ? ((DIM / 4) % 2 ? DIM : DIM + 4) : (DIM % 2 ? DIM : DIM + 1))
+#define BH_STAGE (DIM >= 8 && WGS * BH_STAGE_STRIDE * 4 <= 49152)
+constexpr int kBhStageStride = BH_STAGE_STRIDE;
+constexpr bool kBhStage = BH_STAGE;
 
 // One LDS staging area for every instantiation of the staged half-step in a
 // kernel (a __shared__ array declared in each instantiation would be
@@ -554,11 +554,7 @@ __device__ __forceinline__ void bh_stretch_half(unsigned seed, unsigned odd_or_e
         // those only (2^18 walkers x 48 coordinates 101 -> 62).
         if (DIM < 8 || accepted) bh_store_walker_nt(xp, xk);
         __builtin_nontemporal_store(lx, logfn_X + k);
-        if (out) {
-            // (read again, and not held in registers while the density runs)
-            if (DIM >= 8 && !accepted) bh_load_walker_nt(xp, xk);
-            bh_store_walker_nt(out + (size_t)k * DIM, xk);
-        }
+        if (DIM < 8 && out) bh_store_walker_nt(out + (size_t)k * DIM, xk);
         if (ACCU)
             bh_accu(xk, accepted, blockIdx.x, gridDim.x, step, accept, means, old, bh_accu_lds());
     }
@@ -567,20 +563,33 @@ __device__ __forceinline__ void bh_stretch_half(unsigned seed, unsigned odd_or_e
 // With `out` the half's records after the move go there too: a sample of an
 // ensemble is written by its last step instead of being copied from it (2^21
 // x 16 walkers a half: the copy read and wrote 2 x 134 MB, 100 us for both
-// halves; writing alone 43).
-extern "C" __global__ void __launch_bounds__(WGS)
-bh_stretch_move_bare(unsigned seed, unsigned odd_or_even, unsigned data_len, unsigned params_len,
-                     const float* __restrict__ params, const float* __restrict__ S,
-                     float* __restrict__ X, float* __restrict__ logfn_X, float a, float beta,
-                     unsigned step, unsigned K, int partner, float* __restrict__ out) {
-    if (partner == BH_PARTNER_FLAT)
-        bh_stretch_half<false, BH_PARTNER_FLAT>(seed, odd_or_even, data_len, params_len, params, S,
-                                                X, logfn_X, a, beta, step, K, nullptr, nullptr, out);
-    else
-        bh_stretch_half<false, BH_PARTNER_WALKER>(seed, odd_or_even, data_len, params_len, params,
-                                                  S, X, logfn_X, a, beta, step, K, nullptr,
-                                                  nullptr, out);
-}
+// halves; writing alone 43).  A record that does not move then stays in registers
+// while the density runs, which costs wide ones a wave on each SIMD: past 12
+// coordinates the moves that write a sample are a kernel of their own (2^19
+// walkers a half, correlated Gaussian, us without a sample: 28 coordinates 64 ->
+// 57, 38 167 -> 98; 9 and 12 take 1% less as one kernel).  Records of 8 and more
+// that are not staged have none: a thread's own stores of 48 coordinates take
+// 152 us with 2^18 walkers, the move and a copy 80.
+#define BH_BARE_KERNEL(NAME, OUT)                                                                 \
+    extern "C" __global__ void __launch_bounds__(WGS) NAME(                                       \
+        unsigned seed, unsigned odd_or_even, unsigned data_len, unsigned params_len,              \
+        const float* __restrict__ params, const float* __restrict__ S, float* __restrict__ X,     \
+        float* __restrict__ logfn_X, float a, float beta, unsigned step, unsigned K, int partner, \
+        float* __restrict__ out) {                                                                \
+        if (partner == BH_PARTNER_FLAT)                                                           \
+            bh_stretch_half<false, BH_PARTNER_FLAT>(seed, odd_or_even, data_len, params_len,      \
+                                                    params, S, X, logfn_X, a, beta, step, K,      \
+                                                    nullptr, nullptr, (OUT) ? out : nullptr);     \
+        else                                                                                      \
+            bh_stretch_half<false, BH_PARTNER_WALKER>(seed, odd_or_even, data_len, params_len,    \
+                                                      params, S, X, logfn_X, a, beta, step, K,    \
+                                                      nullptr, nullptr, (OUT) ? out : nullptr);   \
+    }
+BH_BARE_KERNEL(bh_stretch_move_bare, DIM <= 12)
+#if DIM > 12 && BH_STAGE
+BH_BARE_KERNEL(bh_stretch_move_bare_out, true)
+#endif
+#undef BH_BARE_KERNEL
 
 extern "C" __global__ void __launch_bounds__(WGS)
 bh_stretch_move_accu(unsigned seed, unsigned odd_or_even, unsigned data_len,

@@ -1,5 +1,8 @@
-"""Records too wide to stage in LDS: only those that moved are written."""
+"""Records too wide to stage in LDS: only those that moved are written, and a
+sample of them is copied."""
+import numpy as np
 import pytest
+import torch
 
 from bayadera_amd import _lib, engine, models
 
@@ -33,5 +36,28 @@ def test_unmoved_records_are_not_written(wgs, dim):
         ms.append(min(runs))
         s.release()
     assert ms[1] < 0.88 * ms[0], ms
+    sf.release()
+    fac.release()
+
+
+def test_sample_of_records_too_wide_to_stage():
+    """A step moves 2.15 record's lengths (own, partner's, those of the 15% that
+    move), a sample two more where the ensemble is copied: 1.93 times as much."""
+    dim, walkers = 48, 1 << 19
+    fac = engine.HipBayaderaFactory(0, 256)
+    sf = fac.mcmc_factory(models.diag_gaussian_model(dim))
+    s = sf.create_sampler(3, walkers, [0.0] * dim + [1.0] * dim).set_exec(_lib.BH_EXEC_STEPWISE).set_timing(True)
+    s.init_position(4, [-2, 2] * dim)
+    s.burn_in(20, 2.0)
+    out = torch.empty(4 * walkers, dim, device="cuda")
+    steps, samples = [], []
+    for _ in range(6):
+        s.burn_in(20, 2.0)
+        steps.append(s.last_gpu_ms() / 20)
+        s.sample(4 * walkers, out=out)
+        samples.append(s.last_gpu_ms() / 4)
+    assert min(samples) < 1.93 * min(steps), (samples, steps)
+    assert np.array_equal(out[3 * walkers:].cpu().numpy(), s.state()[0].reshape(walkers, dim))
+    s.release()
     sf.release()
     fac.release()
