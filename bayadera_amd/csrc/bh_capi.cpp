@@ -464,7 +464,10 @@ constexpr size_t kKernelTimerPairs = 1024;
 // When an ensemble that fits in one compute unit's LDS runs there (see
 // use_resident).  Steps, per-half-step kernels against resident, us per bare /
 // accounted step (correlated Gaussian):
-//   1024 walkers   dim 4   5.7 / 8.0 -> 0.7 / 0.9    dim 24  17 / 27 -> 11 / 10
+//   1024 walkers   dim 4   5.7 / 8.0 -> 0.7 / 0.9    dim 24  17 / 19 -> 6.5 / 7.5
+//                  dim 38  32 / 45 -> 22 / 27
+//   512            dim 48  37 / 42 -> 29 / 25        dim 77 (independent) 19 / 27 -> 5.4 / 11
+//   256 (groups of 64 walkers)                       dim 128 (independent) 24 / 46 -> 11 / 11
 //   4096           dim 1   6.3 / 7.8 -> 1.4 / 1.9    dim 7   7.3 / 12 -> 3.6 / 4.7
 //   8192           dim 1   5.7 / 7.6 -> 2.6 / 3.5    dim 2   5.7 / 7.7 -> 3.0 / 4.1
 // A half-step takes as long as its passes of 1024 walkers, so the line is
@@ -556,6 +559,14 @@ size_t resident_lds(const bh_stretch* s) {
     return (2 * half + s->W + s->groups) * 4;
 }
 
+// The most threads a resident kernel of these records is launched with: those of
+// the largest half of at most 1024 walkers that fits in LDS.
+unsigned resident_threads(const bh_ctx* c, uint32_t dim) {
+    unsigned t = 1024;
+    while (t > 64 && ((size_t)t * dim + dim - 1 + t) * 8 > (size_t)c->lds_max) t -= 64;
+    return t;
+}
+
 // The ensembles BH_EXEC_RESIDENT accepts: positions, log densities and 8
 // floats per thread within 64 KB.
 bool resident_accepted(const bh_stretch* s) {
@@ -595,7 +606,9 @@ int resident_module(bh_stretch_factory* f) {
     std::vector<char> code;
     BH_TRY(rtc_compile(f->ctx->arch, f->source,
                        {"-DWGS=" + std::to_string(f->ctx->wgs), "-DDIM=" + std::to_string(f->dim),
-                        "-DLOGFN=" + f->logfn_name, "-DBH_RESIDENT=1"},
+                        "-DLOGFN=" + f->logfn_name, "-DBH_RESIDENT=1",
+                        "-DBH_RESIDENT_THREADS=" +
+                            std::to_string(resident_threads(f->ctx, f->dim))},
                        code, nullptr, 0));
     if (!f->resident_mod.mod) BH_TRY(f->resident_mod.load(code));
     BH_TRY(f->resident_mod.fn("bh_stretch_resident", &f->resident));

@@ -934,9 +934,14 @@ __device__ __forceinline__ void bh_resident_slots(
 }
 
 // With and without positions to write: two kernels, so that each has its own
-// registers and its own loops.
+// registers and its own loops.  The host bounds their threads by the ensembles
+// that fit in LDS: records of 38 coordinates and more leave at most 512 walkers
+// to a half, whose threads may have 256 registers each.  Bounded by 1024 threads
+// all had 128, and records from 21 coordinates on spilled (us per bare step,
+// independent / correlated Gaussian: 512 walkers x 48 13.3 / 39.9 -> 3.1 / 29.9,
+// 1024 x 32 6.6 / 22.0 -> 3.1 / 17.9; 256 x 128 independent 37.5 -> 10.9).
 #define BH_RESIDENT_KERNEL(NAME, OUT)                                                             \
-    extern "C" __global__ void __launch_bounds__(1024) NAME(                                      \
+    extern "C" __global__ void __launch_bounds__(BH_RESIDENT_THREADS) NAME(                       \
         const float4* __restrict__ draws, unsigned data_len, unsigned params_len,                 \
         const float* __restrict__ params, float* __restrict__ xs, float* __restrict__ logfn,      \
         unsigned K, float beta, const float* __restrict__ betas, unsigned nsteps,                 \

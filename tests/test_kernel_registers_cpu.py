@@ -37,3 +37,11 @@ def resources(tmp_path, model, dim, wgs, *defines):
 @pytest.mark.parametrize("dim,waves", [(16, 5), (28, 4), (38, 2)])
 def test_half_steps_without_a_sample(tmp_path, dim, waves):
     assert resources(tmp_path, "mvn", dim, 256)["bh_stretch_move_bare"]["waves"] >= waves
+
+
+# a thread of a resident kernel holds a record of each half: 1024 threads leave
+# it 128 registers, the 704 that 28 coordinates fit in LDS 168, 384 and fewer 256
+@pytest.mark.parametrize("dim,threads", [(16, 1024), (24, 768), (28, 704), (48, 384), (64, 256)])
+def test_resident_steps_hold_their_records(tmp_path, dim, threads):
+    r = resources(tmp_path, "diag", dim, 64, "-DBH_RESIDENT=1", f"-DBH_RESIDENT_THREADS={threads}")
+    assert r["bh_stretch_resident"]["scratch"] == 0 and r["bh_stretch_resident_out"]["scratch"] == 0
