@@ -586,9 +586,22 @@ constexpr uint32_t kResidentPad = 8;
 constexpr size_t kResidentWork = (size_t)16 << 20;
 constexpr uint32_t kResidentSteps = 16384;
 
-bool use_resident(const bh_stretch* s) {
+// The fewest steps of a call that run resident: the draws are a launch of their
+// own, and the ensemble is read into LDS and written back for each call.  Calls
+// of 1 / 2 / 3 / 4 steps, us, stepwise against resident:
+//   1024 walkers x 4   15.7 20.6 25.5 52   17.8 18.5 19.5 20
+//   4096 x 7           17.5 24.0 30.5 52   24.5 27.7 31.0 34
+//   8192 x 2           16.5 21.6 26.5 52   22.9 25.7 28.9 32
+//   12288 x 2          16.5 21.6 26.6 52   26.0 30.5 34.8 39
+uint64_t resident_steps(const bh_stretch* s) {
+    return 2u + (s->W >= 4096) + (s->W >= 8192);
+}
+
+// Whether a call of so many steps runs resident.
+bool use_resident(const bh_stretch* s, uint64_t steps) {
     if (s->exec == BH_EXEC_STEPWISE || s->f->glm) return false;
     if (s->exec == BH_EXEC_RESIDENT) return true;
+    if (steps < resident_steps(s)) return false;
     if (s->W > kResidentWalkers || resident_lds(s) > (size_t)s->ctx->lds_max) return false;
     return s->W <= kResidentAnyDensity ||
            ((uint64_t)s->data_len * s->W <= kResidentData &&
@@ -1107,7 +1120,7 @@ int accu_pair(bh_stretch* s) {
 
 int bare_steps(bh_stretch* s, uint64_t n, const float* h_betas) {
     if (n == 0) return BH_OK;
-    if (use_resident(s)) {
+    if (use_resident(s, n)) {
         // the kernel's step counter is 32-bit, as the reference's (int-array)
         uint64_t done = 0;
         while (done < n) {
@@ -1152,7 +1165,7 @@ int accu_steps(bh_stretch* s, uint64_t n) {
         return fail(BH_ERR_STATE, "move! beyond the %llu steps reserved by init-move!",
                     (unsigned long long)s->means_cap);
     if (n == 0) return BH_OK;
-    if (use_resident(s)) {
+    if (use_resident(s, n)) {
         Call call(s->ctx->pool, s->stream);
         BH_TRY(run_resident(s, call, true, s->move_seed, s->move_seed + 1u, 1111, 2222, s->accu_a,
                             1.0f, nullptr, s->move_counter, (uint32_t)n, nullptr));
@@ -2016,7 +2029,7 @@ int bh_stretch_create(bh_stretch_factory* f, uint32_t seed, uint32_t walkers,
         BH_HIP(hipMemcpyAsync(s->params.p, params, (size_t)params_count * sizeof(float),
                               hipMemcpyDefault, s->stream));
     BH_TRY(sync(s->stream));
-    if (use_resident(s.get())) BH_TRY(resident_module(f));
+    if (use_resident(s.get(), UINT64_MAX)) BH_TRY(resident_module(f));
     BH_TRY(bh_stretch_init(s.get(), seed));
     *out = s.release();
     return BH_OK;
@@ -2097,7 +2110,7 @@ int bh_stretch_set_exec(bh_stretch* s, int mode) {
         return fail(BH_ERR_RANGE, "ensemble (%u walkers x %u) does not fit in one work-group's LDS",
                     s->W, s->dim);
     s->exec = mode;
-    if (use_resident(s)) BH_TRY(resident_module(s->f));
+    if (use_resident(s, UINT64_MAX)) BH_TRY(resident_module(s->f));
     return BH_OK;
 }
 
@@ -3257,35 +3270,28 @@ int bh_stretch_sample(bh_stretch* s, float* out, uint64_t ncols) {
     float* o;
     BH_TRY(call.out(out, req, &o, true));
     Timed t(s);
-    if (use_resident(s) && steps < (1ull << 31)) {
-        // whole ensembles straight into the output; of a last part, its step
-        // and a copy
-        const uint32_t whole = (uint32_t)(req / avail);
+    // whole ensembles straight into the output, by resident steps where they run
+    // so; what is left step by step
+    const uint64_t whole = req / avail;
+    uint64_t i = 0;
+    if (whole > 0 && whole < (1ull << 31) && use_resident(s, whole)) {
         BH_TRY(run_resident(s, call, false, s->bare_seed, s->bare_seed + 1u, 3333, 4444, s->bare_a,
-                            1.0f, nullptr, s->bare_counter, whole, o));
-        if (whole < steps) {
-            BH_TRY(run_resident(s, call, false, s->bare_seed, s->bare_seed + 1u, 3333, 4444,
-                                s->bare_a, 1.0f, nullptr, s->bare_counter + whole, 1, nullptr));
-            BH_HIP(hipMemcpyAsync(o + (size_t)whole * avail, s->xs.p,
-                                  (req - (size_t)whole * avail) * sizeof(float),
+                            1.0f, nullptr, s->bare_counter, (uint32_t)whole, o));
+        s->bare_counter += (uint32_t)whole;
+        i = whole;
+    }
+    for (uint64_t ofst = i * avail; i < steps; ++i) {
+        const uint64_t chunk = std::min(avail, req - ofst);
+        // a whole ensemble is written by its moves (in 16-byte pieces), a part of
+        // one copied
+        const bool by_moves = s->f->bare_out && chunk == avail &&
+                              reinterpret_cast<uintptr_t>(o + ofst) % 16 == 0;
+        BH_TRY(bare_pair(s, 1.0f, by_moves ? o + ofst : nullptr));
+        s->bare_counter += 1;
+        if (!by_moves)
+            BH_HIP(hipMemcpyAsync(o + ofst, s->xs.p, chunk * sizeof(float),
                                   hipMemcpyDeviceToDevice, s->stream));
-        }
-        s->bare_counter += (uint32_t)steps;
-    } else {
-        uint64_t ofst = 0;
-        for (uint64_t i = 0; i < steps; ++i) {
-            const uint64_t chunk = std::min(avail, req - ofst);
-            // a whole ensemble is written by its moves (in 16-byte pieces), a
-            // part of one copied
-            const bool by_moves = s->f->bare_out && chunk == avail &&
-                                  reinterpret_cast<uintptr_t>(o + ofst) % 16 == 0;
-            BH_TRY(bare_pair(s, 1.0f, by_moves ? o + ofst : nullptr));
-            s->bare_counter += 1;
-            if (!by_moves)
-                BH_HIP(hipMemcpyAsync(o + ofst, s->xs.p, chunk * sizeof(float),
-                                      hipMemcpyDeviceToDevice, s->stream));
-            ofst += chunk;
-        }
+        ofst += chunk;
     }
     BH_TRY(t.stop());
     s->iter += steps;

@@ -69,3 +69,21 @@ def test_fresh_samplers_share_the_chunk_buffers():
     assert torch.cuda.mem_get_info()[0] == before
     for h in (first, second, sf, fac):
         h.release()
+
+
+@pytest.mark.parametrize("walkers,fewest", [(1024, 2), (4096, 3), (8192, 4)])
+def test_calls_of_few_steps(walkers, fewest):
+    """Calls of fewer steps take the two launches of each step, longer ones one
+    launch, and a resident sampler always one."""
+    fac = engine.HipBayaderaFactory(0, 256)
+    sf = fac.mcmc_factory(models.diag_gaussian_model(2))
+    s = sf.create_sampler(3, walkers, [0, 0, 1, 1]).init_position(4, [-2, 2] * 2)
+    for n in (1, 2, 3, 4):
+        for mode, launches in ((_lib.BH_EXEC_AUTO, 1 if n >= fewest else 2 * n), (_lib.BH_EXEC_RESIDENT, 1)):
+            if mode == _lib.BH_EXEC_RESIDENT and walkers > 4096:
+                continue  # refused
+            s.set_exec(mode).set_kernel_timing(True)
+            s.burn_in(n, 2.0)
+            assert s.kernel_timing()["launches"] == launches
+    for h in (s, sf, fac):
+        h.release()
