@@ -998,7 +998,17 @@ int glm_alloc(bh_stretch* s, unsigned n_points, unsigned k_half) {
 //                    2^24  351    43 + 189 + 92
 // so the line is 2^22 walkers; past 2^25 floats a tile has less than a sector
 // of entries in a region.
+// A density that loops over data hides the direct reads behind its arithmetic,
+// and the sort and the reading are added to it.  A half-step, us, direct / sorted,
+// with 16, 32 and 64 values of a light loop (a difference and its square), of a
+// heavy one (an exponential and a logarithm), and of the gaussian likelihood:
+//   light, dim 1, halves of 2^22   70 / 53    70 / 62    71 / 80
+//   heavy                   2^22   70 / 63    71 / 78    73 / 108
+//                           2^23  159 / 108  160 / 134  166 / 194
+//   gaussian, dim 2         2^22   97 / 82   100 / 107  124 / 154
+// so it is left to densities of few parameters (data and hyperparameters).
 constexpr uint32_t kFoundMin = 1u << 22;
+constexpr uint32_t kFoundParams = 20;
 constexpr unsigned kFoundThreads = 1024;  // of bh_stretch_move_found
 bh::PartnerPlan found_plan(const bh_stretch* s) {
     return bh::PartnerPlan{s->K, s->dim, s->fentries.as<unsigned>(), s->fpos.as<unsigned short>(),
@@ -1007,6 +1017,7 @@ bh::PartnerPlan found_plan(const bh_stretch* s) {
 
 void found_alloc(bh_stretch* s) {
     if (s->f->glm || s->dim > bh::kPartnerMaxDim || s->K < kFoundMin) return;
+    if (s->params_count > kFoundParams) return;
     const bh::PartnerPlan p = found_plan(s);
     const size_t K = s->K, starts = (size_t)p.tiles() * (p.regions() + 1);
     if (p.regions() > bh::kPartnerRegions) return;

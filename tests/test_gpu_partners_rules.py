@@ -1,0 +1,34 @@
+"""Which ensembles have their partners sorted: those of densities that take few
+parameters."""
+import numpy as np
+import pytest
+import torch
+
+from bayadera_amd import engine, models
+
+pytestmark = pytest.mark.gpu
+
+LOOP = """
+inline REAL loop_logpdf(const uint data_len, const uint params_len, const REAL* params, const uint dim,
+                        const REAL* x) {
+    REAL acc = 0.0f;
+    for (uint i = 0; i < data_len; i++) acc -= (params[i] - x[0]) * (params[i] - x[0]);
+    return acc * params[data_len];
+}
+"""
+
+
+@pytest.mark.parametrize("values,is_sorted", [(0, True), (16, True), (32, False), (1000, False)])
+def test_density_of_so_many_values(values, is_sorted):
+    """2^23 walkers of one coordinate take 64 MiB (positions and log densities),
+    and 16 bytes for each walker of a half where partners are sorted."""
+    fac = engine.HipBayaderaFactory(0, 256)
+    sf = fac.mcmc_factory(models.distribution_model(LOOP, "loop", dimension=1, params_size=1))
+    params = np.full(values + 1, 0.01, np.float32)
+    sf.create_sampler(1, 512, params).release()
+    before = torch.cuda.mem_get_info()[0]
+    s = sf.create_sampler(3, 1 << 23, params)
+    taken = before - torch.cuda.mem_get_info()[0]
+    assert (taken > (64 << 20) + (32 << 20)) == is_sorted, taken
+    for h in (s, sf, fac):
+        h.release()
