@@ -484,10 +484,10 @@ __device__ __forceinline__ void bh_stretch_half_staged(unsigned seed, unsigned o
 #pragma unroll
         for (int i = 0; i < DIM; ++i) tile[t * ST + i] = xk[i];
     }
-    // accepted or not: whole lines of 32 log densities take less than masked ones
-    // (2^21 x 16, us per half-step: 70.7 -> 69.7)
-    __builtin_nontemporal_store(lx, logfn_X + k);
+    // where any of a wave's walkers moved, all their log densities: whole lines of
+    // 32 take less than masked ones (2^21 x 16, us per half-step: 70.7 -> 69.7)
     const unsigned long long m = __ballot(accepted);
+    if (m) __builtin_nontemporal_store(lx, logfn_X + k);
     if ((t & 63u) == 0) acc_mask[t >> 6] = m;
     __syncthreads();
     // accepted records back to X as consecutive pieces
@@ -546,14 +546,16 @@ __device__ __forceinline__ void bh_stretch_half(unsigned seed, unsigned odd_or_e
         if (ACCU) old.load(blockIdx.x, gridDim.x, step, accept, means);
         const bool accepted = bh_stretch_walker<PARTNER>(k, K, seed, odd_or_even, step, a, beta, S,
                                                          xk, lx, data_len, params_len, params);
-        // Accepted or not: a line holds several of these small records, so nearly
-        // every line is written anyway, and whole ones take less than masked ones
-        // (us per half-step, 2^23 x 1 158 -> 149, 2^22 x 4 101 -> 96, 2^21 x 7
-        // 118 -> 109; 2^15 x 7 the same).  A record of 8 coordinates or more that
-        // is too wide to stage fills lines of its own, of which few are accepted:
-        // those only (2^18 walkers x 48 coordinates 101 -> 62).
-        if (DIM < 8 || accepted) bh_store_walker_nt(xp, xk);
-        __builtin_nontemporal_store(lx, logfn_X + k);
+        // A line holds several of these small records, and whole lines take less
+        // than masked ones: from so many of a wave's walkers moved on, all are
+        // written (us per half-step with 60%, 20% and none moved, the moved ones
+        // written against all: 2^22 x 1 69 68 60 / 63 63 65, 2^22 x 4 101 95 83 /
+        // 96 96 97, 2^22 x 7 146 131 106 / 137 137 138).  A record of 8
+        // coordinates or more that is too wide to stage fills lines of its own:
+        // the moved ones only (2^18 walkers x 48 coordinates, 15% moved, 101 -> 62).
+        const unsigned moved = (unsigned)__popcll(__ballot(accepted));
+        if ((DIM < 8 && moved >= 3 + DIM * 5 / 2) || accepted) bh_store_walker_nt(xp, xk);
+        if (moved >= 5 || accepted) __builtin_nontemporal_store(lx, logfn_X + k);
         if (DIM < 8 && out) bh_store_walker_nt(out + (size_t)k * DIM, xk);
         if (ACCU)
             bh_accu(xk, accepted, blockIdx.x, gridDim.x, step, accept, means, old, bh_accu_lds());

@@ -1,5 +1,5 @@
-"""Records too wide to stage in LDS: only those that moved are written, and a
-sample of them is copied."""
+"""What a half-step writes: of records too wide to stage in LDS only those that
+moved, with a sample of them copied, and of small ones none where none moved."""
 import numpy as np
 import pytest
 import torch
@@ -59,5 +59,27 @@ def test_sample_of_records_too_wide_to_stage():
     assert min(samples) < 1.93 * min(steps), (samples, steps)
     assert np.array_equal(out[3 * walkers:].cpu().numpy(), s.state()[0].reshape(walkers, dim))
     s.release()
+    sf.release()
+    fac.release()
+
+
+def test_small_records_are_not_written_where_none_moved():
+    """Seven coordinates: 32 bytes are read and at most written for a walker and
+    its log density, and one line of 128 for its partner: 192 and, with none
+    moved, 160, which is 0.83.  Half-way to 1 is 0.92."""
+    dim = 7
+    fac = engine.HipBayaderaFactory(0, 256)
+    sf = fac.mcmc_factory(models.distribution_model(CONSTANT, "constant", dimension=dim, params_size=1))
+    ms = []
+    for value in (0.0, float("-inf")):
+        s = sf.create_sampler(3, 1 << 22, [value]).set_timing(True)
+        s.init_position(4, [-1, 1] * dim)
+        runs = []
+        for _ in range(6):
+            s.burn_in(20, 2.0)
+            runs.append(s.last_gpu_ms())
+        ms.append(min(runs))
+        s.release()
+    assert ms[1] < 0.92 * ms[0], ms
     sf.release()
     fac.release()
