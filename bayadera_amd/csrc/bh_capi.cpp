@@ -1157,15 +1157,19 @@ int bare_steps(bh_stretch* s, uint64_t n, const float* h_betas) {
 }
 
 int init_move(bh_stretch* s, float a, uint64_t steps) {
-    s->move_seed += 2u;
-    s->move_counter = 0;
-    s->accu_a = a;
+    const size_t step_bytes = (size_t)s->dim * s->groups * sizeof(float);
+    if (steps > (SIZE_MAX >> 1) / step_bytes)
+        return fail(BH_ERR_RANGE, "init-move! of %llu steps", (unsigned long long)steps);
+    s->move_ready = false;  // the buffers below may be gone when one cannot be made
     BH_TRY(s->accept.alloc((size_t)s->groups * sizeof(unsigned)));
     BH_HIP(hipMemsetAsync(s->accept.p, 0, (size_t)s->groups * sizeof(unsigned), s->stream));
-    const size_t mbytes = (size_t)s->dim * s->groups * (steps ? steps : 1) * sizeof(float);
+    const size_t mbytes = step_bytes * (steps ? steps : 1);
     BH_TRY(s->means_acc.alloc(mbytes));
     BH_HIP(hipMemsetAsync(s->means_acc.p, 0, mbytes, s->stream));
     s->means_cap = steps ? steps : 1;
+    s->move_seed += 2u;
+    s->move_counter = 0;
+    s->accu_a = a;
     s->move_ready = true;
     return BH_OK;
 }
