@@ -425,7 +425,7 @@ struct bh_stretch {
     uint32_t dim = 0, W = 0, K = 0, wgs = 0, groups = 0;
     uint32_t params_count = 0, data_len = 0, params_len = 0;
     DevBuf xs, logfn, params, accept, means_acc;
-    DevBuf fentries, fpos, fstarts, fg;  // partners found beforehand (see found_alloc)
+    bh::Extra<HipMemory> found;  // partners found beforehand (see found_alloc)
     uint64_t means_cap = 0;
     uint32_t bare_seed = 0, move_seed = 0, bare_counter = 0, move_counter = 0;
     uint64_t iter = 0;
@@ -989,8 +989,9 @@ int glm_alloc(bh_stretch* s, unsigned n_points, unsigned k_half) {
 
 // Whether a sampler's half-steps look their partners up beforehand
 // (partner_sort_kernel), and its buffers for that: 12 + 4 dim bytes for each
-// walker of a half, made with the sampler.  Where the memory is short the moves
-// read their partners themselves, as any other ensemble's.  A half-step, us,
+// walker of a half, made with the sampler.  Where the memory is short, or was
+// since (bh::Extra), the moves read their partners themselves, as any other
+// ensemble's.  A half-step, us,
 // direct against sort (half a step's) + read + move:
 //   dim 1, halves of 2^21   27    11 + 14 + 12     2^22   64   15 + 17 + 19
 //                    2^23  149    22 + 32 + 34     2^24  323   43 + 84 + 63
@@ -1011,23 +1012,18 @@ constexpr uint32_t kFoundMin = 1u << 22;
 constexpr uint32_t kFoundParams = 20;
 constexpr unsigned kFoundThreads = 1024;  // of bh_stretch_move_found
 bh::PartnerPlan found_plan(const bh_stretch* s) {
-    return bh::PartnerPlan{s->K, s->dim, s->fentries.as<unsigned>(), s->fpos.as<unsigned short>(),
-                           s->fstarts.as<unsigned>(), s->fg.as<float>()};
+    return bh::PartnerPlan{s->K, s->dim, s->found.as<unsigned>(0), s->found.as<unsigned short>(1),
+                           s->found.as<unsigned>(2), s->found.as<float>(3)};
 }
 
 void found_alloc(bh_stretch* s) {
     if (s->f->glm || s->dim > bh::kPartnerMaxDim || s->K < kFoundMin) return;
     if (s->params_count > kFoundParams) return;
-    const bh::PartnerPlan p = found_plan(s);
+    const bh::PartnerPlan p{s->K, s->dim, nullptr, nullptr, nullptr, nullptr};
     const size_t K = s->K, starts = (size_t)p.tiles() * (p.regions() + 1);
     if (p.regions() > bh::kPartnerRegions) return;
-    if (s->fentries.alloc(2 * K * sizeof(unsigned)) != BH_OK ||
-        s->fpos.alloc(2 * K * sizeof(unsigned short)) != BH_OK ||
-        s->fstarts.alloc(2 * starts * sizeof(unsigned)) != BH_OK ||
-        s->fg.alloc(K * s->dim * sizeof(float)) != BH_OK) {
-        (void)hipGetLastError();
-        for (DevBuf* b : {&s->fentries, &s->fpos, &s->fstarts, &s->fg}) b->drop();
-    }
+    s->found.take({2 * K * sizeof(unsigned), 2 * K * sizeof(unsigned short),
+                   2 * starts * sizeof(unsigned), K * s->dim * sizeof(float)});
 }
 
 // Which kernel writes a sample from the moves (bh_stretch_move_bare and its _out
@@ -1075,7 +1071,8 @@ int bare_pair(bh_stretch* s, float beta, float* out = nullptr) {
     void* a0[] = {&seed0, &c0, &data_len, &params_len, &params, &S1, &x0, &l0, &a, &beta, &step, &K, &partner, &o0};
     void* a1[] = {&seed1, &c1, &data_len, &params_len, &params, &S0, &x1, &l1, &a, &beta, &step, &K, &partner, &o1};
     const unsigned grid = s->K / s->wgs;
-    if (s->fg.p) {
+    const std::unique_lock<std::mutex> held = s->found.hold();
+    if (s->found.there()) {
         const bh::PartnerPlan p = found_plan(s);
         const float* found = p.g;
         const unsigned short *pos0 = p.pos, *pos1 = p.pos + K;

@@ -51,6 +51,52 @@ int alloc_or_reclaim(void** p, size_t bytes, bool pinned) {
     return rc;
 }
 
+// Device memory that its owner can do without: taken only where it is there
+// without others giving theirs back, and given back when an allocation fails
+// (an owner holds the lock while it queues work on the buffers; releasing them
+// waits for that work).
+template <class Memory>
+class Extra : public Spare {
+    std::mutex mu;
+    std::vector<void*> bufs;
+
+    void drop() {
+        for (void* p : bufs) Memory::release(p, false);
+        bufs.clear();
+    }
+
+public:
+    Extra() = default;
+    Extra(const Extra&) = delete;
+    Extra& operator=(const Extra&) = delete;
+    ~Extra() override {
+        spares().remove(this);
+        drop();
+    }
+    // the buffers of these sizes, or none
+    void take(const std::vector<size_t>& bytes) {
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            for (size_t n : bytes) {
+                void* p = nullptr;
+                if (Memory::alloc(&p, n, false) != 0) return drop();
+                bufs.push_back(p);
+            }
+        }
+        spares().add(this);
+    }
+    std::unique_lock<std::mutex> hold() { return std::unique_lock<std::mutex>(mu); }
+    bool there() const { return !bufs.empty(); }
+    template <class T>
+    T* as(size_t i) const {
+        return static_cast<T*>(bufs[i]);
+    }
+    void give_back() override {
+        std::unique_lock<std::mutex> lk(mu, std::try_to_lock);
+        if (lk) drop();
+    }
+};
+
 // Device and pinned host memory that a context's calls use while they run.
 // A call used to allocate and free each of its buffers and to copy each result
 // down by itself (a copy to pageable memory costs ~9 us of the host's time, a

@@ -91,6 +91,21 @@ int main() {
         std::printf("refused %d\n", call(pool, never, 1) != 0);
         Memory::limit = (size_t)1 << 40;
     }
+    {   // what is only of use goes first: where it is not held, and not for its like
+        Memory::limit = 100 * MiB;
+        Pool pool;
+        const size_t need[1] = {90 * MiB};
+        bh::Extra<Memory> a, b;
+        a.take({30 * MiB, 10 * MiB});
+        b.take({50 * MiB, 20 * MiB});  // the second of them does not fit
+        std::printf("extra_taken %d\n", a.there() && !b.there() && Memory::used == 40 * MiB);
+        {
+            auto held = a.hold();
+            std::printf("extra_held %d\n", call(pool, need, 1) != 0 && a.there());
+        }
+        std::printf("extra_given %d\n", call(pool, need, 1) == 0 && !a.there());
+        Memory::limit = (size_t)1 << 40;
+    }
     std::printf("left %zu\n", Memory::used);
     return 0;
 }
@@ -110,6 +125,6 @@ def result(tmp_path_factory):
 
 @pytest.mark.parametrize("what,value", [
     ("after_large", 0), ("large_beside", 0), ("stale_sizes", 0), ("bounded", 1), ("short_of_memory", 0),
-    ("refused", 1), ("left", 0)])
+    ("refused", 1), ("extra_taken", 1), ("extra_held", 1), ("extra_given", 1), ("left", 0)])
 def test_kept_blocks(result, what, value):
     assert int(result[what]) == value

@@ -1,10 +1,10 @@
 """Which ensembles have their partners sorted: those of densities that take few
-parameters."""
+parameters, while the memory for it is there."""
 import numpy as np
 import pytest
 import torch
 
-from bayadera_amd import engine, models
+from bayadera_amd import _lib, engine, models
 
 pytestmark = pytest.mark.gpu
 
@@ -31,4 +31,25 @@ def test_density_of_so_many_values(values, is_sorted):
     taken = before - torch.cuda.mem_get_info()[0]
     assert (taken > (64 << 20) + (32 << 20)) == is_sorted, taken
     for h in (s, sf, fac):
+        h.release()
+
+
+def test_buffers_given_back():
+    """An allocation that fails takes the buffers (2^22 walkers to a half: 64 MiB),
+    and the moves after it are those of a sampler that kept its own."""
+    fac = engine.HipBayaderaFactory(0, 256)
+    sf = fac.mcmc_factory(models.uniform_model())
+    a, b = (sf.create_sampler(7, 1 << 23, [-1, 2]).init_position(3, [-1, 2]) for _ in range(2))
+    b.move_bare()
+    b.move_bare()
+    want = b.state()
+    b.release()
+    a.move_bare()
+    before = torch.cuda.mem_get_info()[0]
+    with pytest.raises(_lib.BayaderaError):
+        a.init_move(2.0, 1 << 44)  # more than any device holds
+    assert torch.cuda.mem_get_info()[0] - before >= 64 << 20
+    a.move_bare()
+    assert all(np.array_equal(x, y) for x, y in zip(a.state(), want))
+    for h in (a, sf, fac):
         h.release()
