@@ -456,6 +456,7 @@ struct bh_stretch {
     bool ktiming = false;
     std::vector<hipEvent_t> kev;
     size_t kused = 0;
+    uint32_t klaunches = 0;  // within the event pairs
     uint32_t kstride = 1, kcount = 0;  // every kstride-th launch is timed
 };
 
@@ -530,16 +531,19 @@ struct Timed {
 };
 
 // Launches a dominant kernel between two events of the sampler's timing pool
-// when kernel timing is on and the pool has room.
+// when kernel timing is on and the pool has room.  What takes the place of
+// `count` such launches counts as that many.
 template <class F>
-int ktimed(bh_stretch* s, F&& launch_fn) {
-    const bool rec = s->ktiming && (s->kcount++ % s->kstride) == 0 &&
-                     s->kused + 2 <= s->kev.size();
+int ktimed(bh_stretch* s, F&& launch_fn, uint32_t count = 1) {
+    const uint32_t first = s->kcount, due = (first + s->kstride - 1) / s->kstride * s->kstride;
+    s->kcount += count;
+    const bool rec = s->ktiming && due < first + count && s->kused + 2 <= s->kev.size();
     if (rec) BH_HIP(hipEventRecord(s->kev[s->kused], s->stream));
     BH_TRY(launch_fn());
     if (rec) {
         BH_HIP(hipEventRecord(s->kev[s->kused + 1], s->stream));
         s->kused += 2;
+        s->klaunches += count;
     }
     return BH_OK;
 }
@@ -663,23 +667,23 @@ int run_resident(bh_stretch* s, Call& call, bool accu, uint32_t seed_odd, uint32
         unsigned kp = Kp;
         void* da[] = {&seed_odd, &seed_even, &c_odd, &c_even, &K, &kp, &a, &step, &n, &partner,
                       &draws};
-        BH_HIP(hipModuleLaunchKernel(s->f->draws, (K + 255) / 256, std::min(2 * n, 65535u), 1, 256,
-                                     1, 1, 0, s->stream, da, nullptr));
         const float* betas = d_betas ? d_betas + done : nullptr;
         float* out = rtrace;
         if (sample_out) out = sample_out + step_floats * done;
         void* ra[] = {&drawsc, &data_len, &params_len, &params, &xs,  &lf, &K,
                       &beta,   &betas,    &n,          &acc,    &out, &sink};
-        BH_TRY(ktimed(s, [&] {
-            return launch(out ? s->f->resident_out : s->f->resident, 1, nb,
-                          (unsigned)resident_lds(s), s->stream, ra);
+        const float* trace = rtrace;
+        void* ta[] = {&trace, &K, &step, &means};
+        BH_TRY(ktimed(s, [&]() -> int {
+            BH_HIP(hipModuleLaunchKernel(s->f->draws, (K + 255) / 256, std::min(2 * n, 65535u), 1,
+                                         256, 1, 1, 0, s->stream, da, nullptr));
+            BH_TRY(launch(out ? s->f->resident_out : s->f->resident, 1, nb,
+                          (unsigned)resident_lds(s), s->stream, ra));
+            if (accu)
+                BH_HIP(hipModuleLaunchKernel(s->f->trace_accu, s->groups, n, 1, s->wgs, 1, 1, 0,
+                                             s->stream, ta, nullptr));
+            return BH_OK;
         }));
-        if (accu) {
-            const float* trace = rtrace;
-            void* ta[] = {&trace, &K, &step, &means};
-            BH_HIP(hipModuleLaunchKernel(s->f->trace_accu, s->groups, n, 1, s->wgs, 1, 1, 0,
-                                         s->stream, ta, nullptr));
-        }
     }
     return BH_OK;
 }
@@ -1078,17 +1082,19 @@ int bare_pair(bh_stretch* s, float beta, float* out = nullptr) {
         const unsigned short *pos0 = p.pos, *pos1 = p.pos + K;
         void* f0[] = {&seed0, &c0, &data_len, &params_len, &params, &found, &pos0, &x0, &l0, &a, &beta, &step, &K, &o0};
         void* f1[] = {&seed1, &c1, &data_len, &params_len, &params, &found, &pos1, &x1, &l1, &a, &beta, &step, &K, &o1};
-        BH_TRY(ktimed(s, [&]() -> int {
-            const unsigned seeds[2] = {seed0, seed1}, consts[2] = {c0, c1};
-            BH_HIP(bh::launch_partner_sort(s->stream, p, partner == BH_PARTNER_WALKER, seeds, consts,
-                                           step));
-            BH_HIP(bh::launch_partner_read(s->stream, p, 0, S1));
-            return launch(s->f->found, p.tiles(), kFoundThreads, 0, s->stream, f0);
-        }));
-        return ktimed(s, [&]() -> int {
-            BH_HIP(bh::launch_partner_read(s->stream, p, 1, S0));
-            return launch(s->f->found, p.tiles(), kFoundThreads, 0, s->stream, f1);
-        });
+        // (the sort is both half-steps')
+        return ktimed(
+            s,
+            [&]() -> int {
+                const unsigned seeds[2] = {seed0, seed1}, consts[2] = {c0, c1};
+                BH_HIP(bh::launch_partner_sort(s->stream, p, partner == BH_PARTNER_WALKER, seeds,
+                                               consts, step));
+                BH_HIP(bh::launch_partner_read(s->stream, p, 0, S1));
+                BH_TRY(launch(s->f->found, p.tiles(), kFoundThreads, 0, s->stream, f0));
+                BH_HIP(bh::launch_partner_read(s->stream, p, 1, S0));
+                return launch(s->f->found, p.tiles(), kFoundThreads, 0, s->stream, f1);
+            },
+            2);
     }
     const hipFunction_t move = out ? s->f->bare_out : s->f->bare;
     BH_TRY(ktimed(s, [&] { return launch(move, grid, s->wgs, 0, s->stream, a0); }));
@@ -2083,6 +2089,7 @@ int bh_stretch_set_kernel_timing(bh_stretch* s, int on) {
     s->kstride = on > 0 ? (uint32_t)on : 1u;
     s->kcount = 0;
     s->kused = 0;
+    s->klaunches = 0;
     return BH_OK;
 }
 
@@ -2096,8 +2103,8 @@ int bh_stretch_kernel_timing(bh_stretch* s, double* avg_ms, uint32_t* launches) 
         BH_HIP(hipEventElapsedTime(&ms, s->kev[i], s->kev[i + 1]));
         total += ms;
     }
-    *launches = (uint32_t)(s->kused / 2);
-    *avg_ms = s->kused ? total / (double)(s->kused / 2) : 0.0;
+    *launches = s->klaunches;
+    *avg_ms = s->klaunches ? total / (double)s->klaunches : 0.0;
     return BH_OK;
 }
 

@@ -309,10 +309,13 @@ int bh_stretch_set_timing(bh_stretch* s, int on);
 int bh_stretch_last_gpu_ms(const bh_stretch* s, double* ms);
 /* Kernel timing (no reference counterpart): with on = n >= 1, every n-th
  * launch of the sampler's dominant kernel (the stretch-move kernels, the
- * resident kernel, or a GLM sampler's likelihood contraction) is bracketed
- * by HIP events on the sampler's stream, the first 1024 such launches after
+ * resident steps, or a GLM sampler's likelihood contraction) is bracketed
+ * by HIP events on the sampler's stream, the first 1024 such brackets after
  * the call that turned it on (each pair of events costs the stream ~10 us);
- * on = 0 turns it off.  bh_stretch_kernel_timing waits for the stream and
+ * on = 0 turns it off.  A launch of resident steps is one chunk of them, its
+ * draws and accounting (launches of their own) within the bracket.  Where a
+ * large ensemble's partners are sorted, the bracket holds both half-steps of
+ * a step with the sort they share, and counts as two launches.  bh_stretch_kernel_timing waits for the stream and
  * returns their average duration and count.  Turning it on again restarts
  * the count. */
 int bh_stretch_set_kernel_timing(bh_stretch* s, int on);
