@@ -360,12 +360,14 @@ histogram_finalize_kernel(const unsigned* __restrict__ counts, const float* __re
 // Mean and population variance of every row in one pass over the data, in
 // double (the reference's two passes round the mean and each difference to
 // float, amd-gcn-estimate.cl:146-157).  A block sums its values' differences d
-// from its own first value of the row, which are exact in double, and their
-// squares; it leaves its mean and the sum of squares about it.  The blocks'
-// parts are then combined about the mean of all (Chan, Golub, LeVeque).  With
-// a block's value as its origin, cancellation costs at most a factor of the
-// block's count of values: an origin far from the others is itself among the
-// values whose variance is taken.  partial[(blk*m + r)*3]: the block's mean of
+// from its own first value of the row and their squares; it leaves its mean and
+// the sum of squares about it.  The blocks' parts are then combined about the
+// mean of all (Chan, Golub, LeVeque).  A difference is exact in double where the
+// two floats' exponents are at most 29 apart, and rounded once (2^-53 of it)
+// otherwise.  With a block's value as its origin, cancellation multiplies the
+// rounding errors, of the sums and of such differences, by at most the block's
+// count of values: an origin far from the others is itself among the values
+// whose variance is taken.  partial[(blk*m + r)*3]: the block's mean of
 // row r, its sum of squares, its count.  With var 0 plain sums of the values:
 // partial[blk*m + r].
 template <int VAR>
