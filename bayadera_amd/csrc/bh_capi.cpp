@@ -572,7 +572,8 @@ unsigned resident_threads(const bh_ctx* c, uint32_t dim) {
 }
 
 // The ensembles BH_EXEC_RESIDENT accepts: positions, log densities and 8
-// floats per thread within 64 KB.
+// floats per thread within 64 KB.  Fewer than fit today (AUTO takes 4096 x 7,
+// 7168 x 4); what the option refuses has stayed what it was.
 bool resident_accepted(const bh_stretch* s) {
     unsigned nb = s->K <= 1024 ? s->K : 1024;
     while (nb > s->wgs && (s->K % nb) != 0) nb -= s->wgs;
@@ -2126,7 +2127,7 @@ int bh_stretch_set_exec(bh_stretch* s, int mode) {
     BH_ARG(mode == BH_EXEC_AUTO || mode == BH_EXEC_STEPWISE || mode == BH_EXEC_RESIDENT,
            "unknown execution mode %d", mode);
     if (mode == BH_EXEC_RESIDENT && !resident_accepted(s))
-        return fail(BH_ERR_RANGE, "ensemble (%u walkers x %u) does not fit in one work-group's LDS",
+        return fail(BH_ERR_RANGE, "ensemble (%u walkers x %u) fills more than the 64 KB of BH_EXEC_RESIDENT",
                     s->W, s->dim);
     s->exec = mode;
     if (use_resident(s, UINT64_MAX)) BH_TRY(resident_module(s->f));

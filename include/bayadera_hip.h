@@ -43,7 +43,13 @@ extern "C" {
 #define BH_PARTNER_FLAT 0   /* the reference's partner offset (amd-gcn-mcmc-stretch.cl:57) */
 #define BH_PARTNER_WALKER 1 /* whole-walker partner (Goodman-Weare as published) */
 
-#define BH_EXEC_AUTO 0      /* resident kernel when the ensemble fits in LDS */
+/* How a sampler's steps run; the results are the same bits.  AUTO: resident
+ * where that is the faster: ensembles of at most 12,288 walkers that fit in the
+ * LDS of a compute unit (past 1024 walkers with a density that reads few data
+ * and parameters), in calls of more than one to three steps.  RESIDENT takes
+ * ensembles whose positions, log densities and some accounting fill at most
+ * 64 KB (BH_ERR_RANGE otherwise), which is less than AUTO does. */
+#define BH_EXEC_AUTO 0
 #define BH_EXEC_STEPWISE 1  /* two kernels per step, as the reference */
 #define BH_EXEC_RESIDENT 2  /* one work-group runs many steps from LDS */
 

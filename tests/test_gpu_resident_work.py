@@ -87,3 +87,18 @@ def test_calls_of_few_steps(walkers, fewest):
             assert s.kernel_timing()["launches"] == launches
     for h in (s, sf, fac):
         h.release()
+
+
+@pytest.mark.parametrize("wgs", [64, 256])
+@pytest.mark.parametrize("dim,walkers", [(1, 512), (9, 1024), (38, 1024), (2, 2560), (1, 12288), (4, 7168), (7, 4096)])
+def test_ensembles_that_run_resident(wgs, dim, walkers):
+    """By themselves, all their steps in one launch, also where RESIDENT is
+    refused (the ensembles of test_gpu_resident.py among them)."""
+    fac = engine.HipBayaderaFactory(0, wgs)
+    sf = fac.mcmc_factory(models.diag_gaussian_model(dim))
+    s = sf.create_sampler(3, walkers, [0.0] * dim + [1.0] * dim).init_position(4, [-2, 2] * dim)
+    s.set_kernel_timing(True)
+    s.burn_in(9, 2.0)
+    assert s.kernel_timing()["launches"] == 1
+    for h in (s, sf, fac):
+        h.release()
