@@ -1017,7 +1017,14 @@ bh_trace_accu(const float* __restrict__ trace, unsigned K, unsigned step0,
 // need fewer instructions a pass but leave lanes idle: 5% faster there, 6%
 // slower than a lane per record at 192 posteriors of up to 34 dimensions,
 // where this is 12% faster.)  What bounds it now is the vector instructions,
-// the model's half of them.  The slots' stride is odd where the LDS has the
+// the model's half of them.  A lane still takes its own record where that needs
+// fewer instructions and no more lookups: of models of less than 8 coordinates, for
+// which a run of eight passes is mostly idle, and in LDS records of no multiple of
+// 8, which keep the lanes' banks apart (us per bare step of 1000 posteriors of 256
+// walkers, independent Gaussian, runs / lanes: in LDS 1 coordinate 3.8 / 1.9,
+// 4 4.6 / 3.0, 10 6.9 / 4.5, 16 7.6 / 14, 20 10.4 / 8.0, 100 129 / 103; in place
+// 1 4.2 / 1.9, 4 4.9 / 3.6, 10 7.3 / 8.8).  The form of small models is fixed when
+// they are compiled, which leaves them a third to half the registers.  The slots' stride is odd where the LDS has the
 // room (ypad 1), so that the lanes' loads of one coordinate take different
 // banks.  A work-group of 2 nb threads runs two problems, the i-th largest and
 // the i-th smallest of its launch, in step (see batch_paired); the largest
@@ -1146,7 +1153,9 @@ __device__ __forceinline__ void bh_batch_impl(
     const unsigned ld = dim | ypad;  // odd if the LDS has the room
     const unsigned lane = t & 63u;
     float* yw = yb + (size_t)(t - lane) * ld;  // the wave's proposals
-    const float* y = yw + lane * ld;
+    float* y = yw + lane * ld;
+    // a lane to a record
+    const bool lanes = DIM < 8 || (!GSTATE && ((DIM < 12 && DIM != 8) || dim % 8 != 0));
     constexpr int N = 8;  // passes in flight
     const unsigned yw4 = (unsigned)__builtin_amdgcn_readfirstlane((int)bh_lds_offset(yw));
     const unsigned sx4 = GSTATE ? 0u : bh_lds_offset(sx), dim4 = 4 * dim;
@@ -1168,8 +1177,7 @@ __device__ __forceinline__ void bh_batch_impl(
                     BH_KEY1_STRETCH));
                 const float z = __builtin_fmaf(ca * u.y, u.y, cb * u.y) + inv_a;
                 // partner element i at S[(e + i) mod K*dim] (FLAT) or
-                // S[j*dim + i] (WALKER); e in bytes
-                const unsigned total = 4 * K * dim;
+                // S[j*dim + i] (WALKER)
                 unsigned e;
                 if (partner == BH_PARTNER_FLAT) {
                     e = (unsigned)((u.x * (float)K) * (float)dim);
@@ -1179,39 +1187,65 @@ __device__ __forceinline__ void bh_batch_impl(
                     j = j < K ? j : K - 1;
                     e = j * dim;  // e + i < K * dim for i < dim
                 }
-                e *= 4;
-                // the wave's records (a scalar base, byte offsets below)
-                float* xw = X + (size_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(k - lane)) * dim;
                 const float lk = L[k];
-                e -= yw4;  // + iy: the coordinate's place
-                BhRun at = run0;
-                // N passes from the j-th, all of them in the records (FULL)
-                const auto propose = [&](unsigned j, auto FULL) {
-                    float xa[N], sa[N], zr[N];
-                    unsigned ec[N], yo[N];
+                if (lanes) {
+                    const float* xk = X + (size_t)k * dim;
+                    unsigned i = 0;
+                    for (; !GSTATE && i + N <= dim; i += N) {
+                        float xa[N], sa[N];
 #pragma unroll
-                    for (int c = 0; c < N; ++c) {
-                        ec[c] = bh_lane(e, at.r4) + at.iy;
-                        zr[c] = bh_lane(z, at.r4);
-                        yo[c] = __umul24(at.r4, ld) + at.iy;
-                        at.next(steps);
+                        for (int c = 0; c < N; ++c) {
+                            unsigned ec = e + c;
+                            if (ec >= K * dim) ec -= K * dim;
+                            xa[c] = xk[i + c];
+                            sa[c] = S[ec];
+                        }
+#pragma unroll
+                        for (int c = 0; c < N; ++c)
+                            y[i + c] = __builtin_fmaf(z, xa[c] - sa[c], sa[c]);
+                        e += N;
+                        if (e >= K * dim) e -= K * dim;
                     }
-#pragma unroll
-                    for (int c = 0; c < N; ++c) {
-                        // (a pass past the records loads from within them)
-                        xa[c] = bh_at(xw + 64 * (FULL.v || j + c < dim ? j + c : j), 4 * lane);
-                        // past the end: from the start (the smaller, unsigned)
-                        sa[c] = bh_at(S, ec[c] - total < ec[c] ? ec[c] - total : ec[c]);
+                    for (; i < dim; ++i) {
+                        const float xj = S[e];
+                        y[i] = __builtin_fmaf(z, xk[i] - xj, xj);
+                        e = (e + 1 == K * dim) ? 0u : e + 1;
                     }
+                } else {
+                    // the wave's records (a scalar base, byte offsets below)
+                    const float* xw =
+                        X + (size_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(k - lane)) * dim;
+                    const unsigned total = 4 * K * dim;
+                    e = 4 * e - yw4;  // + iy: the coordinate's place
+                    BhRun at = run0;
+                    // N passes from the j-th, all of them in the records (FULL)
+                    const auto propose = [&](unsigned j, auto FULL) {
+                        float xa[N], sa[N], zr[N];
+                        unsigned ec[N], yo[N];
 #pragma unroll
-                    for (int c = 0; c < N; ++c)
-                        if (FULL.v || j + c < dim)
-                            bh_lds(yo[c]) = __builtin_fmaf(zr[c], xa[c] - sa[c], sa[c]);
-                };
-                unsigned j = 0;
-                for (; j + N <= dim; j += N) propose(j, BhTrue{});
-                if (j < dim) propose(j, BhFalse{});
-                bh_wave_sync();
+                        for (int c = 0; c < N; ++c) {
+                            ec[c] = bh_lane(e, at.r4) + at.iy;
+                            zr[c] = bh_lane(z, at.r4);
+                            yo[c] = __umul24(at.r4, ld) + at.iy;
+                            at.next(steps);
+                        }
+#pragma unroll
+                        for (int c = 0; c < N; ++c) {
+                            // (a pass past the records loads from within them)
+                            xa[c] = bh_at(xw + 64 * (FULL.v || j + c < dim ? j + c : j), 4 * lane);
+                            // past the end: from the start (the smaller, unsigned)
+                            sa[c] = bh_at(S, ec[c] - total < ec[c] ? ec[c] - total : ec[c]);
+                        }
+#pragma unroll
+                        for (int c = 0; c < N; ++c)
+                            if (FULL.v || j + c < dim)
+                                bh_lds(yo[c]) = __builtin_fmaf(zr[c], xa[c] - sa[c], sa[c]);
+                    };
+                    unsigned j = 0;
+                    for (; j + N <= dim; j += N) propose(j, BhTrue{});
+                    if (j < dim) propose(j, BhFalse{});
+                    bh_wave_sync();
+                }
                 const float ly = LOGFN(data_len, params_len, prm, dim, y);
                 float zp = 1.0f;
 #pragma unroll 4
@@ -1222,14 +1256,21 @@ __device__ __forceinline__ void bh_batch_impl(
                     L[k] = ly;
                     nacc += 1;
                 }
+                if (lanes) {
+                    if (accepted)
+                        for (unsigned i = 0; i < dim; ++i) X[(size_t)k * dim + i] = y[i];
+                    continue;
+                }
                 bh_wave_sync();
                 if (__builtin_amdgcn_ballot_w64(accepted) != 0) {
                     // no branch: what did not move is stored past the buffer's
                     // end, which the hardware drops, or (LDS) onto the
                     // proposal itself
                     const unsigned keep = accepted ? 0u : 0x80000000u;
-                    const unsigned xo = (unsigned)(xw - sx) * 4;
-                    at = run0;
+                    const unsigned xo =
+                        ((h ? K : 0u) + (unsigned)__builtin_amdgcn_readfirstlane((int)(k - lane))) *
+                        dim4;
+                    BhRun at = run0;
                     const auto move = [&](unsigned j, auto FULL) {
                         float ya[N];
                         unsigned kept[N], yo[N];
