@@ -302,10 +302,12 @@ glm_gauss_pack_kernel(const float* __restrict__ X, const float* __restrict__ y,
 // consecutive rows of one point, whose squares are summed in fp32 in row
 // order and then added to a double.  A block of 4 waves owns 256 points, 64
 // per wave as four column blocks whose coefficients stay in registers; the
-// next row block is loaded while one is multiplied.  The products alone bound
-// it: 100,000 x 16 rows x 4096 points take 119 us (87 at the 150 TFLOP/s
-// the instruction reaches by itself; residuals, squares and sums overlap with
-// it but for 14 us), 167 us as fma chains on the vector units.
+// next row block is loaded while one is multiplied.  Bound by the issue of
+// products and then of the other vector instructions, which follow a block's
+// products: 100,000 x 16 rows x 4096 points take 119 us, in whose cycles the
+// matrix cores are busy 0.67 (6,250 products of 32 cycles to a SIMD) and the
+// 18,900 residuals, squares, sums and addresses of 4 cycles fill 0.25; 0.08 is
+// loads and starts.  As fma chains on the vector units 167 us.
 template <int D>
 __global__ void __launch_bounds__(256)
 glm_gauss_mfma_kernel(const f32x4* __restrict__ Xf, const f32x4* __restrict__ yf, unsigned nblocks,

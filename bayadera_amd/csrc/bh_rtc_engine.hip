@@ -1001,8 +1001,8 @@ bh_trace_accu(const float* __restrict__ trace, unsigned K, unsigned step0,
 #endif  // LOGFN
 
 #ifdef BH_BATCH
-// Many independent posteriors of one model source in one launch: one
-// work-group per problem, its W walkers advanced for all steps of the call
+// Many independent posteriors of one model source in one launch: a
+// work-group per problem (or two), its W walkers advanced for all steps of the call
 // inside the work-group.  A problem b with dimension dims[b] <= DIM and
 // params params + poff[b] runs exactly the single-sampler algorithm
 // (move-bare!, constants 3333/4444) with bare seed seed0 + 2b: the same

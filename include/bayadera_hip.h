@@ -59,7 +59,8 @@ extern "C" {
 #define BH_GLM_LOGISTIC 1   /* y_i ~ Bernoulli(sigmoid(x_i . beta)), beta ~ N(0, s^2 I) */
 #define BH_GLM_GAUSSIAN 2   /* y_i ~ N(x_i . beta, sigma^2), beta ~ N(0, s_b^2 I), log sigma ~ N(0, s_s^2) */
 #define BH_GLM_FP64 0       /* fp64 VALU: the accuracy reference */
-#define BH_GLM_FP32 1       /* plain fp32 VALU contraction and softplus */
+#define BH_GLM_FP32 1       /* plain fp32: VALU contraction and softplus; linear regression on the
+                               fp32 matrix cores (the bits of a chain of fma) */
 #define BH_GLM_BF16 2       /* MFMA, bf16 x bf16 -> fp32, one product */
 #define BH_GLM_BF16X3 3     /* MFMA, proposals split in three bf16 terms (fp32-accurate) */
 #define BH_GLM_FP16X2 4     /* MFMA on an fp16 copy of X, proposals split in two fp16 terms
